@@ -3,8 +3,8 @@
 // lineshape, the exchange step, step_mt; :563-601 the field model; engines/core.py:115-121, 190-217).
 //
 // One lane per isochromat, workgroups of 256 (4 waves of 64), every lane walking the same plain segment records. Per
-// spin the free pool's (Mx, My, Mz) and, with a bound pool, its Mzb; Mz and Mzb carry two-sum low parts. Without a
-// bound pool the longitudinal step is plain T1 recovery.
+// spin the free pool's (Mx, My, Mz) and, with a bound pool, its Mzb; Mz and Mzb carry low parts. Without a bound pool
+// the longitudinal step is plain T1 recovery.
 // - Concomitant field f_c [Hz] of a segment with gradient g: leading order c . (gx^2, gy^2, gz^2, gx gy, gx gz,
 //   gy gz), or exact |B| - f0 - lin = t^2 / (sqrt(u^2 + t^2) + u) (t^2 = (ax . g)^2 + (ay . g)^2, u = f0 + lin, lin the
 //   rest of the offset); it adds to an RF segment's offset (and so to the bound pool's saturation offset) and, times
@@ -14,59 +14,107 @@
 //   that only the bound pool feels); the other half.
 // - Free segment: exact precession (float64 phase, as the plain kernels') and transverse decay; the unsaturated
 //   exchange over the segment.
-// - The exchange over t is exact: z_ss + exp(A t) (z - z_ss) for the 2 x 2 generator A of (Mz, Mzb), in increment
-//   form (exp(A t) - I)(z - z_ss) = (e^{mt} cosh(qt) - 1)(z - z_ss) + e^{mt} sinh(qt)/q (A - m I)(z - z_ss), with
-//   m +- q the eigenvalues and both factors from expm1 of m +- q, so that short steps keep their low bits.
-// - Factors that depend only on the segment's length and the spin (the free segment's decay and unsaturated exchange,
-//   the RF segment's half-step decay) are kept across segments the records mark as having the previous one's dt
-//   (HB_SAME_FREE_DT, HB_SAME_RF_DT): the cache restarts with every dispatch, as the hints do.
-// - ADC: every sample's coil sums over the workgroup (over each wave, then the 4 waves in order in LDS) go to the
-//   partial rows that hb_signal_reduce sums in a fixed order: no atomics. Up to 16 coils the sensitivities sit in
-//   registers and the wave's 2 C sums are one reduce-scatter (each step halves the values a lane carries: 17
-//   shuffles for 8 coils, against 96 for a butterfly per value); more coils take a butterfly per value.
-// - The next segment record is loaded while the current one is stepped.
+// - The exchange over t is exact, in increment form from the rates of change d = A z + c (A the 2 x 2 generator of
+//   (Mz, Mzb), c its source): (exp(A t) - I)(z - z_ss) = t phi1(A t) d, phi1(x) = (e^x - 1) / x, as alpha d +
+//   beta (A - m I) d with m the mean eigenvalue. d is formed from differences (PD - Mz, Mzb - f Mz, f PD - Mzb) that
+//   vanish at equilibrium, so that its rounding vanishes there too, and no steady state (two divisions) is needed.
+//   Short steps (an RF substep: eigenvalues times t under 0.03) take alpha and beta from their series: no square root,
+//   exponential or division; longer ones from the eigenvalues' expm1.
+// - ADC: eight samples at a time are staged in LDS and contracted with the coils on the matrix cores
+//   (contract_device.h), one barrier per eight; the workgroup's sums go to the partial rows that hb_signal_reduce sums
+//   in a fixed order: no atomics.
+//
+// What bounds it: with 65,536 spins every SIMD has one wave, so nothing hides a wave's latency, and a segment costs its
+// chain of dependent instructions. What only depends on a segment's offset (its concomitant field, the saturation's
+// lineshape with its table lookup, the rotation's z component) is kept while HB_SAME_RF_OFFSET says that the next RF
+// segment's is the same, a free segment's phase factors while HB_SAME_FREE does, factors of the length while it stays;
+// an RF train is stepped in a loop of its own that reads four values per substep, a readout run in one that reads none
+// and relaxes the longitudinal components once. The next record is loaded while the current one is stepped, and the
+// lanes touch the records 64 ahead, so that they are in the L2 when their turn comes. 65,536 spins with a bound pool and
+// leading-order fields, 8 coils, 32,256 segments (12,800 RF, 16,384 samples): 9.7 ms, against 34.8 ms with a barrier and
+// a shuffle tree per sample, steady states by division and every factor formed per segment. Of its 5.75 million issue
+// slots a wave uses 2.3 for VALU and 1.0 for scalar instructions and waits in 1.8 (SQ counters).
 #include "bloch_device.h"
+#include "contract_device.h"
 
 #include "../../include/blochparty_amd_mt.h"
 
 namespace hb {
 namespace {
 
-constexpr int kBlockM = 256;
-constexpr int kWavesM = kBlockM / 64;
-constexpr int kMaxCoilsM = 128;
+// hi + lo += d, the low part as Kahan's sum keeps it: exact where |hi| >= |d + lo|, within d's own rounding otherwise
+// (4 operations against two_sum's 7).
+__device__ __forceinline__ void add_low(float& hi, float& lo, float d) {
+    const float y = d + lo, t = hi + y;
+    lo = y - (t - hi);
+    hi = t;
+}
 
-// The exchange step over t: the steady state and the two increment factors.
-struct XStep {
-    float z1, z2;      // steady state -A^-1 c
-    float chm1, sh;    // e^{mt} cosh(qt) - 1, e^{mt} sinh(qt) / q
-    float h, a12, a21; // A - m I = [[h, a12], [a21, -h]]
+// A spin's bound pool: f, the exchange rates k and k f, R1b, T2b, dw, and f PD.
+struct Pool {
+    float f, k, kf, r1b, t2b, dw, fpd;
 };
 
-__device__ __forceinline__ XStep xstep(float t, float pd, float r1, float f, float k, float r1b, float w) {
-    const float kf = k * f;
-    const float a11 = -(r1 + kf), a12 = k, a21 = kf, a22 = -(r1b + k + w);
-    const float c1 = r1 * pd, c2 = r1b * f * pd;
-    const float det = a11 * a22 - a12 * a21;
-    XStep x;
-    x.z1 = (a12 * c2 - a22 * c1) / det;
-    x.z2 = (a21 * c1 - a11 * c2) / det;
+// The exchange step over t of the generator A = [[-(R1 + k f), k], [k f, -(R1b + k + W)]]: the increment of (Mz, Mzb)
+// is alpha d + beta (h d1 + k d2, k f d1 - h d2) with d the rates of change, A - m I = [[h, k], [k f, -h]].
+struct XStep {
+    float alpha, beta, h;
+};
+
+__device__ __forceinline__ XStep xstep(float t, float r1, const Pool& b, float w) {
+    const float a11 = -(r1 + b.kf), a22 = -(b.r1b + b.k + w);
     const float m = 0.5f * (a11 + a22), h = 0.5f * (a11 - a22);
-    const float q = sqrtf(fmaf(h, h, a12 * a21));
-    x.chm1 = 0.5f * (expm1x((m + q) * t) + expm1x((m - q) * t));
-    const float lo = __expf((m - q) * t);
-    if (2.0f * q * t < 1.0f)
-        x.sh = q > 0.0f ? lo * 0.5f * expm1x(2.0f * q * t) / q : t * __expf(m * t);
-    else
-        x.sh = 0.5f * (__expf((m + q) * t) - lo) / q;
-    x.h = h, x.a12 = a12, x.a21 = a21;
+    const float Q = fmaf(h, h, b.k * b.kf);
+    XStep x;
+    x.h = h;
+    const float mt = m * t;
+    if (mt > -0.015f) {  // both eigenvalues are in [2 m, 0]: |lambda t| < 0.03
+        // phi1(z) = 1 + z/2 + z^2/6 + z^3/24 + z^4/120 at z = m t +- sqrt(Q) t: the mean and the divided difference
+        // (the next terms are under 1e-8 of the first)
+        const float y = Q * t * t, m2 = mt * mt;
+        x.alpha = t * (1.0f + 0.5f * mt + (m2 + y) * (1.0f / 6.0f) + mt * fmaf(3.0f, y, m2) * (1.0f / 24.0f));
+        x.beta = t * t * (0.5f + mt * (1.0f / 3.0f) + fmaf(3.0f, m2, y) * (1.0f / 24.0f) +
+                          mt * (m2 + y) * (1.0f / 30.0f));
+        return x;
+    }
+    const float q = sqrtf(Q);
+    const float lm = m - q;                                          // no cancellation: m < 0
+    const float det = r1 * (b.r1b + b.k + w) + b.kf * (b.r1b + w);   // lp lm, without cancellation
+    const float lp = det / lm;
+    const float fp = lp != 0.0f ? expm1x(lp * t) / lp : t, fm = expm1x(lm * t) / lm;
+    x.alpha = 0.5f * (fp + fm);
+    if (q * t > 1e-3f) {
+        x.beta = 0.5f * (fp - fm) / q;
+    } else {  // a (nearly) double eigenvalue: t^2 phi1'(m t), by its series for small m t
+        const float small =
+            0.5f + mt * (1.0f / 3.0f + mt * (0.125f + mt * (1.0f / 30.0f + mt * (1.0f / 144.0f + mt * (1.0f / 840.0f)))));
+        x.beta = t * t * (mt > -0.25f ? small : (__expf(mt) * (mt - 1.0f) + 1.0f) / (mt * mt));
+    }
     return x;
 }
 
-__device__ __forceinline__ void exchange(const XStep& x, State& m, float& mb, float& lb) {
-    const float d1 = m.mz - x.z1, d2 = mb - x.z2;
-    two_sum(m.mz, m.lz, x.chm1 * d1 + x.sh * (x.h * d1 + x.a12 * d2));
-    two_sum(mb, lb, x.chm1 * d2 + x.sh * (x.a21 * d1 - x.h * d2));
+// The increments of (Mz, Mzb) over the step x from (z, b) with the rates of change (d1, d2).
+__device__ __forceinline__ void increments(const XStep& x, const Pool& p, float d1, float d2, float& dz, float& db) {
+    dz = x.alpha * d1 + x.beta * fmaf(x.h, d1, p.k * d2);
+    db = x.alpha * d2 + x.beta * fmaf(p.kf, d1, -(x.h * d2));
+}
+
+// An RF half step from (z, b), the bound pool saturated at w (the low parts, under half an ulp, change nothing over a
+// substep).
+__device__ __forceinline__ void exchange_rf(const XStep& x, const Pool& p, float pd, float r1, float w, float z,
+                                            float b, float& dz, float& db) {
+    const float ex = p.k * fmaf(-p.f, z, b);
+    increments(x, p, fmaf(r1, pd - z, ex), fmaf(p.r1b, p.fpd - b, -fmaf(w, b, ex)), dz, db);
+}
+
+// A free step of the state (unsaturated), from the whole values with their low parts.
+__device__ __forceinline__ void exchange_free(const XStep& x, const Pool& p, float pd, float r1, State& m, float& mb,
+                                              float& lb) {
+    const float ex = p.k * (fmaf(-p.f, m.mz, mb) + fmaf(-p.f, m.lz, lb));
+    float dz, db;
+    increments(x, p, fmaf(r1, (pd - m.mz) - m.lz, ex), fmaf(p.r1b, (p.fpd - mb) - lb, -ex), dz, db);
+    add_low(m.mz, m.lz, dz);
+    add_low(mb, lb, db);
 }
 
 // G(2 pi delta) [s]: the Lorentzian, or T2b F(x) from the table of ln F (held at the cut, 0 past the table's end).
@@ -84,17 +132,6 @@ __device__ __forceinline__ float lineshape_g(const hb_mt& mt, float delta, float
     return t2b * expf(mt.table[i] * (1.0f - a) + mt.table[i + 1] * a);
 }
 
-// Rotation of the state by the rotation vector w (right-handed, angle |w|), as rf_step's: m + a (w x m) + b w x (w x m).
-__device__ __forceinline__ void rotate_state(State& m, float wx, float wy, float wz) {
-    float a, b;
-    rot_ab(wx * wx + wy * wy + wz * wz, a, b);
-    const float cx = wy * m.mz - wz * m.my, cy = wz * m.mx - wx * m.mz, cz = wx * m.my - wy * m.mx;
-    const float ex = wy * cz - wz * cy, ey = wz * cx - wx * cz, ez = wx * cy - wy * cx;
-    m.mx += a * cx + b * ex;
-    m.my += a * cy + b * ey;
-    two_sum(m.mz, m.lz, a * cz + b * ez);
-}
-
 // The spin's concomitant field in segment q, lin the rest of its offset there [Hz]; cc the spin's coefficients.
 __device__ __forceinline__ float conc_field(int mode, const float (&cc)[7], const hb_segment& q, float lin) {
     const float gx = q.g_x, gy = q.g_y, gz = q.g_z;
@@ -107,55 +144,37 @@ __device__ __forceinline__ float conc_field(int mode, const float (&cc)[7], cons
     return den > 0.0f ? t2 / den : 0.0f;
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
+__device__ __forceinline__ int bits_differ(float a, float b) { return __float_as_int(a) ^ __float_as_int(b); }
 
-constexpr int ilog2(int v) { return v <= 1 ? 0 : 1 + ilog2(v >> 1); }
-
-// The wave's sums of V values (V a power of two <= 64), in a fixed order: over lane bits 5, 4, ... each step keeps
-// half the values (a lane with the bit set the upper half) and adds the partner's copy of them, then the remaining
-// low bits are summed by a butterfly. Value i ends on the lanes with lane >> (6 - log2 V) == i, in v[0].
-// (Each step is its own instantiation, so that every index into v is a compile-time constant and v stays in
-// registers without select chains.)
-template <int V, int ST>
-__device__ __forceinline__ void scatter_step(float (&v)[V], int lane) {
-    if constexpr ((V >> ST) > 1) {
-        constexpr int bit = 1 << (5 - ST), half = V >> (ST + 1);
-        const bool up = lane & bit;
-#pragma unroll
-        for (int k = 0; k < half; ++k) {
-            const float send = up ? v[k] : v[k + half], keep = up ? v[k + half] : v[k];
-            v[k] = keep + __shfl_xor(send, bit, 64);
-        }
-        scatter_step<V, ST + 1>(v, lane);
-    }
-}
-
-template <int V>
-__device__ __forceinline__ void wave_scatter_sums(float (&v)[V], int lane) {
-    scatter_step<V, 0>(v, lane);
-#pragma unroll
-    for (int b = 5 - ilog2(V); b >= 0; --b) v[0] += __shfl_xor(v[0], 1 << b, 64);
-}
-
-// NC: the coils' register width (1, 2, 4, 8, 16; C <= NC, the rest zero), or 0 for any count read per sample.
-template <int NC>
-__global__ __launch_bounds__(kBlockM) void forward_mt_kernel(hb_case cs, hb_mt mt, int s0, int s1,
-                                                             float* __restrict__ partial, int rows, int row0) {
-    __shared__ float red[kWavesM][2 * kMaxCoilsM];
+// NT: coil tiles as forward_kernel's (1, 2: the sensitivities in registers; 0: any, read per flush). segs, sens_r,
+// rf_freq and table are the pointers of cs_in and mt_in again, as noalias parameters: no store of the kernel can change
+// what they point to, so the records load through the scalar cache.
+template <int NT>
+__global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt_in, int s0, int s1,
+                                                            float* __restrict__ partial, int rows, int row0,
+                                                            const hb_segment* __restrict__ segs,
+                                                            const float* __restrict__ sens_r,
+                                                            const float* __restrict__ rf_freq,
+                                                            const float* __restrict__ table) {
+    hb_mt mt = mt_in;
+    mt.table = table;
+    extern __shared__ float lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int j = blockIdx.x * kBlockM + tid;
+    const int j = blockIdx.x * kBlock + tid;
     const int np = cs.n_pad;
+    const int nt = NT > 0 ? NT : cs.n_tiles;
+    float* stg = lds + wave * kStgFloats;
+    float* wred = lds + kWaves * kStgFloats;
+    float warm = segs[min(s0 + lane, s1 - 1)].dt;
     const Spin p = load_spin(cs.spins, cs.pos_lo, np, j);
     const Pos64 r64 = pos64(p);
-    const bool pool = mt.pool != nullptr;  // uniform
-    const float f = pool ? mt.pool[j] : 0.0f, k = pool ? mt.pool[np + j] : 0.0f;
-    const float r1b = pool ? mt.pool[2 * np + j] : 1.0f, t2b = pool ? mt.pool[3 * np + j] : 1.0f;
-    const float dw = pool ? mt.pool[4 * np + j] : 0.0f;
     const float b1sq = p.b1 * p.b1;
+    const bool pool = mt.pool != nullptr;  // uniform
+    Pool b;
+    b.f = pool ? mt.pool[j] : 0.0f, b.k = pool ? mt.pool[np + j] : 0.0f;
+    b.r1b = pool ? mt.pool[2 * np + j] : 1.0f, b.t2b = pool ? mt.pool[3 * np + j] : 1.0f;
+    b.dw = pool ? mt.pool[4 * np + j] : 0.0f;
+    b.kf = b.k * b.f, b.fpd = b.f * p.pd;
     State m = load_state(cs.state, np, j);
     float mb = pool ? mt.mb[j] : 0.0f, lb = pool ? mt.mb[np + j] : 0.0f;
     const int cmode = mt.conc_mode;
@@ -164,109 +183,171 @@ __global__ __launch_bounds__(kBlockM) void forward_mt_kernel(hb_case cs, hb_mt m
 #pragma unroll
         for (int i = 0; i < 7; ++i) cc[i] = mt.conc[(size_t)i * np + j];
     }
-    const int C = cs.n_coils, vals = 16 * cs.n_tiles;
-    float sr[NC > 0 ? NC : 1], si[NC > 0 ? NC : 1];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-        sr[c] = c < C ? mt.sens[(size_t)(2 * c) * np + j] : 0.0f;
-        si[c] = c < C ? mt.sens[(size_t)(2 * c + 1) * np + j] : 0.0f;
-    }
-    XStep xf;                       // free segments: the unsaturated exchange over dt (with a bound pool)
+    Sens<NT> S;
+    S.sa = sens_r + (size_t)(lane & 15) * np + blockIdx.x * kBlock + wave * 64 + 16 * (lane >> 4);
+    S.st = 16 * (size_t)np, S.su = 1, S.n_rows = 2 * cs.n_coils;
+    S.load(cs.x_scale, cs.sens_scale, lane);
+    int nb = 0, row = 0, par = 0;   // staged samples, the first one's partial row, the flush's buffer
+    XStep xf = {0.0f, 0.0f, 0.0f};  // free segments: the unsaturated exchange over dt (with a bound pool)
+    XStep xl = {0.0f, 0.0f, 0.0f};  // and over the last readout run
     float e1f = 0.0f, e2f = 0.0f;   // free segments: expm1 of -dt R1 (without a bound pool), -dt R2
+    float e1l = 0.0f;               // the last readout run's expm1 of -L dt R1 (without a bound pool)
+    float cs_ = 1.0f, sn = 0.0f;    // free segments: cos, sin of the precession
     float e1r = 0.0f, e2r = 0.0f;   // RF segments: expm1 of -dt/2 R1 (without a bound pool), -dt/2 R2
+    float wG = 0.0f, wz = 0.0f;     // RF segments: W over |w_rf|^2, the rotation vector's z
+    float run_dt = -1.0f;
+    int run_len = 0;
     bool free_ok = false, rf_ok = false;
-    hb_segment nq = cs.segs[s0];
-    for (int s = s0; s < s1; ++s) {
-        const hb_segment q = nq;
-        if (s + 1 < s1) nq = cs.segs[s + 1];
-        const int fl = q.flags;
-        if (fl & HB_RF) {
-            float bz = offset(p, q);
-            const float fc = cmode != HB_CONC_NONE ? conc_field(cmode, cc, q, bz) : 0.0f;
-            bz += fc;
-            if (!(rf_ok && (fl & HB_SAME_RF_DT))) {
-                e2r = expm1x(-0.5f * q.dt * p.r2);
-                if (!pool) e1r = expm1x(-0.5f * q.dt * p.r1);
-                rf_ok = true;
-            }
-            const float e2 = e2r, e1 = e1r;
-            XStep x;
-            if (pool) {
-                const float w1sq = HB_TWO_PI * HB_TWO_PI * b1sq * (q.rf_x * q.rf_x + q.rf_y * q.rf_y);
-                const float sat = w1sq * lineshape_g(mt, mt.rf_freq[s] - bz - dw, t2b);
-                x = xstep(0.5f * q.dt, p.pd, p.r1, f, k, r1b, sat);
-            }
-            m.mx += m.mx * e2, m.my += m.my * e2;
-            if (pool)
-                exchange(x, m, mb, lb);
-            else
-                two_sum(m.mz, m.lz, (m.mz - p.pd) * e1);
-            const float wz =
-                p.px * q.w_g_x + p.py * q.w_g_y + p.pz * q.w_g_z + (p.db0 * q.w + q.w_b0) + q.w * fc;
-            if (fl & HB_BOUND_ONLY)
-                rotate_state(m, 0.0f, 0.0f, wz);
-            else
-                rotate_state(m, p.b1 * q.w_rf_x, p.b1 * q.w_rf_y, wz);
-            m.mx += m.mx * e2, m.my += m.my * e2;
-            if (pool)
-                exchange(x, m, mb, lb);
-            else
-                two_sum(m.mz, m.lz, (m.mz - p.pd) * e1);
+
+    // what an RF segment's offset, length and RF frequency give: decays, the saturation's lineshape, w_z
+    auto rf_offset = [&](const hb_segment& q, float frf) {
+        e2r = expm1x(-0.5f * q.dt * p.r2);
+        if (!pool) e1r = expm1x(-0.5f * q.dt * p.r1);
+        float bz = offset(p, q);
+        const float fc = cmode != HB_CONC_NONE ? conc_field(cmode, cc, q, bz) : 0.0f;
+        bz += fc;
+        if (pool) {  // W = (2 pi b1 |rf|)^2 G, |w_rf| = 2 pi dt |rf|
+            const float t = q.dt > 0.0f ? p.b1 / q.dt : 0.0f;
+            wG = t * t * lineshape_g(mt, frf - bz - b.dw, b.t2b);
+        }
+        wz = p.px * q.w_g_x + p.py * q.w_g_y + p.pz * q.w_g_z + (p.db0 * q.w + q.w_b0) + q.w * fc;
+        rf_ok = true;
+    };
+    // the Strang step with the transverse rotation vector factors (wrx, wry), wr2 = |w_rf|^2; water: the water feels it
+    auto rf_segment = [&](float t, float wrx, float wry, float wr2, bool water) {
+        XStep x = {0.0f, 0.0f, 0.0f};
+        float w = 0.0f, dz1, db1 = 0.0f;
+        if (pool) {
+            w = wr2 * wG;
+            x = xstep(t, p.r1, b, w);
+            exchange_rf(x, b, p.pd, p.r1, w, m.mz, mb, dz1, db1);
         } else {
+            dz1 = (m.mz - p.pd) * e1r;
+        }
+        const float dx1 = m.mx * e2r, dy1 = m.my * e2r;
+        const float x1 = m.mx + dx1, y1 = m.my + dy1, z1 = m.mz + dz1, b1 = mb + db1;
+        const float wx = water ? p.b1 * wrx : 0.0f, wy = water ? p.b1 * wry : 0.0f;
+        float ra, rb;
+        rot_ab((water ? b1sq * wr2 : 0.0f) + wz * wz, ra, rb);
+        const float cx = wy * z1 - wz * y1, cy = wz * x1 - wx * z1, cz = wx * y1 - wy * x1;
+        const float ex = wy * cz - wz * cy, ey = wz * cx - wx * cz, ez = wx * cy - wy * cx;
+        const float drx = ra * cx + rb * ex, dry = ra * cy + rb * ey, drz = ra * cz + rb * ez;
+        m.mx += dx1 + drx + (x1 + drx) * e2r;
+        m.my += dy1 + dry + (y1 + dry) * e2r;
+        const float z2 = z1 + drz;
+        if (pool) {
+            float dz2, db2;
+            exchange_rf(x, b, p.pd, p.r1, w, z2, b1, dz2, db2);
+            add_low(m.mz, m.lz, dz1 + drz + dz2);
+            add_low(mb, lb, db1 + db2);
+        } else {
+            add_low(m.mz, m.lz, dz1 + drz + (z2 - p.pd) * e1r);
+        }
+    };
+    // the free segment's factors (hints in f, honoured once factors are held)
+    auto free_factors = [&](const hb_segment& q, int f) {
+        if (!free_ok) f &= ~(HB_SAME_FREE | HB_SAME_FREE_DT);
+        if (!(f & HB_SAME_FREE)) {
             double cyc = free_cycles64(r64, p, q);
             if (cmode != HB_CONC_NONE) cyc += (double)(conc_field(cmode, cc, q, offset(p, q)) * q.dt);
             cyc -= rint(cyc);
-            float sn, cs_;
             sincospi(-2.0f * (float)cyc, &sn, &cs_);
-            if (!(free_ok && (fl & HB_SAME_FREE_DT))) {
+            if (!(f & HB_SAME_FREE_DT)) {
                 e2f = expm1x(-q.dt * p.r2);
                 if (pool)
-                    xf = xstep(q.dt, p.pd, p.r1, f, k, r1b, 0.0f);
+                    xf = xstep(q.dt, p.r1, b, 0.0f);
                 else
                     e1f = expm1x(-q.dt * p.r1);
-                free_ok = true;
             }
-            const float nx = cs_ * m.mx - sn * m.my, ny = sn * m.mx + cs_ * m.my;
-            m.mx = nx + nx * e2f;
-            m.my = ny + ny * e2f;
-            if (pool)
-                exchange(xf, m, mb, lb);
-            else
-                two_sum(m.mz, m.lz, (m.mz - p.pd) * e1f);
+            free_ok = true;
         }
-        if (fl & HB_ADC) {  // the workgroup's coil sums of this sample (uniform branch: every lane takes it)
-            const int r = q.pad[0] - row0;
-            if constexpr (NC > 0) {
-                float v[2 * NC];
-#pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    v[2 * c] = sr[c] * m.mx - si[c] * m.my;
-                    v[2 * c + 1] = sr[c] * m.my + si[c] * m.mx;
-                }
-                wave_scatter_sums<2 * NC>(v, lane);
-                constexpr int low = 6 - ilog2(2 * NC);
-                if ((lane & ((1 << low) - 1)) == 0) red[wave][lane >> low] = v[0];
+    };
+    auto precess = [&]() {
+        const float nx = cs_ * m.mx - sn * m.my, ny = sn * m.mx + cs_ * m.my;
+        m.mx = nx + nx * e2f;
+        m.my = ny + ny * e2f;
+    };
+    auto stage = [&](int r) {  // uniform: every lane takes it
+        if (r < 0 || r >= rows) return;
+        if (nb == 0) row = r;
+        stg[nb * kStgStride + lane] = m.mx * S.x_scale;
+        stg[(8 + nb) * kStgStride + lane] = m.my * S.x_scale;
+        if (++nb == 8) {
+            flush<NT>(stg, wred, par, S, nt, 8, row, rows, partial);
+            nb = 0;
+        }
+    };
+
+    int warm_at = s0;
+    hb_segment nq = segs[s0];
+    for (int s = s0; s < s1;) {
+        const hb_segment q = nq;
+        const int fl = q.flags;
+        int len = 1;
+        if (fl & (HB_RUN | HB_TRAIN)) len = max(1, min(q.pad[3], s1 - s));
+        nq = segs[min(s + len, s1 - 1)];  // in flight while this record is stepped
+        if (s >= warm_at) {  // the records up to 128 ahead into the L2 (the value itself is not used)
+            asm volatile("" ::"v"(warm));
+            warm = segs[min(s + 64 + lane, s1 - 1)].dt;
+            warm_at = s + 64;
+        }
+        if (fl & HB_RF) {
+            if (!(fl & HB_SAME_RF_OFFSET) || !rf_ok) rf_offset(q, pool ? rf_freq[s] : 0.0f);
+            float wrx = q.w_rf_x, wry = q.w_rf_y, wr2 = q.w_rf2;
+            const float t = 0.5f * q.dt;
+            if (!(fl & HB_TRAIN)) {
+                rf_segment(t, wrx, wry, wr2, !(fl & HB_BOUND_ONLY));
             } else {
-                for (int c = 0; c < C; ++c) {
-                    const float s_r = mt.sens[(size_t)(2 * c) * np + j], s_i = mt.sens[(size_t)(2 * c + 1) * np + j];
-                    const float re = wave_sum(s_r * m.mx - s_i * m.my), im = wave_sum(s_r * m.my + s_i * m.mx);
-                    if (lane == 0) red[wave][2 * c] = re, red[wave][2 * c + 1] = im;
+                // a train: the next segment's flags and rotation factors are in flight while one is stepped
+                int f = fl;
+                float tt = t;
+                for (int i = 1; i <= len; ++i) {
+                    const hb_segment* nx = segs + s + (i < len ? i : 0);
+                    const int nf = nx->flags;
+                    const float nwx = nx->w_rf_x, nwy = nx->w_rf_y, nw2 = nx->w_rf2;
+                    rf_segment(tt, wrx, wry, wr2, !(f & HB_BOUND_ONLY));
+                    if (i < len && !(nf & HB_SAME_RF_OFFSET)) {
+                        const hb_segment qi = *nx;
+                        rf_offset(qi, pool ? rf_freq[s + i] : 0.0f);
+                        tt = 0.5f * qi.dt;
+                    }
+                    f = nf, wrx = nwx, wry = nwy, wr2 = nw2;
                 }
             }
-            __syncthreads();
-            if (r >= 0 && r < rows && tid < vals) {
-                float v = 0.0f;
-                if (tid < 2 * C) {
-                    v = red[0][tid];
-#pragma unroll
-                    for (int w = 1; w < kWavesM; ++w) v += red[w][tid];
+        } else {
+            free_factors(q, fl);
+            if (fl & HB_RUN) {  // len identical samples: Mxy stepped per sample, the longitudinal step once
+                const float T = (float)len * q.dt;
+                if (bits_differ(q.dt, run_dt) | (len ^ run_len)) {
+                    if (pool)
+                        xl = xstep(T, p.r1, b, 0.0f);
+                    else
+                        e1l = expm1x(-T * p.r1);
+                    run_dt = q.dt, run_len = len;
                 }
-                partial[((size_t)blockIdx.x * rows + r) * vals + tid] = v;
+                const int r0 = q.pad[0] - row0;
+                for (int i = 0; i < len; ++i) {
+                    precess();
+                    stage(r0 + i);
+                }
+                if (pool)
+                    exchange_free(xl, b, p.pd, p.r1, m, mb, lb);
+                else
+                    add_low(m.mz, m.lz, (m.mz - p.pd) * e1l);
+                s += len;
+                continue;
             }
-            __syncthreads();
+            precess();
+            if (pool)
+                exchange_free(xf, b, p.pd, p.r1, m, mb, lb);
+            else
+                add_low(m.mz, m.lz, (m.mz - p.pd) * e1f);
         }
+        if (fl & HB_ADC) stage(q.pad[0] - row0);
         if (fl & HB_SPOIL) m.mx = m.my = 0.0f;
+        s += len;
     }
+    if (nb > 0) flush<NT>(stg, wred, par, S, nt, nb, row, rows, partial);
     store_state(cs.state, np, j, m);
     if (pool) mt.mb[j] = mb, mt.mb[np + j] = lb;
 }
@@ -281,8 +362,8 @@ extern "C" int hb_forward_mt(const hb_case* cs, const hb_mt* mt, int32_t s0, int
     if (mt->pool && (!mt->mb || !mt->rf_freq)) return hipErrorInvalidValue;
     if (mt->conc_mode < HB_CONC_NONE || mt->conc_mode > HB_CONC_EXACT || (mt->conc_mode && !mt->conc))
         return hipErrorInvalidValue;
-    if (cs->n_pad <= 0 || cs->n_pad % kBlockM || cs->n < 0 || cs->n > cs->n_pad) return hipErrorInvalidValue;
-    if (cs->n_coils < 1 || cs->n_coils > kMaxCoilsM || cs->n_tiles < 1 || 8 * cs->n_tiles < cs->n_coils)
+    if (cs->n_pad <= 0 || cs->n_pad % kBlock || cs->n < 0 || cs->n > cs->n_pad) return hipErrorInvalidValue;
+    if (cs->n_coils < 1 || cs->n_coils > 8 * kMaxTiles || cs->n_tiles < 1 || 8 * cs->n_tiles < cs->n_coils)
         return hipErrorInvalidValue;
     if (s0 < 0 || s1 < s0 || s1 > cs->n_segments || rows < 0 || row0 < 0) return hipErrorInvalidValue;
     if (mt->pool && mt->lineshape == HB_LINE_SUPERLORENTZIAN && (!mt->table || mt->n_table < 2 || !(mt->dlx > 0.0f)))
@@ -290,20 +371,13 @@ extern "C" int hb_forward_mt(const hb_case* cs, const hb_mt* mt, int32_t s0, int
     if (mt->pool && mt->lineshape != HB_LINE_SUPERLORENTZIAN && mt->lineshape != HB_LINE_LORENTZIAN)
         return hipErrorInvalidValue;
     if (s1 == s0) return hipSuccess;
-    const dim3 grid(cs->n_pad / kBlockM), block(kBlockM);
-    hipStream_t st = (hipStream_t)stream;
-    const int C = cs->n_coils;
-    if (C <= 1)
-        hipLaunchKernelGGL(forward_mt_kernel<1>, grid, block, 0, st, *cs, *mt, s0, s1, partial, rows, row0);
-    else if (C <= 2)
-        hipLaunchKernelGGL(forward_mt_kernel<2>, grid, block, 0, st, *cs, *mt, s0, s1, partial, rows, row0);
-    else if (C <= 4)
-        hipLaunchKernelGGL(forward_mt_kernel<4>, grid, block, 0, st, *cs, *mt, s0, s1, partial, rows, row0);
-    else if (C <= 8)
-        hipLaunchKernelGGL(forward_mt_kernel<8>, grid, block, 0, st, *cs, *mt, s0, s1, partial, rows, row0);
-    else if (C <= 16)
-        hipLaunchKernelGGL(forward_mt_kernel<16>, grid, block, 0, st, *cs, *mt, s0, s1, partial, rows, row0);
-    else
-        hipLaunchKernelGGL(forward_mt_kernel<0>, grid, block, 0, st, *cs, *mt, s0, s1, partial, rows, row0);
+    if (cs->n_tiles > kMaxTiles) return hipErrorInvalidValue;
+    const dim3 grid(cs->n_pad / kBlock), block(kBlock);
+    const size_t lds = sizeof(float) * lds_floats(cs->n_tiles);
+    auto kernel = cs->n_tiles == 1   ? forward_mt_kernel<1>
+                  : cs->n_tiles == 2 ? forward_mt_kernel<2>
+                                     : forward_mt_kernel<0>;
+    hipLaunchKernelGGL(kernel, grid, block, lds, (hipStream_t)stream, *cs, *mt, s0, s1, partial, rows, row0, cs->segs,
+                       mt->sens, mt->rf_freq, mt->table);
     return hipGetLastError();
 }

@@ -523,7 +523,8 @@ def prepare_case(phantom: Phantom, seq: Sequence, coils=None, m_init=None, *, ch
     rows = [int(adc_cum[e] - adc_cum[s]) for s, e in zip(starts, ends)]
     rec = segment_table(seq, starts, reused, runs=not aligned and not full, nufft=plan)
     if full:
-        mt.mark_bound_only(rec, seq)
+        freq = mt.frequencies(phantom, seq)
+        mt.mark_records(rec, seq, starts, freq)
     covered = np.zeros(len(seq), dtype=bool)  # segments applied as reused-pulse maps
     for _, k, occ in reused:
         for a, _ in occ:
@@ -561,7 +562,7 @@ def prepare_case(phantom: Phantom, seq: Sequence, coils=None, m_init=None, *, ch
     if plan is not None:
         attach_nufft(case, plan, order, seq, adc_np, starts, ends, dev)
     if full:
-        mt.attach(case, phantom, seq, coils, m_init, n, n_pad, dev, conc)
+        mt.attach(case, phantom, coils, m_init, n, n_pad, dev, conc, freq)
     if surrogate and case.n_pulses:
         from . import surrogate as sur
 

@@ -14,6 +14,7 @@ plain path's.
 from __future__ import annotations
 
 import ctypes
+import math
 
 import numpy as np
 import torch
@@ -23,7 +24,7 @@ from ..sequence import flag_array
 from . import hip
 
 LINE = {"lorentzian": 1, "superlorentzian": 2}
-BOUND_ONLY = 262144  # HB_BOUND_ONLY of include/blochparty_amd_mt.h
+BOUND_ONLY, SAME_RF_OFFSET = 262144, 524288  # HB_BOUND_ONLY, HB_SAME_RF_OFFSET of include/blochparty_amd_mt.h
 
 
 class HbMt(ctypes.Structure):
@@ -51,9 +52,14 @@ def check_pool(bound: X.BoundPool) -> None:
         raise NotImplementedError("hip engine: a super-Lorentzian without its cut (cutoff=None) is not implemented")
 
 
-def attach(case, phantom, seq, coils, m_init, n: int, n_pad: int, dev, conc=None) -> None:
+def frequencies(phantom, seq) -> torch.Tensor | None:
+    """(S,) float32 RF frequencies as the kernels read them, or None without a bound pool (which alone uses them)."""
+    return None if phantom.bound is None else X.rf_frequency(seq).detach().float().cpu()
+
+
+def attach(case, phantom, coils, m_init, n: int, n_pad: int, dev, conc=None, freq=None) -> None:
     """The full variant's device buffers of ``case`` (``case.extra["mt"]``): the sensitivities, the bound pool's when
-    the phantom has one, and ``conc`` = (coefficients (N, 6 or 7), mode) of the concomitant fields."""
+    the phantom has one (``freq``: ``frequencies``), and ``conc`` = (coefficients (N, 6 or 7), mode) of the concomitant fields."""
     C = coils.shape[1]
     sens = torch.zeros(2 * C, n_pad, dtype=torch.float32)
     sens[0::2, :n] = coils.real.T.float().cpu()
@@ -66,11 +72,16 @@ def attach(case, phantom, seq, coils, m_init, n: int, n_pad: int, dev, conc=None
         coef[: conc[0].shape[1], :n] = conc[0].detach().float().cpu().T
         out.update(conc=coef.to(dev).contiguous(), conc_mode=int(conc[1]))
     if phantom.bound is not None:
-        out.update(_pool_buffers(phantom, seq, m_init, n, n_pad, dev))
+        out.update(_pool_buffers(phantom, freq, m_init, n, n_pad, dev))
+        # the exchange may bring the bound pool's magnetization into the free pool: its bound for the contraction
+        # (powers of two: the smaller scale serves both)
+        mb = float(out["mb"].abs().sum(0).max())
+        if mb > 0 and math.isfinite(mb):
+            case.x_scale = min(case.x_scale, math.ldexp(1.0, -min(100, max(-100, math.ceil(math.log2(mb)) + 1))))
     case.extra["mt"] = out
 
 
-def _pool_buffers(phantom, seq, m_init, n: int, n_pad: int, dev) -> dict:
+def _pool_buffers(phantom, rf_freq, m_init, n: int, n_pad: int, dev) -> dict:
     bound = phantom.bound
     check_pool(bound)
     like = phantom.pd.detach().double().cpu()
@@ -84,7 +95,6 @@ def _pool_buffers(phantom, seq, m_init, n: int, n_pad: int, dev) -> dict:
     mb = torch.zeros(2, n_pad, dtype=torch.float32)
     mb[0, :n] = mb64.float()
     mb[1, :n] = (mb64 - mb64.float().double()).float()
-    rf_freq = X.rf_frequency(seq).detach().float().cpu()
     lx0, dlx, logf = X.superlorentzian_table()
     return dict(pool=pool.float().to(dev).contiguous(), mb=mb.to(dev).contiguous(), mb0=mb.to(dev).contiguous(),
                 rf_freq=rf_freq.to(dev).contiguous(), table=torch.from_numpy(logf.astype(np.float32)).to(dev),
@@ -114,10 +124,30 @@ def needed(phantom, seq, conc=None) -> bool:
     return phantom.bound is not None or bound_only or (conc is not None and bool(conc[1]))
 
 
-def mark_bound_only(rec, seq) -> None:
-    """HB_BOUND_ONLY on the records of RF that only the bound pool feels (the water ignores it)."""
+def mark_records(rec, seq, starts, freq=None) -> None:
+    """The full variant's marks: HB_BOUND_ONLY on RF that only the bound pool feels (the water ignores it), readout runs
+    (HB_RUN), and HB_SAME_RF_OFFSET on RF segments whose duration, gradient, b0_offset and RF frequency (as the kernel
+    reads them, in float32; ``freq``: ``frequencies``) are those of the RF segment before them in the dispatch
+    (``starts``: its first segments)."""
+    from . import driver
+
+    flags = rec["flags"]
     if seq.bound_only is not None:
-        rec["flags"][flag_array(seq.bound_only)] |= BOUND_ONLY
+        flags[flag_array(seq.bound_only)] |= BOUND_ONLY
+    S = len(rec)
+    first = np.zeros(S, dtype=bool)
+    first[np.asarray(starts, dtype=np.int64)] = True
+    chunk_id = np.cumsum(first) - 1
+    is_rf, adc, spoil = (flags & bit != 0 for bit in (driver.RF, driver.ADC, driver.SPOIL))
+    key = rec["d"].copy()  # equal length and moments: equal gradient and b0_offset
+    driver.mark_runs(flags, rec, key, is_rf, adc, spoil, chunk_id, np.ones(S, dtype=bool))
+    idx = np.flatnonzero(is_rf)
+    if len(idx) > 1:
+        bits = np.ascontiguousarray(rec["f"][:, [0, 3, 4, 5, 6]])[idx].view(np.int32)
+        if freq is not None:
+            bits = np.concatenate([bits, freq.numpy()[idx].view(np.int32)[:, None]], 1)
+        same = (bits[1:] == bits[:-1]).all(1) & (chunk_id[idx[1:]] == chunk_id[idx[:-1]])
+        flags[idx[1:][same]] |= SAME_RF_OFFSET
 
 
-__all__ = ["HbMt", "attach", "bind", "check_pool", "forward_dispatch", "mark_bound_only", "needed", "struct"]
+__all__ = ["HbMt", "attach", "bind", "check_pool", "forward_dispatch", "mark_records", "needed", "struct"]
