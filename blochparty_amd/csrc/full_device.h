@@ -11,9 +11,9 @@
 //       w = -2 pi dt (b1 rf_x, b1 rf_y, bz) ((0, 0, w_z) for RF only the bound pool feels), the other half.
 //   free: precession by phi = -2 pi (r . m + db0 dt + b0_area + f_c dt) (m the segment's gradient moment), decay E2
 //       = exp(-dt R2), the unsaturated exchange X(dt, 0) (or T1 recovery).
-//   X(t, W): z' = z_ss + exp(A t) (z - z_ss), A = [[-(R1 + k f), k], [k f, -(R1b + k + W)]], c = (R1 PD, R1b f PD),
-//       z_ss = -A^-1 c; exp(A t) = P I + R (A - m I), m = tr A / 2, Q = (a11 - a22)^2 / 4 + a12 a21 >= 0,
-//       P = e^{m t} cosh(sqrt(Q) t), R = e^{m t} sinh(sqrt(Q) t) / sqrt(Q) (even in sqrt(Q): series for small Q t^2).
+//   X(t, W): z' = z + (exp(A t) - I) A^-1 (A z + c), A = [[-(R1 + k f), k], [k f, -(R1b + k + W)]], c = (R1 PD,
+//       R1b f PD): the increment al d + be (A - m I) d of the rates of change d = A z + c, m = tr A / 2, Q =
+//       (a11 - a22)^2 / 4 + a12 a21 >= 0 (Xch; series for short steps).
 // Reverse: for lambda = dL/d(state after), dL/d(state before) and the gradients of every parameter the step reads,
 // by hand-written reverse mode through the same intermediates (the rotation's as adjoint_device.h states it).
 #pragma once
@@ -50,6 +50,9 @@ struct Seg {
     double dt, rfx, rfy, gx, gy, gz, b0, frf;
     double mx, my, mz, b0a;  // float64 gradient moment and b0_offset area of the segment
     int flags;
+    // what the last segment of the kind that the cache has seen shares with this one: an RF segment's gradient,
+    // b0_offset and RF frequency (same_off) or length (same_dt), everything of a free segment (same_free)
+    bool same_off, same_dt, same_free;
 };
 
 struct Line {
@@ -129,83 +132,113 @@ HB_HD inline Conc conc_field(int mode, const double (&c)[7], double gx, double g
 }
 
 // ---- the exchange step X(t, W) of (Mz, Mzb) ----
+// The increment over t is al d + be (A - m I) d with d = A z + c the rates of change: al and be the mean and the divided
+// difference of f(lambda) = (e^{lambda t} - 1) / lambda over the eigenvalues m +- sqrt(Q) (no steady state, no division
+// on the short steps). al_m, be_m: d/dm; be_q: d be / dQ (d al / dQ = be_m / 2).
 struct Xch {
-    double a11, a12, a21, a22, c1, c2, inv, z1, z2, m, hh, Q, P, R, dRdQ, t;
+    double a11, a12, a21, a22, c1, c2, m, hh, Q, al, be, al_m, be_m, be_q, t;
 };
+
+// The series in x = m t, y = Q t^2: with S_n, D_n the mean and the divided difference of (x +- sqrt y)^n (S_{n+1} =
+// x S_n + y D_n, D_{n+1} = x D_n + S_n), al = t sum S_n / (n+1)!, be = t^2 sum D_n / (n+1)!; d/dx S_n = n S_{n-1},
+// d/dx D_n = n D_{n-1}, E_n = d/dy D_n: E_{n+1} = x E_n + n D_{n-1} / 2. N terms: truncation (|x| + sqrt y)^N / (N+1)!.
+template <int N>
+HB_HD inline void xch_series(Xch& X) {
+    const double t = X.t, x = X.m * t, y = X.Q * t * t;
+    double S = 1.0, D = 0.0, S1 = 0.0, D1 = 0.0, E = 0.0;  // S_n, D_n, S_{n-1}, D_{n-1}, E_n
+    double a = 1.0, b = 0.0, ax = 0.0, bx = 0.0, by = 0.0, f = 1.0;
+#if defined(__HIPCC__)
+#pragma unroll
+#endif
+    for (int n = 1; n < N; ++n) {
+        const double E2 = x * E + 0.5 * (n - 1) * D1, S2 = x * S + y * D, D2 = x * D + S;
+        S1 = S, D1 = D, S = S2, D = D2, E = E2;
+        f /= n + 1;
+        a += f * S, b += f * D;
+        ax += f * n * S1, bx += f * n * D1, by += f * E;
+    }
+    X.al = t * a, X.be = t * t * b;
+    X.al_m = t * t * ax, X.be_m = t * t * t * bx, X.be_q = t * t * t * t * by;
+}
 
 HB_HD inline Xch xch_setup(double t, double pd, double r1, double f, double k, double r1b, double w) {
     Xch X;
     X.t = t;
     X.a11 = -(r1 + k * f), X.a12 = k, X.a21 = k * f, X.a22 = -(r1b + k + w);
     X.c1 = r1 * pd, X.c2 = r1b * f * pd;
-    X.inv = 1.0 / (X.a11 * X.a22 - X.a12 * X.a21);  // det = R1 R1b + ... > 0 for R1 > 0
-    X.z1 = (X.a12 * X.c2 - X.a22 * X.c1) * X.inv;
-    X.z2 = (X.a21 * X.c1 - X.a11 * X.c2) * X.inv;
     X.m = 0.5 * (X.a11 + X.a22), X.hh = 0.5 * (X.a11 - X.a22);
     X.Q = X.hh * X.hh + X.a12 * X.a21;
-    const double x = X.Q * t * t;
-    if (x < 0.01) {  // cosh, sinh / q and d(sinh / q)/dQ by their series in x = Q t^2 (truncation < 3e-14)
-        const double E = exp(X.m * t);
-        const double C = 1.0 + x * (1.0 / 2 + x * (1.0 / 24 + x * (1.0 / 720 + x * (1.0 / 40320 + x / 3628800))));
-        const double S = t * (1.0 + x * (1.0 / 6 + x * (1.0 / 120 + x * (1.0 / 5040 + x * (1.0 / 362880)))));
-        const double dS = t * t * t *
-                          (1.0 / 6 + x * (1.0 / 60 + x * (1.0 / 1680 + x * (1.0 / 90720 + x * (1.0 / 7983360)))));
-        X.P = E * C, X.R = E * S, X.dRdQ = E * dS;
-    } else {  // both eigenvalues m +- q are <= 0: no overflow
-        const double q = sqrt(X.Q);
-        const double e1 = exp((X.m + q) * t), e2 = exp((X.m - q) * t);
-        X.P = 0.5 * (e1 + e2), X.R = 0.5 * (e1 - e2) / q;
-        X.dRdQ = (t * X.P - X.R) / (2.0 * X.Q);
+    const double rho = -2.0 * X.m * t;  // |lambda t| is at most this (both eigenvalues are <= 0)
+    if (rho < 0.002) {
+        xch_series<5>(X);  // an RF substep
+    } else if (rho < 0.05) {
+        xch_series<8>(X);
+    } else if (rho < 0.5) {
+        xch_series<13>(X);
+    } else {  // from exp(A t) = P I + R (A - m I): P = 1 + m al + Q be, R = al + m be
+        const double x = X.Q * t * t;
+        double P, R, dR;  // e^{mt} cosh(qt), e^{mt} sinh(qt) / q, dR/dQ
+        if (x < 0.01) {   // by their series in x = Q t^2 (truncation < 3e-14)
+            const double E = exp(X.m * t);
+            P = E * (1.0 + x * (1.0 / 2 + x * (1.0 / 24 + x * (1.0 / 720 + x * (1.0 / 40320 + x / 3628800)))));
+            R = E * t * (1.0 + x * (1.0 / 6 + x * (1.0 / 120 + x * (1.0 / 5040 + x * (1.0 / 362880)))));
+            dR = E * t * t * t *
+                 (1.0 / 6 + x * (1.0 / 60 + x * (1.0 / 1680 + x * (1.0 / 90720 + x * (1.0 / 7983360)))));
+        } else {  // both eigenvalues m +- q are <= 0: no overflow
+            const double q = sqrt(X.Q);
+            const double e1 = exp((X.m + q) * t), e2 = exp((X.m - q) * t);
+            P = 0.5 * (e1 + e2), R = 0.5 * (e1 - e2) / q;
+            dR = (t * P - R) / (2.0 * X.Q);
+        }
+        const double det = r1 * (r1b + k + w) + k * f * (r1b + w), i = 1.0 / det;  // m^2 - Q > 0 for R1 > 0
+        X.al = (X.m * (P - 1.0) - X.Q * R) * i;
+        X.be = (X.m * R - (P - 1.0)) * i;
+        X.al_m = ((P - 1.0) + X.m * t * P - X.Q * t * R - 2.0 * X.m * X.al) * i;
+        X.be_m = (R + X.m * t * R - t * P - 2.0 * X.m * X.be) * i;
+        X.be_q = (X.m * dR - 0.5 * t * R + X.be) * i;
     }
     return X;
 }
 
 HB_HD inline void xch_apply(const Xch& X, double& z, double& b) {
-    const double d1 = z - X.z1, d2 = b - X.z2;
-    z = X.z1 + X.P * d1 + X.R * (X.hh * d1 + X.a12 * d2);
-    b = X.z2 + X.P * d2 + X.R * (X.a21 * d1 - X.hh * d2);
+    const double d1 = X.a11 * z + X.a12 * b + X.c1, d2 = X.a21 * z + X.a22 * b + X.c2;
+    z += X.al * d1 + X.be * (X.hh * d1 + X.a12 * d2);
+    b += X.al * d2 + X.be * (X.a21 * d1 - X.hh * d2);
+}
+
+// The transpose of xch_apply's linear part, on l = dL/d(after): the gradients (g1, g2) along the rates of change.
+HB_HD inline void xch_transpose(const Xch& X, double& lz, double& lb, double& g1, double& g2) {
+    g1 = lz * (X.al + X.be * X.hh) + lb * X.be * X.a21;
+    g2 = lz * X.be * X.a12 + lb * (X.al - X.be * X.hh);
+    lz += X.a11 * g1 + X.a21 * g2;
+    lb += X.a12 * g1 + X.a22 * g2;
 }
 
 // Reverse of xch_apply (set up from p's pool) from the state (z, b) before it: (lz, lb) = dL/d(after) in,
 // dL/d(before) out. The gradients along pd, R1, f, k, R1b, W and t are added to g[0..6].
 HB_HD inline void xch_reverse(const Xch& X, const Params& p, double z, double b, double& lz, double& lb,
                               double (&g)[7]) {
-    const double d1 = z - X.z1, d2 = b - X.z2;
+    const double d1 = X.a11 * z + X.a12 * b + X.c1, d2 = X.a21 * z + X.a22 * b + X.c2;
     const double Lz = lz, Lb = lb;
-    const double bP = Lz * d1 + Lb * d2;
-    const double bR = Lz * (X.hh * d1 + X.a12 * d2) + Lb * (X.a21 * d1 - X.hh * d2);
-    const double bd1 = Lz * (X.P + X.R * X.hh) + Lb * X.R * X.a21;
-    const double bd2 = Lz * X.R * X.a12 + Lb * (X.P - X.R * X.hh);
-    double bhh = X.R * (Lz * d1 - Lb * d2);
-    double b12 = Lz * X.R * d2, b21 = Lb * X.R * d1;
-    const double bz1 = Lz - bd1, bz2 = Lb - bd2;
-    lz = bd1, lb = bd2;
-    const double bm = X.t * (bP * X.P + bR * X.R);
-    const double bQ = bP * 0.5 * X.t * X.R + bR * X.dRdQ;
-    const double bt = bP * (X.m * X.P + X.Q * X.R) + bR * (X.m * X.R + X.P);
-    bhh += 2.0 * X.hh * bQ;
-    b12 += X.a21 * bQ;
-    b21 += X.a12 * bQ;
-    double b11 = 0.5 * (bm + bhh), b22 = 0.5 * (bm - bhh);
-    const double bc1 = (-X.a22 * bz1 + X.a21 * bz2) * X.inv;
-    const double bc2 = (X.a12 * bz1 - X.a11 * bz2) * X.inv;
-    const double bdet = -(X.z1 * bz1 + X.z2 * bz2) * X.inv;
-    b12 += X.c2 * bz1 * X.inv;
-    b22 -= X.c1 * bz1 * X.inv;
-    b21 += X.c1 * bz2 * X.inv;
-    b11 -= X.c2 * bz2 * X.inv;
-    b11 += X.a22 * bdet;
-    b22 += X.a11 * bdet;
-    b12 -= X.a21 * bdet;
-    b21 -= X.a12 * bdet;
+    const double bal = Lz * d1 + Lb * d2;
+    const double bbe = Lz * (X.hh * d1 + X.a12 * d2) + Lb * (X.a21 * d1 - X.hh * d2);
+    double b1, b2;  // dL/d(d1, d2), also dL/d(c1, c2)
+    xch_transpose(X, lz, lb, b1, b2);
+    const double bm = bal * X.al_m + bbe * X.be_m;
+    const double bQ = 0.5 * bal * X.be_m + bbe * X.be_q;
+    const double R = X.al + X.m * X.be;  // d be / dt; d al / dt = 1 + m al + Q be
+    const double bt = bal * (1.0 + X.m * X.al + X.Q * X.be) + bbe * R;
+    const double bhh = X.be * (Lz * d1 - Lb * d2) + 2.0 * X.hh * bQ;
+    const double b11 = b1 * z + 0.5 * (bm + bhh), b22 = b2 * b + 0.5 * (bm - bhh);
+    const double b12 = b1 * b + X.be * Lz * d2 + X.a21 * bQ, b21 = b2 * z + X.be * Lb * d1 + X.a12 * bQ;
     // a11 = -(R1 + k f), a12 = k, a21 = k f, a22 = -(R1b + k + W), c1 = R1 PD, c2 = R1b f PD
-    g[0] += p.r1 * bc1 + p.r1b * p.f * bc2;                     // pd
-    g[1] += -b11 + p.pd * bc1;                                  // R1
-    g[2] += p.k * (b21 - b11) + p.r1b * p.pd * bc2;             // f
-    g[3] += -p.f * b11 + b12 + p.f * b21 - b22;                 // k
-    g[4] += -b22 + p.f * p.pd * bc2;                            // R1b
-    g[5] += -b22;                                               // W
-    g[6] += bt;                                              // t
+    g[0] += p.r1 * b1 + p.r1b * p.f * b2;                     // pd
+    g[1] += -b11 + p.pd * b1;                                 // R1
+    g[2] += p.k * (b21 - b11) + p.r1b * p.pd * b2;            // f
+    g[3] += -p.f * b11 + b12 + p.f * b21 - b22;               // k
+    g[4] += -b22 + p.f * p.pd * b2;                           // R1b
+    g[5] += -b22;                                             // W
+    g[6] += bt;                                               // t
 }
 
 // ---- rotation by w: R(w) m = m + s1 (w x m) + s2 w x (w x m) ----
@@ -289,30 +322,34 @@ HB_HD inline void longitudinal(const Model& md, const Params& p, const Xch& X, d
         z = p.pd + (z - p.pd) * e1;
 }
 
-// Factors that depend only on a segment's length and the spin, kept while consecutive segments of the kind have the
-// same dt: the free segment's decay and unsaturated exchange, the RF segment's half-step decay.
+// Factors kept from segment to segment: those that depend only on a segment's length and the spin while consecutive
+// segments of the kind have the same dt (the free segment's decay and unsaturated exchange, the RF segment's half-step
+// decay), the free segment's precession while same_free, and the saturation's lineshape with its derivatives while
+// same_off says that the offset and the RF frequency stay.
 struct Cache {
     double free_dt, rf_dt;  // the lengths the factors belong to (< 0: none yet)
-    double fe2, fe1, re2, re1;
+    double fe2, fe1, re2, re1, sn, cs;
+    double G, gd, gt;
     Xch fx;
 };
 
 HB_HD inline Cache no_cache() {
     Cache c;
     c.free_dt = c.rf_dt = -1.0;
-    c.fe2 = c.fe1 = c.re2 = c.re1 = 0.0;
+    c.fe2 = c.fe1 = c.re2 = c.re1 = c.sn = c.cs = 0.0;
+    c.G = c.gd = c.gt = 0.0;
     return c;
 }
 
-HB_HD inline Step step(const Model& md, const Params& p, const Seg& q, const St& m0, Cache& k) {
+// What a segment does that does not depend on the state.
+HB_HD inline Step set_up(const Model& md, const Params& p, const Seg& q, Cache& k) {
     Step s;
     s.lin = p.px * q.gx + p.py * q.gy + p.pz * q.gz + p.db0 + q.b0;
     s.cc = conc_field(md.conc, p.cc, q.gx, q.gy, q.gz, s.lin);
     s.bz = s.lin + s.cc.fc;
-    St m = m0;
     if (q.flags & kRf) {
         const double h = 0.5 * q.dt;
-        if (k.rf_dt != q.dt) {
+        if (!q.same_dt && k.rf_dt != q.dt) {
             k.re2 = exp(-h * p.r2);
             k.re1 = md.pool ? 1.0 : exp(-h * p.r1);
             k.rf_dt = q.dt;
@@ -320,27 +357,24 @@ HB_HD inline Step step(const Model& md, const Params& p, const Seg& q, const St&
         s.e2 = k.re2, s.e1 = k.re1;
         if (md.pool) {
             s.Wk = kTwoPi * kTwoPi * p.b1 * p.b1 * (q.rfx * q.rfx + q.rfy * q.rfy);
-            s.G = line_g(md.line, q.frf - s.bz - p.dw, p.t2b, s.gd, s.gt);
+            if (!q.same_off) k.G = line_g(md.line, q.frf - s.bz - p.dw, p.t2b, k.gd, k.gt);
+            s.G = k.G, s.gd = k.gd, s.gt = k.gt;
             s.W = s.Wk * s.G;
             s.X = xch_setup(h, p.pd, p.r1, p.f, p.k, p.r1b, s.W);
         }
-        m.x *= s.e2, m.y *= s.e2;
-        longitudinal(md, p, s.X, s.e1, m.z, m.b);
-        s.m1 = m;
         const bool water = !(q.flags & kBoundOnly);
         s.w[0] = water ? -kTwoPi * q.dt * p.b1 * q.rfx : 0.0;
         s.w[1] = water ? -kTwoPi * q.dt * p.b1 * q.rfy : 0.0;
         s.w[2] = -kTwoPi * q.dt * s.bz;
         s.rot = rot_factors(s.w[0] * s.w[0] + s.w[1] * s.w[1] + s.w[2] * s.w[2]);
-        rotate(s.rot, s.w[0], s.w[1], s.w[2], m.x, m.y, m.z);
-        s.m2 = m;
-        m.x *= s.e2, m.y *= s.e2;
-        longitudinal(md, p, s.X, s.e1, m.z, m.b);
     } else {
-        double cyc = p.px * q.mx + p.py * q.my + p.pz * q.mz + p.db0 * q.dt + q.b0a + s.cc.fc * q.dt;
-        cyc -= rint(cyc);
-        sincospi_d(-2.0 * cyc, &s.sn, &s.cs);
-        if (k.free_dt != q.dt) {
+        if (!q.same_free) {
+            double cyc = p.px * q.mx + p.py * q.my + p.pz * q.mz + p.db0 * q.dt + q.b0a + s.cc.fc * q.dt;
+            cyc -= rint(cyc);
+            sincospi_d(-2.0 * cyc, &k.sn, &k.cs);
+        }
+        s.sn = k.sn, s.cs = k.cs;
+        if (!q.same_free && k.free_dt != q.dt) {
             k.fe2 = exp(-q.dt * p.r2);
             k.fe1 = md.pool ? 1.0 : exp(-q.dt * p.r1);
             if (md.pool) k.fx = xch_setup(q.dt, p.pd, p.r1, p.f, p.k, p.r1b, 0.0);
@@ -348,11 +382,57 @@ HB_HD inline Step step(const Model& md, const Params& p, const Seg& q, const St&
         }
         s.e2 = k.fe2, s.e1 = k.fe1;
         if (md.pool) s.X = k.fx;
+    }
+    return s;
+}
+
+// The state through the segment set up in s (its intermediates and s.after).
+HB_HD inline void advance(const Model& md, const Params& p, const Seg& q, const St& m0, Step& s) {
+    St m = m0;
+    if (q.flags & kRf) {
+        m.x *= s.e2, m.y *= s.e2;
+        longitudinal(md, p, s.X, s.e1, m.z, m.b);
+        s.m1 = m;
+        rotate(s.rot, s.w[0], s.w[1], s.w[2], m.x, m.y, m.z);
+        s.m2 = m;
+        m.x *= s.e2, m.y *= s.e2;
+        longitudinal(md, p, s.X, s.e1, m.z, m.b);
+    } else {
         s.ux = s.cs * m.x - s.sn * m.y, s.uy = s.sn * m.x + s.cs * m.y;
         m.x = s.e2 * s.ux, m.y = s.e2 * s.uy;
         longitudinal(md, p, s.X, s.e1, m.z, m.b);
     }
     s.after = m;
+}
+
+// The transpose of advance alone: l = dL/d(after) in (spoil and ADC source applied), dL/d(before) out.
+HB_HD inline void retreat(const Model& md, const Seg& q, const Step& s, St& l) {
+    auto lon = [&]() {
+        if (md.pool) {
+            double g1, g2;
+            xch_transpose(s.X, l.z, l.b, g1, g2);
+        } else {
+            l.z *= s.e1;
+        }
+    };
+    if (q.flags & kRf) {
+        l.x *= s.e2, l.y *= s.e2;
+        lon();
+        Rot back = s.rot;  // R(w)^T = R(-w)
+        rotate(back, -s.w[0], -s.w[1], -s.w[2], l.x, l.y, l.z);
+        l.x *= s.e2, l.y *= s.e2;
+        lon();
+    } else {
+        const double x = s.e2 * l.x, y = s.e2 * l.y;
+        l.x = s.cs * x + s.sn * y;
+        l.y = s.cs * y - s.sn * x;
+        lon();
+    }
+}
+
+HB_HD inline Step step(const Model& md, const Params& p, const Seg& q, const St& m0, Cache& k) {
+    Step s = set_up(md, p, q, k);
+    advance(md, p, q, m0, s);
     return s;
 }
 

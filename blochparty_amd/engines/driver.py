@@ -532,8 +532,11 @@ def prepare_case(phantom: Phantom, seq: Sequence, coils=None, m_init=None, *, ch
     rf_cum = np.concatenate([[0], np.cumsum(flag_array(seq.is_rf) & ~covered)])
     # the coil contraction's scales: |M| <= max(PD, |m_init|) along any sequence (rotations keep |M|, relaxation
     # moves it toward (0, 0, PD))
-    sens_a = sens_operand(coils, n, n_pad, n_tiles)
-    sens_scale = pow2_scale(float(sens_a.abs().max()) if sens_a.numel() else 0.0)
+    if full:  # its kernels read the sensitivities in rows (mt.attach)
+        sens_a, largest = torch.zeros(0, dtype=torch.float32), torch.view_as_real(coils.detach().to(torch.complex128))
+    else:
+        sens_a = largest = sens_operand(coils, n, n_pad, n_tiles)
+    sens_scale = pow2_scale(float(largest.abs().max()) if largest.numel() else 0.0)
     x_scale = pow2_scale(max(float(phantom.pd.detach().abs().max()) if n else 0.0,
                              float((m64[0] * m64[0] + m64[1] * m64[1] + m64[2] * m64[2]).max().sqrt()) if n
                              else 0.0))

@@ -202,6 +202,8 @@ def _sweep(case, ckpts, every, h, lam, sens, nc, need_seg, need_coil, gs, gc, se
     gseg = torch.empty(n_blocks * every * 8 if need_seg else 1, dtype=torch.float32, device=dev)
     red = torch.empty(max(1, -(-n_blocks // SEG_CHUNK) * every * 8 if need_seg else 1), dtype=torch.float64,
                       device=dev)
+    need = lib.hb_adjoint_full_workspace(n_pad, every, nc)
+    work = torch.empty(need, dtype=torch.float64, device=dev) if need else None
     stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
     for c in reversed(range(len(ckpts))):
         s0, s1 = case.starts[c], case.ends[c]
@@ -209,9 +211,10 @@ def _sweep(case, ckpts, every, h, lam, sens, nc, need_seg, need_coil, gs, gc, se
         ad = HbFullAdjoint(ck.data_ptr(), ck[6].data_ptr() if pool else None, traj.data_ptr(), lam.data_ptr(),
                            gs.data_ptr(), gc.data_ptr(), gseg.data_ptr(), h.data_ptr(), sens.data_ptr(), nc, every,
                            int(need_coil), int(need_seg))
-        rc = lib.hb_adjoint_full(ctypes.byref(cs), ctypes.byref(mts), ctypes.byref(ad), s0, s1, stream)
+        rc = lib.hb_adjoint_full_chunks(ctypes.byref(cs), ctypes.byref(mts), ctypes.byref(ad), s0, s1,
+                                        None if work is None else work.data_ptr(), stream)
         if rc != 0:
-            raise RuntimeError(f"HIP error {rc} in hb_adjoint_full: {lib.hb_error_string(rc).decode()}")
+            raise RuntimeError(f"HIP error {rc} in hb_adjoint_full_chunks: {lib.hb_error_string(rc).decode()}")
         if need_seg:
             kern.seg_reduce(gseg.data_ptr(), n_blocks, every, s0, s1 - s0, red.data_ptr(), seg.data_ptr(), None)
 

@@ -43,6 +43,10 @@ def bind(lib) -> None:
     lib.hb_adjoint_full.restype = ctypes.c_int
     lib.hb_adjoint_full.argtypes = [ctypes.POINTER(hip.HbCase), ctypes.POINTER(HbMt), ctypes.c_void_p, ctypes.c_int32,
                                     ctypes.c_int32, ctypes.c_void_p]
+    lib.hb_adjoint_full_chunks.restype = ctypes.c_int
+    lib.hb_adjoint_full_chunks.argtypes = [*lib.hb_adjoint_full.argtypes[:-1], ctypes.c_void_p, ctypes.c_void_p]
+    lib.hb_adjoint_full_workspace.restype = ctypes.c_int64
+    lib.hb_adjoint_full_workspace.argtypes = [ctypes.c_int32] * 3
 
 
 def check_pool(bound: X.BoundPool) -> None:
@@ -140,7 +144,9 @@ def mark_records(rec, seq, starts, freq=None) -> None:
     chunk_id = np.cumsum(first) - 1
     is_rf, adc, spoil = (flags & bit != 0 for bit in (driver.RF, driver.ADC, driver.SPOIL))
     key = rec["d"].copy()  # equal length and moments: equal gradient and b0_offset
+    hints = flags & (driver.SAME_FREE | driver.NEXT_FREE)  # of the runs' inner segments: the adjoint walks them
     driver.mark_runs(flags, rec, key, is_rf, adc, spoil, chunk_id, np.ones(S, dtype=bool))
+    flags |= hints
     idx = np.flatnonzero(is_rf)
     if len(idx) > 1:
         bits = np.ascontiguousarray(rec["f"][:, [0, 3, 4, 5, 6]])[idx].view(np.int32)

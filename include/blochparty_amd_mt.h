@@ -92,6 +92,14 @@ typedef struct hb_full_adjoint {
 int hb_adjoint_full(const hb_case* cs, const hb_mt* mt, const hb_full_adjoint* ad, int32_t s0, int32_t s1,
                     void* stream);
 
+/* The same with a workspace of hb_adjoint_full_workspace(n_pad, k_max, nc) doubles: where the case has too few spins to
+ * fill the chip, the interval is reversed in chunks of segments side by side, from the adjoint at each chunk's end
+ * (found by a sweep of its own beside the replay); the chunks' gradients are added in a fixed order. work NULL, or a
+ * workspace of 0 doubles (which may be NULL): as hb_adjoint_full. */
+int64_t hb_adjoint_full_workspace(int32_t n_pad, int32_t k_max, int32_t nc);
+int hb_adjoint_full_chunks(const hb_case* cs, const hb_mt* mt, const hb_full_adjoint* ad, int32_t s0, int32_t s1,
+                           double* work, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

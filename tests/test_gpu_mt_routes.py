@@ -126,3 +126,58 @@ def test_marks():
             assert torch.equal(seq.grad[s:s + n], seq.grad[s].expand(n, 3))
         if chunk == S:
             assert [n for _, n in runs] == [n - (i % 4 == 3) for i, n in enumerate(SPANS) if n - (i % 4 == 3) >= 4]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_spins,coils,every", [(40, 1, 64), (300, 5, 64), (600, 16, 192), (256, 0, 128)])
+@pytest.mark.parametrize("lineshape", ["superlorentzian", "none"])
+def test_reverse_in_chunks(gpu, n_spins, coils, every, lineshape):
+    """hb_adjoint_full_chunks with a workspace (the interval reversed in chunks side by side) against hb_adjoint_full
+    (one walk): the same float64 sums in another grouping, lambda carried in float64 either way, so 1e-9 of the largest
+    (per-segment sums: the float32 partials' rounding, 1e-6)."""
+    import ctypes
+
+    from blochparty_amd.engines import adjoint, driver, full_adjoint, hip, mt
+
+    if lineshape == "none":
+        ph = replace(pooled(n_spins, 3), bound=None)
+    else:
+        ph = pooled(n_spins, 3, lineshape)
+    seq = blocks(SPANS, TRAINS)
+    g = torch.Generator().manual_seed(1)
+    conc = (1e-7 * torch.randn(n_spins, 6, generator=g, dtype=f64), 1)
+    c = torch.complex(*torch.randn(2, n_spins, max(coils, 1), generator=g, dtype=f64))
+    case = driver.prepare_case(ph, seq, c, chunk=every, aligned=True, conc=conc)
+    ckpts = driver.run_forward(case, keep=True)
+    nc = adjoint.adjoint_width(coils) if coils else 0
+    sens = adjoint.adjoint_sens(c, case.n_pad, nc).cuda()
+    h = torch.randn(case.n_adc, max(nc, 1), 2, generator=g).cuda()
+    h[:, coils:] = 0
+    lam0 = torch.randn(4, case.n_pad, generator=g).cuda()
+    lam0[:, n_spins:] = 0
+    lib = hip.load()
+    mt.bind(lib)
+    cs, mts = case.struct(), mt.struct(case.extra["mt"])
+    z = lambda *s: torch.zeros(*s, dtype=f64, device="cuda")
+    outs = []
+    for chunks in (False, True):
+        gs, gc, lam = z(20, case.n_pad), z(2 * max(nc, 1), case.n_pad), lam0.clone()
+        n_blocks = case.n_pad // 256
+        traj = torch.empty(every * 4 * case.n_pad, device="cuda")
+        gseg = torch.zeros(len(ckpts), n_blocks, every, 8, device="cuda")
+        need = lib.hb_adjoint_full_workspace(case.n_pad, every, nc)
+        assert need > 0
+        work = torch.full((need,), float("nan"), dtype=f64, device="cuda")
+        for i in reversed(range(len(ckpts))):
+            ad = full_adjoint.HbFullAdjoint(ckpts[i].data_ptr(), ckpts[i][6].data_ptr() if ph.bound else None,
+                                            traj.data_ptr(), lam.data_ptr(), gs.data_ptr(), gc.data_ptr(),
+                                            gseg[i].data_ptr(), h.data_ptr(), sens.data_ptr(), nc, every, 1, 1)
+            rc = lib.hb_adjoint_full_chunks(ctypes.byref(cs), ctypes.byref(mts), ctypes.byref(ad), case.starts[i],
+                                            case.ends[i], work.data_ptr() if chunks else None, None)
+            assert rc == 0
+        torch.cuda.synchronize()
+        outs.append((gs[:, :n_spins].cpu(), gc[:, :n_spins].cpu(), lam[:, :n_spins].cpu().double(),
+                     gseg.sum(1).cpu().double()))
+    for a, b, tol in zip(*outs, (1e-9, 1e-9, 1e-6, 1e-6)):
+        scale = a.abs().amax(-1, keepdim=True).clamp_min(1e-300)
+        assert bool(((a - b).abs() <= tol * scale.max() if a.ndim > 2 else (a - b).abs() <= tol * scale).all())
