@@ -12,9 +12,9 @@
 // order. No atomics: the signal is the same bit for bit on every run.
 //
 // Precision of the product: for up to two tiles (16 coils) both operands are split into float16 pairs, x = hi + lo
-// (x scaled into [-1, 1] by powers of two), and D = Ah Bh + Ah Bl + Al Bh on v_mfma_f32_16x16x32_f16: float16
-// products are exact in the float32 accumulator, and the pairs hold each operand to 2^-24 relative (2^-25 absolute
-// below 1/4), so D is as close to the exact sum as a float32 product would be, at six 16-cycle instructions per tile
+// (x scaled into [-2^8, 2^8] by powers of two), and D = Ah Bh + Ah Bl + Al Bh on v_mfma_f32_16x16x32_f16: float16
+// products are exact in the float32 accumulator, and the pairs hold each operand to 2^-24 relative (2^-33 of the bound
+// at least), so D is as close to the exact sum as a float32 product would be, at six 16-cycle instructions per tile
 // and flush in place of sixteen 32-cycle v_mfma_f32_16x16x4f32. More tiles use the float32 instruction, with the
 // sensitivities read from memory.
 #pragma once
@@ -38,13 +38,17 @@ constexpr int kMaxTiles = 16;   // 128 coils: LDS = 4 x 16 x 68 + 4 x 8 x 256 fl
 // LDS: every wave's staging block, then two buffers of the waves' coil sums (flushes alternate between them).
 __host__ __device__ constexpr int lds_floats(int nt) { return kWaves * kStgFloats + 2 * kWaves * 8 * 16 * nt; }
 
+// Float16's smallest step is 2^-24, so the low part of a value scaled to 2^-6 of the bound would keep it to 2^-19 only:
+// the operands are lifted by this power of two (undone exactly by out_scale), which leaves 2^8 above the bound.
+constexpr float kLift = 256.0f;
+
 // x of lane (jj + 8) mod 16 of this lane's row of 16 (DPP row_ror:8).
 __device__ __forceinline__ float dpp_ror8(float x) {
     return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0x128, 0xf, 0xf, false));
 }
 
 // x = hi + lo in float16 for eight floats: hi rounded to nearest, lo the rounded remainder (exact in float32). For
-// |x| <= 1 the pair holds x to 2^-24 |x| or 2^-25, whichever is larger (lo may be subnormal: the matrix cores take
+// |x| < 65504 the pair holds x to 2^-24 |x| or 2^-25, whichever is larger (lo may be subnormal: the matrix cores take
 // float16 subnormals as they are).
 __device__ __forceinline__ void split8(const float* x, h8& hi, h8& lo) {
 #pragma unroll
@@ -80,10 +84,15 @@ struct Sens {
     }
 
     // sa, st, su and n_rows are set; x_scale_ and sens_scale as hb_case's (0 reads as 1)
-    __device__ __forceinline__ void load(float x_scale_, float sens_scale, int lane) {
+    __device__ __forceinline__ void scales(float x_scale_, float& sens_scale) {
         x_scale = x_scale_ > 0.0f ? x_scale_ : 1.0f;
         if (!(sens_scale > 0.0f)) sens_scale = 1.0f;
+        if (NT > 0) x_scale *= kLift, sens_scale *= kLift;
         out_scale = 1.0f / (NT > 0 ? x_scale * sens_scale : x_scale);
+    }
+
+    __device__ __forceinline__ void load(float x_scale_, float sens_scale, int lane) {
+        scales(x_scale_, sens_scale);
         if constexpr (NT > 0) {
 #pragma unroll
             for (int t = 0; t < NT; ++t)
@@ -97,6 +106,18 @@ struct Sens {
         }
     }
 };
+
+// The wave's complex coil sums of tile t from its product acc, into mine in the output order [sample][tile][coil][re, im].
+__device__ __forceinline__ void store_pq(float* mine, int vals, int t, int lane, const f4& acc) {
+    const int g = lane >> 4, jj = lane & 15;
+    // rows 4 g .. 4 g + 3 of lane (g, jj) are Re S_c0, Im S_c0, Re S_c1, Im S_c1 (c0 = 2 g, c1 = 2 g + 1) at
+    // column jj; the partner column jj +- 8 sits in the same row of 16 lanes: DPP row_ror:8. Lanes jj < 8 form
+    // coil c0's (P, Q) at sample jj, lanes jj >= 8 coil c1's at sample jj - 8.
+    const float r0 = dpp_ror8(acc[0]), r1 = dpp_ror8(acc[1]), r2 = dpp_ror8(acc[2]), r3 = dpp_ror8(acc[3]);
+    const bool first = jj < 8;
+    const f2 pq = first ? (f2){acc[0] - r1, r0 + acc[1]} : (f2){r2 - acc[3], acc[2] + r3};
+    *reinterpret_cast<f2*>(mine + (jj & 7) * vals + 16 * t + 2 * (2 * g + (jj >> 3))) = pq;  // one 8-byte store
+}
 
 // The coil sums of the nb (<= 8) staged samples of every wave, added over the workgroup, into the partial rows
 // [row, row + nb) of this workgroup. Every lane of the workgroup calls it. One barrier: a wave reads only its own
@@ -146,14 +167,7 @@ __device__ __forceinline__ void flush_to(float* stg, float* wred2, int& par, con
             for (int u = 0; u < 16; ++u)
                 acc = __builtin_amdgcn_mfma_f32_16x16x4f32(S.at(t, u, jj), b[u], acc, 0, 0, 0);
         }
-        // rows 4 g .. 4 g + 3 of lane (g, jj) are Re S_c0, Im S_c0, Re S_c1, Im S_c1 (c0 = 2 g, c1 = 2 g + 1) at
-        // column jj; the partner column jj +- 8 sits in the same row of 16 lanes: DPP row_ror:8. Lanes jj < 8 form
-        // coil c0's (P, Q) at sample jj, lanes jj >= 8 coil c1's at sample jj - 8.
-        const float r0 = dpp_ror8(acc[0]), r1 = dpp_ror8(acc[1]), r2 = dpp_ror8(acc[2]), r3 = dpp_ror8(acc[3]);
-        const bool first = jj < 8;
-        const f2 pq = first ? (f2){acc[0] - r1, r0 + acc[1]} : (f2){r2 - acc[3], acc[2] + r3};
-        // this wave's sums in the output order [sample][tile][coil][re, im]: one 8-byte store per lane
-        *reinterpret_cast<f2*>(mine + (jj & 7) * vals + 16 * t + 2 * (2 * g + (jj >> 3))) = pq;
+        store_pq(mine, vals, t, lane, acc);
     }
     __syncthreads();
     // columns [0, k_first) to out, [k_first, k_first + k_skip) dropped, the rest to out_rest (output value

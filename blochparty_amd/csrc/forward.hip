@@ -97,14 +97,247 @@ __device__ __forceinline__ void nufft_run(const hb_case& cs, const hb_nufft& nu,
     run_jump(q, p, cyc, e1_run, m);
 }
 
-// NT: coil tiles (0: any, the sensitivities read from memory per flush); NUT: NUFFT runs with up to NUT decay terms
-// (0: none; the terms' weights are held in registers); RF: RF segments are stepped (false when every pulse of the
+// ---- NUFFT runs whose windows hold at most kCols columns (cells x terms): the spreading as one matrix product.
+//
+// A spin's weight on each column, psi(cell) e^{-R2 tau_m}, is real and the same for every run of a kind (one phase per
+// sample), so it is formed once per kind and kept in registers as matrix-core operands (kCols x 64 spins per wave, as
+// float16 hi and lo parts); so is the start's phase factor. Per run the lanes then only form S_c c (c = Mxy times that
+// factor) for every coil: lane (g, jj) the value jj (Re S_0 c, Im S_0 c, ...) of spins 16 g .. 16 g + 15, from the
+// sensitivities it and its neighbour lane keep for those spins and c broadcast through LDS, so that the products come
+// out in the operand layout. D[value][column] = sum over spins (S_c c) w on v_mfma_f32_16x16x32_f16 (three products
+// of hi and lo parts, as the samples'), 12 per coil tile; the waves' sums are added in LDS in a fixed order. Where a
+// run's window was staged column by column (nufft_run: three flushes, each splitting 16 values per lane anew, and the
+// window's kernel values and two sines of a float64 phase per run), a run costs about 95 VALU instructions instead of
+// 430 (SQ counters of the whole
+// kernel: 330 VALU instructions per wave and repetition of the 64^3 GRE, 512 staged). A single reused pulse's map is
+// held too (12 registers, some of them spilled: still faster than reading it from the L2 at every occurrence, 83.2 ->
+// 72.9 ms). 64^3 x 4 spins, 8 coils: 83.5 -> 70.6 ms a pass; 96^3, 16 coils: 219.3 -> 189.3 ms. Four waves per SIMD
+// (128 registers) and three (168, no spills) measured the same at a million spins; four keep 262,144 spins in one
+// round of workgroups. Only for dispatches without stepped RF: the RF loop is faster with five waves than this is with
+// four. Reading the next record ahead costs 32 scalar moves a record and measured 8 % slower.
+constexpr int kCols = 32;
+constexpr float kWeightLift = 1024.0f;  // the weights (<= 1) in float16's range, as kLift
+constexpr int kColTiles = kCols / 16;
+
+// LDS of these kernels: the samples' staging block, then two buffers of the waves' sums (kCols columns each; also the
+// weights' scratch while they are formed), then c of every wave (64 Re, 64 -Im, 64 Im).
+__host__ __device__ constexpr int lds_floats_cols(int nt) {
+    return kWaves * kStgFloats + 2 * kWaves * kCols * 16 * nt + kWaves * 192;
+}
+
+__device__ __forceinline__ void wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int NT>
+struct Spread {
+    float a[NT][16];                         // value jj of spins 16 g + u: Re S_0, Im S_0, Re S_1, ... scaled
+    h8 wh[kColTiles][2], wl[kColTiles][2];   // the weights of column 16 tile + jj, spins 16 g + u (u < 8, u >= 8)
+    float cp, sp;                            // cos, sin of the start's phase factor times the values' scale
+    int kind, cols;                          // the kind they belong to (-1: none yet), its window's columns
+
+    // sens_scale: Sens::scales' (lifted)
+    __device__ __forceinline__ void load(const float* __restrict__ sa, float sens_scale) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int u = 0; u < 16; ++u) a[t][u] = sa[t * 1024 + u * 64] * sens_scale;
+        kind = -1, cols = 0, cp = sp = 0.0f;
+    }
+};
+
+// x of lane ^ 1 (DPP quad permutation; folded into the instruction that uses it).
+__device__ __forceinline__ float dpp_xor1(float x) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(x), 0xB1, 0xf, 0xf, true));
+}
+
+// The staged samples' sums (flush_to's, from Spread's values: eight spins per lane are split at a time, anew per flush,
+// which costs 32 instructions per eight samples and holds no operand in registers).
+template <int NT>
+__device__ __forceinline__ void flush_spread(const float* stg, float* wred2, int& par, const Spread<NT>& W,
+                                             float out_scale, int nb, int row, int rows, float* __restrict__ partial) {
+    constexpr int vals = 16 * NT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, jj = lane & 15;
+    float* wred = wred2 + par * (kWaves * kCols * vals);
+    par ^= 1;
+    wave_fence();
+    float* mine = wred + wave * kCols * vals;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        h8 ah[2], bh[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            float x[8];
+            h8 al, bl;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                x[e] = W.a[t][8 * i + e];
+                asm volatile("" : "+v"(x[e]));  // keeps the compiler from hoisting the split out of the event loop
+            }
+            split8(x, ah[i], al);
+            *reinterpret_cast<f4*>(x) = *reinterpret_cast<const f4*>(stg + jj * kStgStride + 16 * g + 8 * i);
+            *reinterpret_cast<f4*>(x + 4) = *reinterpret_cast<const f4*>(stg + jj * kStgStride + 16 * g + 8 * i + 4);
+            split8(x, bh[i], bl);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, bh[i], acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bl, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bh[i], acc, 0, 0, 0);
+        store_pq(mine, vals, t, lane, acc);
+    }
+    __syncthreads();
+    const int keep = row + nb <= rows ? nb : (rows > row ? rows - row : 0);  // never past the rows
+    float* out = partial + ((size_t)blockIdx.x * rows + row) * vals;
+    for (int v = tid; v < keep * vals; v += kBlock) {
+        float s = wred[v];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) s += wred[w * kCols * vals + v];
+        out[v] = s * out_scale;
+    }
+}
+
+__device__ __forceinline__ void load16(float (&x)[16], const float* src) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        const f4 y = reinterpret_cast<const f4*>(src)[v];
+        x[4 * v] = y[0], x[4 * v + 1] = y[1], x[4 * v + 2] = y[2], x[4 * v + 3] = y[3];
+    }
+}
+
+// The weights and phase factor of a run's kind. Every lane of the workgroup calls it (the kind is uniform).
+template <int NT>
+__device__ __forceinline__ void make_weights(Spread<NT>& W, const hb_nufft& nu, const hb_segment& q, const Spin& p,
+                                             const Pos64& r64, float* wred, float x_scale, int lane, int wave) {
+    const int kind = q.pad[2];
+    const int ng = (int)nu.params[0], terms = (int)nu.params[2], shift = (int)nu.params[4];
+    const float h = nu.params[6 + HB_NUFFT_MAX_TERMS];       // 2 / width: z per grid cell
+    const float bl2 = nu.params[7 + HB_NUFFT_MAX_TERMS];     // beta log2(e)
+    const double cyc = free_cycles64(r64, p, q);
+    const double fr = cyc - floor(cyc);
+    const double xg = fr * ng;  // float64: at x ~ ng a float32 position is 1e-5 of a cycle off at the last sample
+    double ph = fr * shift;
+    ph -= rint(ph);
+    float sp, cp;
+    sincospi(-2.0f * (float)ph, &sp, &cp);
+    W.cp = cp * x_scale, W.sp = sp * x_scale;
+    const int* win = nu.win + ((size_t)kind * gridDim.x + blockIdx.x) * 2;
+    W.kind = kind;
+    W.cols = min(win[1] * terms, kCols);
+    // z = (cell - x) 2 / width: at the window's first cell from the float64 position (x ~ ng would leave a float32
+    // z 1e-6 off), then by float32 steps (|z| error under 3e-7 over a 32-cell window)
+    const float z0 = (float)(((double)win[0] - xg) * (double)h);
+    float* scr = wred + wave * 1024;  // 16 columns x 64 spins
+    const int g = lane >> 4, jj = lane & 15;
+    __syncthreads();  // the sums' buffers are free
+    int m = 0;
+    float lcf = 0.0f;
+#pragma unroll
+    for (int t = 0; t < kColTiles; ++t) {
+#pragma unroll 1
+        for (int r = 0; r < 16; ++r) {
+            const float z = fmaf(lcf, h, z0);
+            const float u = fmaf(-z, z, 1.0f);
+            // the ES kernel e^{beta (sqrt(1 - z^2) - 1)} = 2^{beta log2(e) (sqrt(u) - 1)}, zero outside |z| < 1, on the
+            // hardware square root and exp2 (about 1 ulp each; the argument's rounding, |arg| < 20, leaves the
+            // kernel value within 2e-6 relative)
+            const float kv =
+                u > 0.0f ? __builtin_amdgcn_exp2f(fmaf(bl2, __builtin_amdgcn_sqrtf(u), -bl2)) : 0.0f;
+            const float em = __builtin_amdgcn_exp2f(-(nu.params[6 + m] * 1.4426950408889634f) * p.r2);
+            scr[r * 64 + lane] = 16 * t + r < W.cols ? kv * em * kWeightLift : 0.0f;
+            if (++m == terms) m = 0, lcf += 1.0f;
+        }
+        wave_fence();
+        float x[16];
+        load16(x, scr + jj * 64 + 16 * g);
+        split8(x, W.wh[t][0], W.wl[t][0]);
+        split8(x + 8, W.wh[t][1], W.wl[t][1]);
+        wave_fence();
+    }
+    __syncthreads();
+}
+
+// One NUFFT readout run (record q: pad[1] its slot, pad[2] its kind, pad[3] its length): its window's columns into its
+// slot of the grid partials, then the exact jump over it.
+template <int NT>
+__device__ __forceinline__ void spread_run(const Spread<NT>& W, const hb_nufft& nu, const hb_segment& q, const Spin& p,
+                                           const Pos64& r64, float& e1_run, State& m, float* wred, float* cbuf, int& par,
+                                           float out_scale, int tid) {
+    constexpr int vals = 16 * NT;
+    const int lane = tid & 63, wave = tid >> 6, g = lane >> 4, jj = lane & 15;
+    const float ci_ = m.mx * W.sp + m.my * W.cp;
+    cbuf[lane] = m.mx * W.cp - m.my * W.sp;
+    cbuf[64 + lane] = -ci_;
+    cbuf[128 + lane] = ci_;
+    wave_fence();
+    float* buf = wred + par * (kWaves * kCols * vals);
+    par ^= 1;
+    float* mine = buf + wave * (kCols * vals);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        f4 acc[kColTiles];
+        h8 vh[2];
+#pragma unroll
+        for (int k = 0; k < kColTiles; ++k) acc[k] = (f4){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {  // eight spins per lane at a time, the small products first
+            h8 vl;
+            float x[8];
+#pragma unroll
+            for (int v = 0; v < 2; ++v) {
+                const f4 cr = *reinterpret_cast<const f4*>(cbuf + 16 * g + 8 * i + 4 * v);
+                // values Re S c = Sr cr - Si ci (even jj), Im S c = Si cr + Sr ci (odd): the partner lane's S
+                const f4 ci = *reinterpret_cast<const f4*>(cbuf + 64 + 64 * (jj & 1) + 16 * g + 8 * i + 4 * v);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int u = 8 * i + 4 * v + e;
+                    x[4 * v + e] = fmaf(dpp_xor1(W.a[t][u]), ci[e], W.a[t][u] * cr[e]);
+                }
+            }
+            split8(x, vh[i], vl);
+#pragma unroll
+            for (int k = 0; k < kColTiles; ++k) {
+                if (16 * k < W.cols) {  // uniform
+                    acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl, W.wh[k][i], acc[k], 0, 0, 0);
+                    acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[i], W.wl[k][i], acc[k], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kColTiles; ++k) {
+            if (16 * k < W.cols) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+                    acc[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[i], W.wh[k][i], acc[k], 0, 0, 0);
+                // values 4 g .. 4 g + 3 of column 16 k + jj
+                *reinterpret_cast<f4*>(mine + (16 * k + jj) * vals + 16 * t + 4 * g) = acc[k];
+            }
+        }
+    }
+    __syncthreads();
+    if (4 * tid < W.cols * vals) {
+        f4 s = reinterpret_cast<const f4*>(buf)[tid];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) s += reinterpret_cast<const f4*>(buf + w * (kCols * vals))[tid];
+        float* out = nu.part + ((size_t)q.pad[1] * gridDim.x + blockIdx.x) * nu.cols * vals;
+        reinterpret_cast<f4*>(out)[tid] = s * (out_scale * (1.0f / kWeightLift));
+    }
+    if (!(q.flags & HB_SAME_RUN)) e1_run = expm1x(-((float)q.pad[3] * q.dt) * p.r1);
+    double cyc = 0.0;
+    if (!(q.flags & (HB_XY_DEAD | HB_PULSE_SPOIL))) cyc = free_cycles64(r64, p, q);
+    run_jump(q, p, cyc, e1_run, m);
+}
+
+// NT: coil tiles (0: any, the sensitivities read from memory per flush); NUT: NUFFT runs: 0 none, 1 by spread_run (NT 1 or
+// 2, windows of at most kCols columns), 4 and 8 by nufft_run with up to NUT decay terms (their weights in registers); RF: RF segments are stepped (false when every pulse of the
 // dispatch is applied as a map: the RF step is then left out, and its registers).
 // The read-only inputs and the NUFFT partials come in again as noalias parameters (the same pointers as in cs_in and
 // nu_in): no store of the kernel can change the records, so they load through the scalar cache instead of one vector
 // load per wave and a readfirstlane per value.
 template <int NT, int NUT, bool RF>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 ? 3 : 5))) void forward_kernel(
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 ? 3 : NUT == 1 ? 4 : 5))) void forward_kernel(
     hb_case cs_in, int s0, int s1, float* __restrict__ partial, int rows, hb_nufft nu_in,
     const hb_segment* __restrict__ segs, const float* __restrict__ spins, const float* __restrict__ pos_lo,
     const float* __restrict__ sens_a, const float* __restrict__ maps, const float* __restrict__ nu_params,
@@ -124,21 +357,61 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
     const Pos64 r64 = pos64(p);
     const float b1sq = p.b1 * p.b1;
     State m = load_state(cs.state, np, j);
+    // The dispatch's records into the L2s, 256 a workgroup: each XCD's first workgroups (workgroups go round robin over
+    // the 8 XCDs) touch them all, so that no wave waits for memory at a record's first use. A dispatch of 17,000 records
+    // takes 2 MB of an XCD's 4 MB; 32^3 x 4 spins, every RF substep: 78.4 -> 61.3 ms; 96^3, maps and NUFFT runs, 16 coils:
+    // 196.5 -> 189.1 ms.
+    {
+        const int first = blockIdx.x >> 3, stride = max(1, min((int)gridDim.x >> 3, 64));
+        if (first < stride) {
+            float touched = 0.0f;
+            for (int r = s0 + first * kBlock + tid; r < s1; r += stride * kBlock) touched += segs[r].dt;
+            asm volatile("" ::"v"(touched));
+        }
+    }
     Sens<NT> S;
     S.sa = cs.sens_a + (size_t)(blockIdx.x * kWaves + wave) * nt * 1024 + lane;
     S.st = 1024, S.su = 64, S.n_rows = 16 * nt;
-    S.load(cs.x_scale, cs.sens_scale, lane);
+    int nb = 0, row = 0, par = 0;
+    constexpr bool MAT = NUT == 1;
+    constexpr int NS = NT > 0 ? NT : 1;
+    Spread<NS> W;
+    float* cbuf = wred + 2 * kWaves * kCols * 16 * NS + wave * 192;
+    if constexpr (MAT) {
+        float scale = cs.sens_scale;
+        S.scales(cs.x_scale, scale);
+        W.load(S.sa, scale);
+    } else {
+        S.load(cs.x_scale, cs.sens_scale, lane);
+    }
+    // the staged samples (all of them, or at the end the nb left) into the partial rows
+    auto flush_samples = [&](int count, int at) {
+        if constexpr (MAT) {
+            flush_spread<NS>(stg, wred, par, W, S.out_scale, count, at, rows, partial);
+        } else {
+            flush<NT>(stg, wred, par, S, nt, count, at, rows, partial);
+        }
+    };
     Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     float e1_run = 0.0f;  // expm1(-L dt R1) of the last readout run (per sample or NUFFT)
     // the NUFFT decay terms e^{-R2 tau_m}: the spin's, the same for every run
-    float em[NUT > 0 ? NUT : 1];
-    if constexpr (NUT > 0) {
+    float em[NUT > 1 ? NUT : 1];
+    if constexpr (NUT > 1) {
         const int terms = (int)nu.params[2];
 #pragma unroll
         for (int t = 0; t < NUT; ++t)
             em[t] = t < terms ? __builtin_amdgcn_exp2f(-(nu.params[6 + t] * 1.4426950408889634f) * p.r2) : 0.0f;
     }
-    int nb = 0, row = 0, par = 0;
+    // a single reused pulse's map in registers (more pulses: read per occurrence)
+    constexpr bool MAP = MAT;
+    const bool one_map = MAP && cs.n_pulses == 1;  // uniform
+    float U[MAP ? 12 : 1];
+    if constexpr (MAP) {
+        if (one_map) {
+#pragma unroll
+            for (int i = 0; i < 12; ++i) U[i] = cs.maps[(size_t)i * np + j];
+        }
+    }
     // a dispatch that starts inside a reused pulse's occurrence or a NUFFT run (checkpoint intervals do not avoid
     // them): the record was applied at its first segment, in the dispatch before
     int s_start = s0;
@@ -147,84 +420,101 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
         const hb_segment& hq = cs.segs[head];
         s_start = head + ((hq.flags & HB_PULSE) ? hq.pad[2] : hq.pad[3]);
     }
-    for (int s = s_start; s < s1; ++s) {
-        const hb_segment q = cs.segs[s];
-        const int f = q.flags;
-        if constexpr (NUT > 0) {
-            if (f & HB_NUFFT) {  // a readout run as a type-1 NUFFT: spread onto the grid window, jump the run
-                nufft_run<NT, NUT>(cs, nu, q, p, r64, em, e1_run, m, stg, wred, par, S, nt, lane, nb, row, rows,
-                                   partial);
-                s += q.pad[3] - 1;
-                continue;
-            }
+    // (With spread_run the loop runs from one change of the runs' kind to the next: the weights, formed between, do not
+    // change inside it and stay in their registers.)
+    for (int s = s_start; s < s1;) {
+        if constexpr (MAT) {
+            const hb_segment q = cs.segs[s];
+            if ((q.flags & HB_NUFFT) && q.pad[2] != W.kind)
+                make_weights<NS>(W, nu, q, p, r64, wred, S.x_scale, lane, wave);
         }
-        if (RF && (f & HB_TRAIN)) {  // RF substeps of a shaped pulse, in a loop of their own (only RF state live)
-            const int L = q.pad[3];
-            RfRec cur = load_rf(&cs.segs[s]);
-            for (int i = 1; i <= L; ++i) {
-                const RfRec nxt = load_rf(&cs.segs[s + (i < L ? i : 0)]);  // in flight while this one is stepped
-                rf_step(cur, cur.flags, p, b1sq, m, k);
-                cur = nxt;
-            }
-            s += L - 1;
-            continue;
-        }
-        if (f & HB_RUN) {  // L identical free ADC segments: Mxy stepped and sampled per segment, Mz relaxed once
-            const int L = q.pad[3];
-            if (!(f & HB_SAME_FREE)) {
-                sincospi(-2.0f * free_cycles(r64, p, q), &k.s, &k.c);
-                if (!(f & HB_SAME_FREE_DT)) {
-                    k.e1 = expm1x(-q.dt * p.r1);
-                    k.e2 = expm1x(-q.dt * p.r2);
+        for (; s < s1; ++s) {
+            const hb_segment q = cs.segs[s];
+            const int f = q.flags;
+            if constexpr (NUT > 0) {
+                if (f & HB_NUFFT) {  // a readout run as a type-1 NUFFT: spread onto the grid window, jump the run
+                    if constexpr (MAT) {
+                        if (q.pad[2] != W.kind) break;
+                        spread_run<NS>(W, nu, q, p, r64, e1_run, m, wred, cbuf, par, S.out_scale, tid);
+                    } else {
+                        nufft_run<NT, NUT>(cs, nu, q, p, r64, em, e1_run, m, stg, wred, par, S, nt, lane, nb, row, rows,
+                                           partial);
+                    }
+                    s += q.pad[3] - 1;
+                    continue;
                 }
             }
-            if (!(f & HB_SAME_RUN)) e1_run = expm1x(-(float)L * q.dt * p.r1);
-            for (int i = 0; i < L; ++i) {
-                const float nx = k.c * m.mx - k.s * m.my, ny = k.s * m.mx + k.c * m.my;
-                m.mx = nx + nx * k.e2;
-                m.my = ny + ny * k.e2;
+            if (RF && (f & HB_TRAIN)) {  // RF substeps of a shaped pulse, in a loop of their own (only RF state live)
+                const int L = q.pad[3];
+                RfRec cur = load_rf(&cs.segs[s]);
+                for (int i = 1; i <= L; ++i) {
+                    const RfRec nxt = load_rf(&cs.segs[s + (i < L ? i : 0)]);  // in flight while this one is stepped
+                    rf_step(cur, cur.flags, p, b1sq, m, k);
+                    cur = nxt;
+                }
+                s += L - 1;
+                continue;
+            }
+            if (f & HB_RUN) {  // L identical free ADC segments: Mxy stepped and sampled per segment, Mz relaxed once
+                const int L = q.pad[3];
+                if (!(f & HB_SAME_FREE)) {
+                    sincospi(-2.0f * free_cycles(r64, p, q), &k.s, &k.c);
+                    if (!(f & HB_SAME_FREE_DT)) {
+                        k.e1 = expm1x(-q.dt * p.r1);
+                        k.e2 = expm1x(-q.dt * p.r2);
+                    }
+                }
+                if (!(f & HB_SAME_RUN)) e1_run = expm1x(-(float)L * q.dt * p.r1);
+                for (int i = 0; i < L; ++i) {
+                    const float nx = k.c * m.mx - k.s * m.my, ny = k.s * m.mx + k.c * m.my;
+                    m.mx = nx + nx * k.e2;
+                    m.my = ny + ny * k.e2;
+                    stg[nb * kStgStride + lane] = m.mx * S.x_scale;
+                    stg[(8 + nb) * kStgStride + lane] = m.my * S.x_scale;
+                    if (++nb == 8) {
+                        flush_samples(8, row);
+                        row += 8;
+                        nb = 0;
+                    }
+                }
+                two_sum(m.mz, m.lz, (m.mz - p.pd) * e1_run);
+                s += L - 1;
+                continue;
+            }
+            if (f & HB_PULSE) {  // a reused pulse: m += Rz(psi) (D Rz(-psi) m + v), then skip its segments
+                // cos, sin of the occurrence's RF phase (host float64)
+                if (MAP && one_map)
+                    apply_map(U, 1, q.w_rf_x, q.w_rf_y, m);
+                else
+                    apply_map(cs.maps + (size_t)q.pad[1] * 12 * np + j, np, q.w_rf_x, q.w_rf_y, m);
+                if (f & HB_PULSE_SPOIL) m.mx = m.my = 0.0f;
+                s += q.pad[2] - 1;
+                continue;
+            }
+            if (f & HB_SPOILED_FREE) {  // only Mz survives the spoil: relax it, zero Mxy
+                two_sum(m.mz, m.lz, (m.mz - p.pd) * expm1x(-q.dt * p.r1));
+                m.mx = m.my = 0.0f;
+                if (f & HB_MERGED) s += q.pad[3] - 1;
+                continue;
+            }
+            if constexpr (RF)
+                step(q, f, p, r64, b1sq, m, k);
+            else
+                free_step(q, f, p, r64, m, k);
+            if (f & HB_MERGED) s += q.pad[3] - 1;
+            if (f & HB_ADC) {
                 stg[nb * kStgStride + lane] = m.mx * S.x_scale;
                 stg[(8 + nb) * kStgStride + lane] = m.my * S.x_scale;
                 if (++nb == 8) {
-                    flush<NT>(stg, wred, par, S, nt, 8, row, rows, partial);
+                    flush_samples(8, row);
                     row += 8;
                     nb = 0;
                 }
             }
-            two_sum(m.mz, m.lz, (m.mz - p.pd) * e1_run);
-            s += L - 1;
-            continue;
+            if (f & HB_SPOIL) m.mx = m.my = 0.0f;
         }
-        if (f & HB_PULSE) {  // a reused pulse: m += Rz(psi) (D Rz(-psi) m + v), then skip its segments
-            // cos, sin of the occurrence's RF phase (host float64)
-            apply_map(cs.maps + (size_t)q.pad[1] * 12 * np + j, np, q.w_rf_x, q.w_rf_y, m);
-            if (f & HB_PULSE_SPOIL) m.mx = m.my = 0.0f;
-            s += q.pad[2] - 1;
-            continue;
-        }
-        if (f & HB_SPOILED_FREE) {  // only Mz survives the spoil: relax it, zero Mxy
-            two_sum(m.mz, m.lz, (m.mz - p.pd) * expm1x(-q.dt * p.r1));
-            m.mx = m.my = 0.0f;
-            if (f & HB_MERGED) s += q.pad[3] - 1;
-            continue;
-        }
-        if constexpr (RF)
-            step(q, f, p, r64, b1sq, m, k);
-        else
-            free_step(q, f, p, r64, m, k);
-        if (f & HB_MERGED) s += q.pad[3] - 1;
-        if (f & HB_ADC) {
-            stg[nb * kStgStride + lane] = m.mx * S.x_scale;
-            stg[(8 + nb) * kStgStride + lane] = m.my * S.x_scale;
-            if (++nb == 8) {
-                flush<NT>(stg, wred, par, S, nt, 8, row, rows, partial);
-                row += 8;
-                nb = 0;
-            }
-        }
-        if (f & HB_SPOIL) m.mx = m.my = 0.0f;
     }
-    if (nb > 0) flush<NT>(stg, wred, par, S, nt, nb, row, rows, partial);
+    if (nb > 0) flush_samples(nb, row);
     store_state(cs.state, np, j, m);
 }
 
@@ -273,9 +563,10 @@ namespace hb {
 template <int NUT, bool RF>
 static void launch_nt(const hb_case& cs, int s0, int s1, float* partial, int rows, const hb_nufft& nu, dim3 grid,
                       dim3 block, size_t lds, hipStream_t st) {
-    auto kernel = cs.n_tiles == 1   ? forward_kernel<1, NUT, RF>
-                  : cs.n_tiles == 2 ? forward_kernel<2, NUT, RF>
-                                    : forward_kernel<0, NUT, RF>;
+    auto kernel = cs.n_tiles == 1 ? forward_kernel<1, NUT, RF> : forward_kernel<2, NUT, RF>;
+    if constexpr (NUT != 1) {
+        if (cs.n_tiles > 2) kernel = forward_kernel<0, NUT, RF>;
+    }
     hipLaunchKernelGGL(kernel, grid, block, lds, st, cs, s0, s1, partial, rows, nu, cs.segs, cs.spins, cs.pos_lo,
                        cs.sens_a, cs.maps, nu.params, nu.win, nu.part);
 }
@@ -283,10 +574,10 @@ static void launch_nt(const hb_case& cs, int s0, int s1, float* partial, int row
 template <int NUT>
 static void launch_forward(const hb_case& cs, int s0, int s1, float* partial, int rows, const hb_nufft& nu,
                            dim3 grid, dim3 block, size_t lds, hipStream_t st) {
-    if (cs.rf_free)
+    if (NUT == 1 || cs.rf_free)
         launch_nt<NUT, false>(cs, s0, s1, partial, rows, nu, grid, block, lds, st);
     else
-        launch_nt<NUT, true>(cs, s0, s1, partial, rows, nu, grid, block, lds, st);
+        launch_nt<NUT == 1 ? 0 : NUT, true>(cs, s0, s1, partial, rows, nu, grid, block, lds, st);
 }
 }  // namespace hb
 
@@ -308,6 +599,9 @@ extern "C" int hb_forward(const hb_case* cs, int32_t s0, int32_t s1, float* part
     const hb_nufft arg = nu ? *nu : none;
     if (!nu)
         launch_forward<0>(*cs, s0, s1, partial, rows, arg, grid, block, lds, st);
+    else if (nu->cols <= kCols && cs->n_tiles <= 2 && cs->rf_free)  // see spread_run
+        launch_forward<1>(*cs, s0, s1, partial, rows, arg, grid, block, sizeof(float) * lds_floats_cols(cs->n_tiles),
+                          st);
     else if (nu->terms <= 4)
         launch_forward<4>(*cs, s0, s1, partial, rows, arg, grid, block, lds, st);
     else
