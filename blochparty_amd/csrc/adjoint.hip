@@ -257,104 +257,138 @@ __device__ __forceinline__ void nufft_reverse(const hb_segment& q, const hb_adjo
     acc.v[A_DB0] += gb;
 }
 
+// The interval's records and the samples' h rows into the L2s (as forward_kernel's: 256 records a workgroup, each XCD's
+// first workgroups touch them all), so that no wave waits for memory at a record's or a row's first use: 64 segments of 8,169
+// spins take 72 us instead of 93.
+template <int NC>
+__device__ __forceinline__ void touch_interval(const hb_segment* __restrict__ segs, const float* __restrict__ h, int s0,
+                                               int s1) {
+    const int first = blockIdx.x >> 3, stride = max(1, min((int)gridDim.x >> 3, 64));
+    if (first >= stride) return;
+    float touched = 0.0f;
+    for (int r = s0 + first * kBlockA + threadIdx.x; r < s1; r += stride * kBlockA) {
+        const int f = segs[r].flags, row = segs[r].pad[0];
+        touched += (float)f;
+        if (NC > 0 && (f & HB_ADC)) {
+#pragma unroll
+            for (int c = 0; c < 2 * NC; c += 32) touched += h[(size_t)row * 2 * NC + c];
+        }
+    }
+    asm volatile("" ::"v"(touched));
+}
+
+// The interval replayed from its checkpoint: r8[b] = the state before segment s0 + 8 b (low parts folded).
+template <bool NU>
+__device__ __forceinline__ void replay_interval(const hb_case& cs, const hb_adjoint& ad, const Spin& p, float b1sq, int j,
+                                                int s0, int s1) {
+    const int np = cs.n_pad;
+    State m = load_state(ad.ckpt, np, j);
+    Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    bool free_ok = false, rf_ok = false;
+    int s_start = s0;
+    if (cs.segs[s0].flags & HB_PULSE_BODY) {  // inside an occurrence or a run begun in an earlier interval
+        const hb_segment& hq = cs.segs[cs.segs[s0].pad[3]];
+        const int e = min(cs.segs[s0].pad[3] + ((hq.flags & HB_PULSE) ? hq.pad[2] : hq.pad[3]), s1);
+        r8_after_span(ad.r8, np, j, s0, s1, s0 - 1, e, m);
+        s_start = e;
+    }
+    for (int s = s_start; s < s1; ++s) {
+        if (((s - s0) & 7) == 0) {
+            float* r = ad.r8 + (size_t)((s - s0) >> 3) * 3 * np;
+            r[j] = m.mx, r[np + j] = m.my, r[2 * np + j] = m.mz + m.lz;
+        }
+        const hb_segment q = cs.segs[s];
+        if (q.flags & HB_PULSE) {  // a reused pulse: its map, then the state stands over the occurrence
+            apply_map(cs.maps + (size_t)q.pad[1] * 12 * np + j, np, q.w_rf_x, q.w_rf_y, m);
+            if (q.flags & HB_PULSE_SPOIL) m.mx = m.my = 0.0f;
+            const int e = min(s + q.pad[2], s1);
+            r8_after_span(ad.r8, np, j, s0, s1, s, e, m);
+            s = e - 1;
+            continue;
+        }
+        if (NU && (q.flags & HB_NUFFT)) {  // a readout run: its jump (its samples add nothing to the state)
+            run_jump(q, p, free_cycles64(pos64(p), p, q), expm1x(-((float)q.pad[3] * q.dt) * p.r1), m);
+            const int e = min(s + q.pad[3], s1);
+            r8_after_span(ad.r8, np, j, s0, s1, s, e, m);
+            s = e - 1;
+            continue;
+        }
+        if (q.flags & HB_TRAIN) {  // an RF train: its own loop, the next record in flight (forward_kernel's)
+            const int L = min(q.pad[3], s1 - s);
+            RfRec cur = load_rf(&cs.segs[s]);
+            for (int i = 1; i <= L; ++i) {
+                const RfRec nxt = load_rf(&cs.segs[s + (i < L ? i : 0)]);
+                if (i > 1 && ((s + i - 1 - s0) & 7) == 0) {
+                    float* r = ad.r8 + (size_t)((s + i - 1 - s0) >> 3) * 3 * np;
+                    r[j] = m.mx, r[np + j] = m.my, r[2 * np + j] = m.mz + m.lz;
+                }
+                rf_step(cur, live_flags(cur.flags, true, rf_ok, 0, HB_SAME_RF_DT), p, b1sq, m, k);
+                rf_ok = true;
+                cur = nxt;
+            }
+            s += L - 1;
+            continue;
+        }
+        const int f = live_flags(q.flags, free_ok, rf_ok, HB_SAME_FREE, HB_SAME_RF_DT);
+        step(q, f, p, b1sq, m, k);
+        if (f & HB_RF) rf_ok = true; else free_ok = true;
+        if (f & HB_SPOIL) m.mx = m.my = 0.0f;
+    }
+}
+
 // NU: the table has NUFFT runs (their reverse raises the register pressure of the unrolled block loop, so the other
 // tables take the variant without it).
 // The read-only inputs come in again as noalias parameters (the same pointers as in cs_in and ad_in): no store of the
 // kernel can change what they point to, so the loads at wave-uniform addresses (the records, h rows, NUFFT tables)
 // go through the scalar cache instead of one vector load per wave and a readfirstlane per value.
-template <int NC, bool SEG, bool NU>
+// CHUNK: the reverse of chunk blockIdx.y ([s0 + chunk y, ...), chunk a power of two from 8 to 64) of an interval without
+// maps and runs that sweep_kernel has replayed: from the adjoint at the chunk's end (lam_c), its gradients, float32 sums
+// over the chunk as between two flushes below, into part[y] (8 + 2 NC, n_pad) for chunk_sums_kernel.
+template <int NC, bool SEG, bool NU, bool CHUNK = false>
 __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8 ? 2 : 1))) void adjoint_kernel(
     hb_case cs_in, hb_adjoint ad_in, int s0, int s1, const hb_segment* __restrict__ segs,
     const float* __restrict__ spins, const float* __restrict__ pos_lo, const float* __restrict__ maps,
     const float* __restrict__ ckpt, const float* __restrict__ h, const float* __restrict__ sens,
     const float* __restrict__ maps_d, const float* __restrict__ nu_params, const int32_t* __restrict__ nu_win,
-    const float* __restrict__ nu_grid) {
+    const float* __restrict__ nu_grid, int chunk, const float* __restrict__ lam_c, float* __restrict__ part) {
     hb_case cs = cs_in;
     cs.segs = segs, cs.spins = spins, cs.pos_lo = pos_lo, cs.maps = maps;
     hb_adjoint ad = ad_in;
     ad.ckpt = ckpt, ad.h = h, ad.sens = sens, ad.maps_d = maps_d;
     ad.nu_params = nu_params, ad.nu_win = nu_win, ad.nu_grid = nu_grid;
     __shared__ float segbuf[2][kWavesA][8][8];  // alternate buffers: one barrier per workgroup sum
-    __shared__ double accs[(8 + 2 * NC) * kBlockA];  // float64 accumulators: slot a of lane tid at a * kBlockA + tid
-    __shared__ double seeds_l[12 * kBlockA];          // a single reused pulse's seeds, same layout
+    // float64 accumulators: slot a of lane tid at a * kBlockA + tid
+    __shared__ double accs[CHUNK ? 1 : (8 + 2 * NC) * kBlockA];
+    __shared__ double seeds_l[CHUNK ? 1 : 12 * kBlockA];  // a single reused pulse's seeds, same layout
     int sbuf = 0;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int j = blockIdx.x * kBlockA + tid;
     const int np = cs.n_pad;
     const bool coil_grads = NC > 0 && ad.coil_grads;
-    const bool seeds_in_lds = cs.n_pulses == 1 && ad.seeds;  // uniform
-    if (seeds_in_lds) {
+    const bool seeds_in_lds = !CHUNK && cs.n_pulses == 1 && ad.seeds;  // uniform
+    if constexpr (!CHUNK) {
+        touch_interval<NC>(segs, h, s0, s1);
+        if (seeds_in_lds) {
 #pragma unroll
-        for (int a = 0; a < 12; ++a) seeds_l[a * kBlockA + tid] = ad.seeds[(size_t)a * np + j];
-    }
+            for (int a = 0; a < 12; ++a) seeds_l[a * kBlockA + tid] = ad.seeds[(size_t)a * np + j];
+        }
 #pragma unroll
-    for (int a = 0; a < 8; ++a) accs[a * kBlockA + tid] = ad.gs[(size_t)a * np + j];
-    if (coil_grads) {
+        for (int a = 0; a < 8; ++a) accs[a * kBlockA + tid] = ad.gs[(size_t)a * np + j];
+        if (coil_grads) {
 #pragma unroll
-        for (int c = 0; c < 2 * NC; ++c) accs[(8 + c) * kBlockA + tid] = ad.gc[(size_t)c * np + j];
+            for (int c = 0; c < 2 * NC; ++c) accs[(8 + c) * kBlockA + tid] = ad.gc[(size_t)c * np + j];
+        }
     }
     const Spin p = load_spin(cs.spins, cs.pos_lo, np, j);
     const float b1sq = p.b1 * p.b1;
     const bool rf_only = SEG && ad.seg_grads == 2;
 
-    // 1. replay the interval, r8[b] = state before segment s0 + 8 b (low parts folded)
-    {
-        State m = load_state(ad.ckpt, np, j);
-        Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-        bool free_ok = false, rf_ok = false;
-        int s_start = s0;
-        if (cs.segs[s0].flags & HB_PULSE_BODY) {  // inside an occurrence or a run begun in an earlier interval
-            const hb_segment& hq = cs.segs[cs.segs[s0].pad[3]];
-            const int e = min(cs.segs[s0].pad[3] + ((hq.flags & HB_PULSE) ? hq.pad[2] : hq.pad[3]), s1);
-            r8_after_span(ad.r8, np, j, s0, s1, s0 - 1, e, m);
-            s_start = e;
-        }
-        for (int s = s_start; s < s1; ++s) {
-            if (((s - s0) & 7) == 0) {
-                float* r = ad.r8 + (size_t)((s - s0) >> 3) * 3 * np;
-                r[j] = m.mx, r[np + j] = m.my, r[2 * np + j] = m.mz + m.lz;
-            }
-            const hb_segment q = cs.segs[s];
-            if (q.flags & HB_PULSE) {  // a reused pulse: its map, then the state stands over the occurrence
-                apply_map(cs.maps + (size_t)q.pad[1] * 12 * np + j, np, q.w_rf_x, q.w_rf_y, m);
-                if (q.flags & HB_PULSE_SPOIL) m.mx = m.my = 0.0f;
-                const int e = min(s + q.pad[2], s1);
-                r8_after_span(ad.r8, np, j, s0, s1, s, e, m);
-                s = e - 1;
-                continue;
-            }
-            if (NU && (q.flags & HB_NUFFT)) {  // a readout run: its jump (its samples add nothing to the state)
-                run_jump(q, p, free_cycles64(pos64(p), p, q), expm1x(-((float)q.pad[3] * q.dt) * p.r1), m);
-                const int e = min(s + q.pad[3], s1);
-                r8_after_span(ad.r8, np, j, s0, s1, s, e, m);
-                s = e - 1;
-                continue;
-            }
-            if (q.flags & HB_TRAIN) {  // an RF train: its own loop, the next record in flight (forward_kernel's)
-                const int L = min(q.pad[3], s1 - s);
-                RfRec cur = load_rf(&cs.segs[s]);
-                for (int i = 1; i <= L; ++i) {
-                    const RfRec nxt = load_rf(&cs.segs[s + (i < L ? i : 0)]);
-                    if (i > 1 && ((s + i - 1 - s0) & 7) == 0) {
-                        float* r = ad.r8 + (size_t)((s + i - 1 - s0) >> 3) * 3 * np;
-                        r[j] = m.mx, r[np + j] = m.my, r[2 * np + j] = m.mz + m.lz;
-                    }
-                    rf_step(cur, live_flags(cur.flags, true, rf_ok, 0, HB_SAME_RF_DT), p, b1sq, m, k);
-                    rf_ok = true;
-                    cur = nxt;
-                }
-                s += L - 1;
-                continue;
-            }
-            const int f = live_flags(q.flags, free_ok, rf_ok, HB_SAME_FREE, HB_SAME_RF_DT);
-            step(q, f, p, b1sq, m, k);
-            if (f & HB_RF) rf_ok = true; else free_ok = true;
-            if (f & HB_SPOIL) m.mx = m.my = 0.0f;
-        }
-    }
+    // 1. replay the interval
+    if constexpr (!CHUNK) replay_interval<NU>(cs, ad, p, b1sq, j, s0, s1);
 
     // 2. reverse sweep
-    float lx = ad.lam[j], ly = ad.lam[np + j], lz = ad.lam[2 * np + j];
+    const float* l0 = CHUNK ? lam_c + (size_t)blockIdx.y * 3 * np : ad.lam;
+    float lx = l0[j], ly = l0[np + j], lz = l0[2 * np + j];
     float sr[NC > 0 ? NC : 1], si[NC > 0 ? NC : 1], gr[NC > 0 ? NC : 1], gi[NC > 0 ? NC : 1];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
@@ -370,15 +404,19 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
     // a record that adds to the accumulators was reversed since the last flush (else they hold exact zeros and the
     // flush is skipped: the float64 sums are the same bit for bit, and spans of pulses and runs cost no HBM traffic)
     bool dirty = false;
-    const int n8 = (s1 - s0 + 7) >> 3;
-    for (int b = n8 - 1; b >= 0; --b) {
+    int n8 = (s1 - s0 + 7) >> 3, b_end = 0;
+    if constexpr (CHUNK) {
+        b_end = (int)blockIdx.y * (chunk >> 3);
+        n8 = min(n8, b_end + (chunk >> 3));
+    }
+    for (int b = n8 - 1; b >= b_end; --b) {
         const int sb = s0 + 8 * b;
         const int nseg = min(8, s1 - sb);
         // a block inside one reused pulse's occurrence is the identity: only its (zero) segment gradients
         const hb_segment& qf = cs.segs[sb];
         const hb_segment& ql = cs.segs[sb + nseg - 1];
         bool flush_point = (sb & 63) == 0;
-        if ((qf.flags & ql.flags & HB_PULSE_BODY) && qf.pad[3] == ql.pad[3]) {
+        if (!CHUNK && (qf.flags & ql.flags & HB_PULSE_BODY) && qf.pad[3] == ql.pad[3]) {
             // so is every block from the first one after the record's head down to this one: all skipped at once
             const int head = qf.pad[3];
             const int b_min = head < s0 ? 0 : (head + 1 - s0 + 7) >> 3;
@@ -401,11 +439,11 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
                 if (i < nseg) {
                     before[i] = {m.mx, m.my, m.mz + m.lz};
                     const hb_segment q = cs.segs[sb + i];
-                    if (q.flags & HB_PULSE_BODY) {
+                    if (!CHUNK && (q.flags & HB_PULSE_BODY)) {
                         after[i] = {m.mx, m.my};
                         continue;
                     }
-                    if (q.flags & HB_PULSE) {
+                    if (!CHUNK && (q.flags & HB_PULSE)) {
                         apply_map(cs.maps + (size_t)q.pad[1] * 12 * np + j, np, q.w_rf_x, q.w_rf_y, m);
                         after[i] = {m.mx, m.my};
                         if (q.flags & HB_PULSE_SPOIL) m.mx = m.my = 0.0f;
@@ -432,7 +470,7 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
             if (i < nseg) {
                 const int s = sb + i;
                 const hb_segment q = cs.segs[s];
-                if (q.flags & HB_PULSE_BODY) continue;  // the identity, no gradients
+                if (!CHUNK && (q.flags & HB_PULSE_BODY)) continue;  // the identity, no gradients
                 if constexpr (NU) {
                     if (q.flags & HB_NUFFT) {
                         nufft_reverse<NC>(q, ad, p, before[i], lx, ly, lz, acc, sr, si, gr, gi);
@@ -440,7 +478,7 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
                         continue;
                     }
                 }
-                if (q.flags & HB_PULSE) {
+                if (!CHUNK && (q.flags & HB_PULSE)) {
                     if (q.flags & HB_PULSE_SPOIL) lx = ly = 0.0f;
                     pulse_reverse<SEG>(q, cs, ad, j, before[i], after[i], lx, ly, lz, sg, seeds_l, seeds_in_lds);
                     if (SEG) seg_add(segd, sg, i, lane);
@@ -495,7 +533,7 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
             sbuf ^= 1;
         }
         }
-        if (flush_point && dirty) {  // every 64 segments: into the float64 accumulators
+        if (!CHUNK && flush_point && dirty) {  // every 64 segments: into the float64 accumulators
             dirty = false;
 #pragma unroll
             for (int a = 0; a < 8; ++a) {
@@ -512,6 +550,16 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
             }
         }
     }
+    if constexpr (CHUNK) {
+        float* o = part + (size_t)blockIdx.y * (8 + 2 * NC) * np + j;
+#pragma unroll
+        for (int a = 0; a < 8; ++a) o[(size_t)a * np] = acc.v[a];
+        if (coil_grads) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) o[(size_t)(8 + 2 * c) * np] = gr[c], o[(size_t)(9 + 2 * c) * np] = gi[c];
+        }
+        return;
+    }
     // an interval that does not start at a multiple of 64 leaves a remainder (only possible for the first one)
 #pragma unroll
     for (int a = 0; a < 8; ++a) ad.gs[(size_t)a * np + j] = accs[a * kBlockA + tid] + (double)acc.v[a];
@@ -527,6 +575,114 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
         for (int a = 0; a < 12; ++a) ad.seeds[(size_t)a * np + j] = seeds_l[a * kBlockA + tid];
     }
     ad.lam[j] = lx, ad.lam[np + j] = ly, ad.lam[2 * np + j] = lz;
+}
+
+// ---- Intervals reversed in chunks of segments, for cases with too few spins to fill the chip (no maps, no runs).
+//
+// Walked by one lane per spin, 55,296 spins keep one wave on each SIMD and wait for a record or a row at every segment.
+// The bare adjoint needs no state and the replay no adjoint: sweep_kernel takes both over the interval side by side
+// (workgroups [0, n_pad / 256) the replay, the rest lambda from lam after s1 to lam before s0, its value at every chunk's
+// end in lam_c); then adjoint_kernel<.., CHUNK> reverses the chunks, with their gradients, in parallel, and
+// chunk_sums_kernel adds them, last chunk first, in float64. Chunks start at multiples of their length, which depends
+// only on the number of spins, so the gradients are the same bit for bit for any interval length (a multiple of 64).
+// What bounds it then: the sweep's chain (0.31 us a segment, its records from the scalar cache one ahead) and the chunks'
+// VALU work. 24^3 x 4 spins (216 workgroups), every RF substep, 8 coils, 347 intervals of 384 segments, forward and
+// reverse: 271 -> 149 ms (533 us an interval in one walk, 318 in chunks); 28^3 x 4, 16 coils: 671 -> 284 ms; a 128^2
+// turbo spin echo's map fit (32 workgroups, 64 segments an interval): 81 -> 50 ms a call.
+template <int NC>
+__global__ __launch_bounds__(kBlockA) void sweep_kernel(hb_case cs_in, hb_adjoint ad_in, int s0, int s1, int chunk,
+                                                        float* __restrict__ lam_c, const hb_segment* __restrict__ segs,
+                                                        const float* __restrict__ spins,
+                                                        const float* __restrict__ pos_lo, const float* __restrict__ ckpt,
+                                                        const float* __restrict__ h, const float* __restrict__ sens) {
+    hb_case cs = cs_in;
+    cs.segs = segs, cs.spins = spins, cs.pos_lo = pos_lo;
+    hb_adjoint ad = ad_in;
+    ad.ckpt = ckpt;
+    const int np = cs.n_pad, n_blocks = np / kBlockA;
+    const bool back = (int)blockIdx.x >= n_blocks;  // uniform
+    const int j = ((int)blockIdx.x - (back ? n_blocks : 0)) * kBlockA + threadIdx.x;
+    touch_interval<NC>(segs, h, s0, s1);
+    const Spin p = load_spin(cs.spins, cs.pos_lo, np, j);
+    const float b1sq = p.b1 * p.b1;
+    if (!back) {
+        replay_interval<false>(cs, ad, p, b1sq, j, s0, s1);
+        return;
+    }
+    float sr[NC > 0 ? NC : 1], si[NC > 0 ? NC : 1];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        sr[c] = sens[(2 * c) * (size_t)np + j];
+        si[c] = sens[(2 * c + 1) * (size_t)np + j];
+    }
+    const Pos64 r64 = pos64(p);
+    float lx = ad.lam[j], ly = ad.lam[np + j], lz = ad.lam[2 * np + j];
+    Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    bool free_ok = false, rf_ok = false;
+    auto keep = [&](int s) {  // lambda after segment s, where s ends a chunk
+        if (s == s1 - 1 || ((s + 1 - s0) & (chunk - 1)) == 0) {
+            float* o = lam_c + (size_t)((s - s0) / chunk) * 3 * np + j;
+            o[0] = lx, o[np] = ly, o[2 * (size_t)np] = lz;
+        }
+    };
+    constexpr int kEnds = HB_ADC | HB_SPOIL;
+    for (int s = s1 - 1; s >= s0; --s) {
+        keep(s);
+        const int f0 = segs[s].flags;
+        if ((f0 & (HB_RF | kEnds)) == HB_RF) {  // RF segments without sample or spoil: the next record in flight
+            RfRec cur = load_rf(&segs[s]);
+            while (true) {
+                const RfRec nxt = load_rf(&segs[max(s - 1, s0)]);
+                lambda_rf(cur, rf_ok && (cur.flags & HB_NEXT_RF_DT), p, b1sq, lx, ly, lz, k);
+                rf_ok = true;
+                if (s == s0 || (nxt.flags & (HB_RF | kEnds)) != HB_RF) break;
+                --s;
+                keep(s);
+                cur = nxt;
+            }
+            continue;
+        }
+        const hb_segment q = segs[s];
+        const int f = live_flags(q.flags, free_ok, rf_ok, HB_NEXT_FREE, HB_NEXT_RF_DT);
+        if (f & HB_SPOIL) lx = ly = 0.0f;
+        if (NC > 0 && (f & HB_ADC)) {
+            const float* hrow = h + (size_t)q.pad[0] * 2 * NC;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const float hr = hrow[2 * c], hi = hrow[2 * c + 1];
+                lx += hr * sr[c] + hi * si[c];
+                ly += hi * sr[c] - hr * si[c];
+            }
+        }
+        if (f & HB_RF) {
+            lambda_rf(load_rf(&segs[s]), f & HB_NEXT_RF_DT, p, b1sq, lx, ly, lz, k);
+            rf_ok = true;
+        } else {
+            if (!(f & HB_NEXT_FREE)) {
+                sincospi(-2.0f * free_cycles(r64, p, q), &k.s, &k.c);
+                k.e1 = expm1x(-q.dt * p.r1);
+                k.e2 = expm1x(-q.dt * p.r2);
+            }
+            const float ax = k.c * lx + k.s * ly, ay = k.c * ly - k.s * lx;
+            lx = ax + ax * k.e2;
+            ly = ay + ay * k.e2;
+            lz = lz + lz * k.e1;
+            free_ok = true;
+        }
+    }
+    ad.lam[j] = lx, ad.lam[np + j] = ly, ad.lam[2 * np + j] = lz;
+}
+
+// Row a of the chunks' gradients added to gs (a < 8) or gc in float64, last chunk first; one lane per (row, spin).
+__global__ __launch_bounds__(kBlockA) void adjoint_chunk_sums_kernel(const float* __restrict__ part, int n_chunks,
+                                                                     int rows, int np, double* __restrict__ gs,
+                                                                     double* __restrict__ gc) {
+    const int a = blockIdx.y, j = blockIdx.x * kBlockA + threadIdx.x;
+    double* out = (a < 8 ? gs + (size_t)a * np : gc + (size_t)(a - 8) * np) + j;
+    double t = *out;
+#pragma unroll 8
+    for (int c = n_chunks - 1; c >= 0; --c) t += (double)part[((size_t)c * rows + a) * np + j];
+    *out = t;
 }
 
 // seg[s0 + k][g] = sum over workgroups of gseg[b][k][g], float64, in a fixed order: the workgroups in chunks of
@@ -566,7 +722,37 @@ static hipError_t launch_adjoint(const hb_case* cs, const hb_adjoint* ad, int s0
     auto kernel = ad->seg_grads ? (nu ? adjoint_kernel<NC, true, true> : adjoint_kernel<NC, true, false>)
                                 : (nu ? adjoint_kernel<NC, false, true> : adjoint_kernel<NC, false, false>);
     hipLaunchKernelGGL(kernel, grid, block, 0, st, *cs, *ad, s0, s1, cs->segs, cs->spins, cs->pos_lo, cs->maps,
-                       ad->ckpt, ad->h, ad->sens, ad->maps_d, ad->nu_params, ad->nu_win, ad->nu_grid);
+                       ad->ckpt, ad->h, ad->sens, ad->maps_d, ad->nu_params, ad->nu_win, ad->nu_grid, 0, nullptr,
+                       nullptr);
+    return hipGetLastError();
+}
+
+// Segments per chunk of a case of n_blocks workgroups, or 0: not in chunks. Chunks are as long as 256 workgroups per 64
+// segments allow (32 workgroups: 8 segments, measured 50 ms against 54 with 16). In chunks the reverse also needs no
+// float64 sums in LDS, so it gains beyond a full chip: 512 workgroups 457 -> 449 ms, 1,000 workgroups 1,395 -> 1,239 ms;
+// the line is the largest size measured (the workspace grows with the spins).
+constexpr int kChunkBlocks = 1024;
+
+static int chunk_of(int n_blocks) {
+    if (n_blocks > kChunkBlocks) return 0;
+    int chunk = 8;
+    while (chunk < 64 && 64 / (2 * chunk) * n_blocks >= 256) chunk *= 2;
+    return chunk;
+}
+
+template <int NC>
+static hipError_t launch_chunks(const hb_case* cs, const hb_adjoint* ad, int s0, int s1, float* work, hipStream_t st) {
+    const int n_blocks = cs->n_pad / kBlockA, chunk = chunk_of(n_blocks), n_chunks = (s1 - s0 + chunk - 1) / chunk;
+    float* part = work + (size_t)n_chunks * 3 * cs->n_pad;
+    hipLaunchKernelGGL((sweep_kernel<NC>), dim3(2 * n_blocks), dim3(kBlockA), 0, st, *cs, *ad, s0, s1, chunk, work,
+                       cs->segs, cs->spins, cs->pos_lo, ad->ckpt, ad->h, ad->sens);
+    auto kernel = ad->seg_grads ? adjoint_kernel<NC, true, false, true> : adjoint_kernel<NC, false, false, true>;
+    hipLaunchKernelGGL(kernel, dim3(n_blocks, n_chunks), dim3(kBlockA), 0, st, *cs, *ad, s0, s1, cs->segs, cs->spins,
+                       cs->pos_lo, cs->maps, ad->ckpt, ad->h, ad->sens, ad->maps_d, ad->nu_params, ad->nu_win,
+                       ad->nu_grid, chunk, work, part);
+    const int coil_rows = NC > 0 && ad->coil_grads ? 2 * NC : 0;
+    hipLaunchKernelGGL(adjoint_chunk_sums_kernel, dim3(n_blocks, 8 + coil_rows), dim3(kBlockA), 0, st, part, n_chunks,
+                       8 + 2 * NC, cs->n_pad, ad->gs, ad->gc);
     return hipGetLastError();
 }
 
@@ -586,6 +772,33 @@ extern "C" int hb_adjoint_interval(const hb_case* cs, const hb_adjoint* ad, int3
         case 4: return launch_adjoint<4>(cs, ad, s0, s1, st);
         case 8: return launch_adjoint<8>(cs, ad, s0, s1, st);
         case 16: return launch_adjoint<16>(cs, ad, s0, s1, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+extern "C" int64_t hb_adjoint_chunks_workspace(int32_t n_pad, int32_t k_max, int32_t nc) {
+    using namespace hb;
+    if (n_pad < kBlockA || n_pad % kBlockA || k_max < 1 || nc < 0 || nc > 16) return 0;
+    const int chunk = chunk_of(n_pad / kBlockA);
+    return chunk ? (int64_t)((k_max + chunk - 1) / chunk) * (3 + 8 + 2 * nc) * n_pad : 0;
+}
+
+extern "C" int hb_adjoint_chunks(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, float* work,
+                                 void* stream) {
+    using namespace hb;
+    if (!cs || !ad || cs->n_pad <= 0 || cs->n_pad % kBlockA) return hipErrorInvalidValue;
+    if (s0 < 0 || s1 < s0 || s1 > cs->n_segments || s1 - s0 > ad->k_max) return hipErrorInvalidValue;
+    if (!work || cs->n_pulses || ad->nu_params || s0 % 64 || !chunk_of(cs->n_pad / kBlockA))
+        return hb_adjoint_interval(cs, ad, s0, s1, stream);
+    if (s1 == s0) return hipSuccess;
+    hipStream_t st = (hipStream_t)stream;
+    switch (ad->nc) {
+        case 0: return launch_chunks<0>(cs, ad, s0, s1, work, st);
+        case 1: return launch_chunks<1>(cs, ad, s0, s1, work, st);
+        case 2: return launch_chunks<2>(cs, ad, s0, s1, work, st);
+        case 4: return launch_chunks<4>(cs, ad, s0, s1, work, st);
+        case 8: return launch_chunks<8>(cs, ad, s0, s1, work, st);
+        case 16: return launch_chunks<16>(cs, ad, s0, s1, work, st);
         default: return hipErrorInvalidValue;
     }
 }

@@ -237,13 +237,15 @@ def _sweep(case, cs, ckpts, every, h, lam, sens, nc, need_seg, need_coil, lib, s
         grid = torch.empty(len(pl.runs) * pl.terms * pl.ng * 2 * nc, dtype=torch.float32, device=dev)
         lib.nufft_adjoint_grid(h.data_ptr(), nc, nu["row_of"].data_ptr(), len(pl.runs), pl.n, pl.ng, pl.terms,
                                nu["nu_tw"].data_ptr(), nu["nu_lw"].data_ptr(), grid.data_ptr())
+    need = hip.load().hb_adjoint_chunks_workspace(n_pad, every, nc) if not case.n_pulses and nu is None else 0
+    work = torch.empty(need, dtype=torch.float32, device=dev) if need else None
     for c in reversed(range(len(ckpts))):
         s0, s1 = case.starts[c], case.ends[c]
         ad = hip.HbAdjoint(ckpts[c].data_ptr(), r8.data_ptr(), lam.data_ptr(), gs.data_ptr(), gc.data_ptr(),
                            gseg.data_ptr(), h.data_ptr(), sens.data_ptr(), ptr(maps_d), ptr(seeds),
                            None if nu is None else nu["nu"].data_ptr(), None if nu is None else nu["nu_win"].data_ptr(),
                            ptr(grid), nc, int(need_seg), int(need_coil), every)
-        lib.adjoint_interval(ctypes.byref(cs), ctypes.byref(ad), s0, s1)
+        lib.adjoint_chunks(ctypes.byref(cs), ctypes.byref(ad), s0, s1, ptr(work))
         if need_seg:
             lib.seg_reduce(gseg.data_ptr(), n_blocks, every, s0, s1 - s0, red.data_ptr(), seg.data_ptr(),
                            case.segs.data_ptr())

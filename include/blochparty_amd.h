@@ -319,6 +319,14 @@ typedef struct hb_adjoint {
 
 int hb_adjoint_interval(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, void* stream);
 
+/* The same with a workspace of hb_adjoint_chunks_workspace(n_pad, k_max, nc) floats: an interval of a table without
+ * reused pulses and NUFFT runs (n_pulses 0, nu_params NULL) that starts at a multiple of 64, of a case with too few
+ * spins to fill the chip, is reversed in chunks of segments side by side, from the adjoint at each chunk's end (found by
+ * a sweep of its own beside the replay); the chunks' gradients are added in a fixed order, the same bit for bit for any
+ * interval length. Any other interval, and work NULL (also where the workspace is 0): as hb_adjoint_interval. */
+int64_t hb_adjoint_chunks_workspace(int32_t n_pad, int32_t k_max, int32_t nc);
+int hb_adjoint_chunks(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, float* work, void* stream);
+
 /* Fixed-order sum of an interval's per-workgroup segment gradients (replaces seg_reduce, cuda/seg_reduce.cu:3-11):
  * seg[(s0 + k) * 8 + g] = sum over b < n_blocks of gseg[(b * k_max + k) * 8 + g], float64, for k < len (the
  * workgroups in chunks of 256, each summed in order, then the chunks in order). work:
