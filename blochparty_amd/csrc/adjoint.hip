@@ -19,6 +19,7 @@
 // Reused pulses (maps) and NUFFT readout runs are one record each, their other segments identity bodies: the replay
 // jumps over them, the reverse skips the 8-blocks inside them (pulse_reverse, nufft_reverse below).
 #include "adjoint_device.h"
+#include "nufft_back.h"
 
 namespace hb {
 
@@ -162,19 +163,18 @@ __device__ __forceinline__ void pulse_reverse(const hb_segment& q, const hb_case
 //      A_c; for a parameter theta of K, dL/dtheta = Re(m0 conj(sum_c conj(S_c) dA_c/dtheta)): R2 through the decay
 //      terms (-tau_m e^{-R2 tau_m}), the phase per sample through ph and the cells' z (psi', dz/dfr = -ng 2 / width).
 // The phase per sample cyc = bz dt (bz = g.r + db0 + b0_offset) gives the position and db0 gradients.
-template <int NC>
+// OUT: the samples (2.) were taken beside the sweep (nufft_back.hip): qx, qy is what they add to lambda.
+template <int NC, bool OUT>
 __device__ __forceinline__ void nufft_reverse(const hb_segment& q, const hb_adjoint& ad, const Spin& p,
-                                              const Stash& m0, float& lx, float& ly, float& lz, Acc& acc,
+                                              const Stash& m0, float qx, float qy, float& lx, float& ly, float& lz, Acc& acc,
                                               const float (&sr)[NC > 0 ? NC : 1], const float (&si)[NC > 0 ? NC : 1],
                                               float (&gr)[NC > 0 ? NC : 1], float (&gi)[NC > 0 ? NC : 1]) {
     const float* par = ad.nu_params;
     const int L = q.pad[3], kind = q.pad[2], run = q.pad[4];
-    const int ng = (int)par[0], terms = (int)par[2], shift = (int)par[4];
-    const float hz = par[6 + HB_NUFFT_MAX_TERMS], bl2 = par[7 + HB_NUFFT_MAX_TERMS];
-    const double cyc = free_cycles64(pos64(p), p, q);
     const float T = (float)L * q.dt;
     float dcyc = 0.0f;  // dL/dcyc
     // 1. the jump
+    const double cyc = free_cycles64(pos64(p), p, q);
     if (q.flags & (HB_XY_DEAD | HB_PULSE_SPOIL)) {
         lx = ly = 0.0f;
     } else {
@@ -197,7 +197,11 @@ __device__ __forceinline__ void nufft_reverse(const hb_segment& q, const hb_adjo
         lz = lz + lz * d1;
     }
     // 2. the samples
-    if constexpr (NC > 0) {
+    if constexpr (OUT) {
+        lx += qx, ly += qy;
+    } else if constexpr (NC > 0) {
+        const int ng = (int)par[0], terms = (int)par[2], shift = (int)par[4];
+        const float hz = par[6 + HB_NUFFT_MAX_TERMS], bl2 = par[7 + HB_NUFFT_MAX_TERMS];
         const double fr = cyc - floor(cyc);
         const double xg = fr * ng;
         double ph = fr * shift;
@@ -278,9 +282,10 @@ __device__ __forceinline__ void touch_interval(const hb_segment* __restrict__ se
 }
 
 // The interval replayed from its checkpoint: r8[b] = the state before segment s0 + 8 b (low parts folded).
+// m0: (with NU) Mx, My at the start of every run r of the interval into rows 2 (r - r0), 2 (r - r0) + 1, or NULL.
 template <bool NU>
 __device__ __forceinline__ void replay_interval(const hb_case& cs, const hb_adjoint& ad, const Spin& p, float b1sq, int j,
-                                                int s0, int s1) {
+                                                int s0, int s1, float* __restrict__ m0 = nullptr, int r0 = 0) {
     const int np = cs.n_pad;
     State m = load_state(ad.ckpt, np, j);
     Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
@@ -307,6 +312,10 @@ __device__ __forceinline__ void replay_interval(const hb_case& cs, const hb_adjo
             continue;
         }
         if (NU && (q.flags & HB_NUFFT)) {  // a readout run: its jump (its samples add nothing to the state)
+            if (m0) {
+                float* o = m0 + (size_t)(2 * (q.pad[4] - r0)) * np + j;
+                o[0] = m.mx, o[np] = m.my;
+            }
             run_jump(q, p, free_cycles64(pos64(p), p, q), expm1x(-((float)q.pad[3] * q.dt) * p.r1), m);
             const int e = min(s + q.pad[3], s1);
             r8_after_span(ad.r8, np, j, s0, s1, s, e, m);
@@ -344,7 +353,9 @@ __device__ __forceinline__ void replay_interval(const hb_case& cs, const hb_adjo
 // CHUNK: the reverse of chunk blockIdx.y ([s0 + chunk y, ...), chunk a power of two from 8 to 64) of an interval without
 // maps and runs that sweep_kernel has replayed: from the adjoint at the chunk's end (lam_c), its gradients, float32 sums
 // over the chunk as between two flushes below, into part[y] (8 + 2 NC, n_pad) for chunk_sums_kernel.
-template <int NC, bool SEG, bool NU, bool CHUNK = false>
+// OUT (with NU): replayed by runs_replay_kernel, the runs' samples taken by nufft_back.hip (lam_c: their rows, two per
+// run, of the interval's runs from chunk on).
+template <int NC, bool SEG, bool NU, bool CHUNK = false, bool OUT = false>
 __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8 ? 2 : 1))) void adjoint_kernel(
     hb_case cs_in, hb_adjoint ad_in, int s0, int s1, const hb_segment* __restrict__ segs,
     const float* __restrict__ spins, const float* __restrict__ pos_lo, const float* __restrict__ maps,
@@ -384,7 +395,7 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
     const bool rf_only = SEG && ad.seg_grads == 2;
 
     // 1. replay the interval
-    if constexpr (!CHUNK) replay_interval<NU>(cs, ad, p, b1sq, j, s0, s1);
+    if constexpr (!CHUNK && !OUT) replay_interval<NU>(cs, ad, p, b1sq, j, s0, s1);
 
     // 2. reverse sweep
     const float* l0 = CHUNK ? lam_c + (size_t)blockIdx.y * 3 * np : ad.lam;
@@ -473,7 +484,12 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
                 if (!CHUNK && (q.flags & HB_PULSE_BODY)) continue;  // the identity, no gradients
                 if constexpr (NU) {
                     if (q.flags & HB_NUFFT) {
-                        nufft_reverse<NC>(q, ad, p, before[i], lx, ly, lz, acc, sr, si, gr, gi);
+                        float qx = 0.0f, qy = 0.0f;
+                        if constexpr (OUT) {
+                            const float* o = lam_c + (size_t)(2 * (q.pad[4] - chunk)) * np + j;
+                            qx = o[0], qy = o[np];
+                        }
+                        nufft_reverse<NC, OUT>(q, ad, p, before[i], qx, qy, lx, ly, lz, acc, sr, si, gr, gi);
                         dirty = true;
                         continue;
                     }
@@ -757,6 +773,60 @@ static hipError_t launch_chunks(const hb_case* cs, const hb_adjoint* ad, int s0,
 }
 
 }  // namespace hb
+
+namespace hb {
+// The replay alone, for the intervals whose runs are taken beside the sweep.
+__global__ __launch_bounds__(kBlockA) void runs_replay_kernel(hb_case cs_in, hb_adjoint ad_in, int s0, int s1,
+                                                              const hb_segment* __restrict__ segs,
+                                                              const float* __restrict__ spins,
+                                                              const float* __restrict__ pos_lo,
+                                                              const float* __restrict__ maps,
+                                                              const float* __restrict__ ckpt, float* __restrict__ m0,
+                                                              int r0) {
+    hb_case cs = cs_in;
+    cs.segs = segs, cs.spins = spins, cs.pos_lo = pos_lo, cs.maps = maps;
+    hb_adjoint ad = ad_in;
+    ad.ckpt = ckpt;
+    const int j = blockIdx.x * kBlockA + threadIdx.x;
+    touch_interval<0>(segs, nullptr, s0, s1);
+    const Spin p = load_spin(cs.spins, cs.pos_lo, cs.n_pad, j);
+    replay_interval<true>(cs, ad, p, p.b1 * p.b1, j, s0, s1, m0, r0);
+}
+
+template <int NC>
+static void launch_runs(const hb_case* cs, const hb_adjoint* ad, int s0, int s1, int r0, const float* q, hipStream_t st) {
+    auto kernel = ad->seg_grads ? adjoint_kernel<NC, true, true, false, true> : adjoint_kernel<NC, false, true, false, true>;
+    hipLaunchKernelGGL(kernel, dim3(cs->n_pad / kBlockA), dim3(kBlockA), 0, st, *cs, *ad, s0, s1, cs->segs, cs->spins,
+                       cs->pos_lo, cs->maps, ad->ckpt, ad->h, ad->sens, ad->maps_d, ad->nu_params, ad->nu_win,
+                       ad->nu_grid, r0, q, nullptr);
+}
+}  // namespace hb
+
+extern "C" int hb_adjoint_runs(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, const int32_t* heads,
+                               int32_t r0, int32_t r1, int32_t cols, float* work, double* g, void* stream) {
+    using namespace hb;
+    if (!cs || !ad || cs->n_pad <= 0 || cs->n_pad % kBlockA) return hipErrorInvalidValue;
+    if (s0 < 0 || s1 < s0 || s1 > cs->n_segments || s1 - s0 > ad->k_max) return hipErrorInvalidValue;
+    if (!ad->nu_params || !ad->nu_win || !ad->nu_grid || r0 < 0 || r1 < r0 || (r1 > r0 && (!heads || !work || !g)))
+        return hipErrorInvalidValue;
+    if (!nufft_back_takes(ad->nc, cols)) return hipErrorInvalidValue;
+    if (s1 == s0) return hipSuccess;
+    hipStream_t st = (hipStream_t)stream;
+    float* q = work + (size_t)2 * (r1 - r0) * cs->n_pad;
+    hipLaunchKernelGGL(runs_replay_kernel, dim3(cs->n_pad / kBlockA), dim3(kBlockA), 0, st, *cs, *ad, s0, s1, cs->segs,
+                       cs->spins, cs->pos_lo, cs->maps, ad->ckpt, work, r0);
+    if (r1 > r0) launch_nufft_back({work, q, g, cs->n_pad, r0, r1, ad->coil_grads}, *cs, *ad, heads, st);
+    switch (ad->nc) {
+        case 1: launch_runs<1>(cs, ad, s0, s1, r0, q, st); break;
+        case 2: launch_runs<2>(cs, ad, s0, s1, r0, q, st); break;
+        case 4: launch_runs<4>(cs, ad, s0, s1, r0, q, st); break;
+        case 8: launch_runs<8>(cs, ad, s0, s1, r0, q, st); break;
+        default: launch_runs<16>(cs, ad, s0, s1, r0, q, st); break;
+    }
+    return hipGetLastError();
+}
+
+extern "C" int32_t hb_adjoint_runs_takes(int32_t nc, int32_t cols) { return hb::nufft_back_takes(nc, cols); }
 
 extern "C" int hb_adjoint_interval(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, void* stream) {
     using namespace hb;

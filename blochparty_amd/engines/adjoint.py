@@ -239,16 +239,33 @@ def _sweep(case, cs, ckpts, every, h, lam, sens, nc, need_seg, need_coil, lib, s
                                nu["nu_tw"].data_ptr(), nu["nu_lw"].data_ptr(), grid.data_ptr())
     need = hip.load().hb_adjoint_chunks_workspace(n_pad, every, nc) if not case.n_pulses and nu is None else 0
     work = torch.empty(need, dtype=torch.float32, device=dev) if need else None
+    runs = None
+    if grid is not None and hip.load().hb_adjoint_runs_takes(nc, nu["cols"]):
+        heads = np.fromiter((a for a, _ in nu["plan"].runs), dtype=np.int32, count=len(nu["plan"].runs))
+        at = np.searchsorted(heads, [*case.starts, case.ends[-1]])  # each interval's first run
+        runs = (torch.from_numpy(heads).to(dev),
+                torch.empty(4 * max(1, int(np.diff(at).max())) * n_pad, dtype=torch.float32, device=dev),
+                torch.zeros(5 + 2 * nc, n_pad, dtype=torch.float64, device=dev), at)
     for c in reversed(range(len(ckpts))):
         s0, s1 = case.starts[c], case.ends[c]
         ad = hip.HbAdjoint(ckpts[c].data_ptr(), r8.data_ptr(), lam.data_ptr(), gs.data_ptr(), gc.data_ptr(),
                            gseg.data_ptr(), h.data_ptr(), sens.data_ptr(), ptr(maps_d), ptr(seeds),
                            None if nu is None else nu["nu"].data_ptr(), None if nu is None else nu["nu_win"].data_ptr(),
                            ptr(grid), nc, int(need_seg), int(need_coil), every)
-        lib.adjoint_chunks(ctypes.byref(cs), ctypes.byref(ad), s0, s1, ptr(work))
+        if runs is not None:  # the runs' samples beside the sweep
+            lib.adjoint_runs(ctypes.byref(cs), ctypes.byref(ad), s0, s1, runs[0].data_ptr(), int(runs[3][c]),
+                             int(runs[3][c + 1]), nu["cols"], runs[1].data_ptr(), runs[2].data_ptr())
+        else:
+            lib.adjoint_chunks(ctypes.byref(cs), ctypes.byref(ad), s0, s1, ptr(work))
         if need_seg:
             lib.seg_reduce(gseg.data_ptr(), n_blocks, every, s0, s1 - s0, red.data_ptr(), seg.data_ptr(),
                            case.segs.data_ptr())
+    if runs is not None:
+        g = runs[2]
+        gs[6] += g[0]
+        gs[:4] += g[1:5]
+        if need_coil:
+            gc += g[5:]
 
 
 FD_TURN = 1e-4  # rad: how far a central-difference step turns a reused pulse's rotation

@@ -93,6 +93,7 @@ SIGNATURES = {
     "hb_nufft_adjoint_grid": [_P, _I, _P, _I, _I, _I, _I, _P, _P, _P, _V],
     "hb_adjoint_interval": [ctypes.POINTER(HbCase), ctypes.POINTER(HbAdjoint), _I, _I, _V],
     "hb_adjoint_chunks": [ctypes.POINTER(HbCase), ctypes.POINTER(HbAdjoint), _I, _I, _P, _V],
+    "hb_adjoint_runs": [ctypes.POINTER(HbCase), ctypes.POINTER(HbAdjoint), _I, _I, _P, _I, _I, _I, _P, _P, _V],
     "hb_seg_reduce": [_P, _I, _I, _I, _I, _P, _P, _P, _V],
     "hb_pulse_maps": [ctypes.POINTER(HbCase), _P, _P, _I, _P, _I, _P, _V],
     "hb_pulse_map_grads": [ctypes.POINTER(HbCase), _P, _P, _I, _P, _P, _P, _V],
@@ -124,6 +125,8 @@ def load() -> ctypes.CDLL:
         lib.hb_abi_version.restype = ctypes.c_int
         lib.hb_mlp_workspace.restype = ctypes.c_int64
         lib.hb_mlp_workspace.argtypes = [ctypes.c_int32]
+        lib.hb_adjoint_runs_takes.restype = ctypes.c_int32
+        lib.hb_adjoint_runs_takes.argtypes = [ctypes.c_int32] * 2
         lib.hb_adjoint_chunks_workspace.restype = ctypes.c_int64
         lib.hb_adjoint_chunks_workspace.argtypes = [ctypes.c_int32] * 3
         lib.hb_signal_reduce_workspace.restype = ctypes.c_int64

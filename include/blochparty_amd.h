@@ -327,6 +327,18 @@ int hb_adjoint_interval(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int
 int64_t hb_adjoint_chunks_workspace(int32_t n_pad, int32_t k_max, int32_t nc);
 int hb_adjoint_chunks(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, float* work, void* stream);
 
+/* The same for an interval of a table with NUFFT runs, the runs' samples taken beside the sweep (they need neither the
+ * adjoint nor, but for their gradients, the state): the replay, leaving each run's starting Mxy; then for the runs
+ * [r0, r1) whose first segments, heads[r] (int32, one per run of the table), lie in the interval, what they add to lambda
+ * and their gradients, added to g: (5 + 2 nc, n_pad) float64, dL/d(R2, px, py, pz, db0) and (with coil_grads) the coil
+ * gradients, which the caller adds to gs and gc after its last interval (kept apart, they are added run by run and so the
+ * same bit for bit for any interval length); then the sweep with its other gradients into gs and gc. work: 4 (r1 - r0)
+ * n_pad floats. Taken where hb_adjoint_runs_takes(nc, cols) says so, cols the largest window's cells times the terms;
+ * otherwise hipErrorInvalidValue (hb_adjoint_interval takes every table). */
+int32_t hb_adjoint_runs_takes(int32_t nc, int32_t cols);
+int hb_adjoint_runs(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, const int32_t* heads, int32_t r0,
+                    int32_t r1, int32_t cols, float* work, double* g, void* stream);
+
 /* Fixed-order sum of an interval's per-workgroup segment gradients (replaces seg_reduce, cuda/seg_reduce.cu:3-11):
  * seg[(s0 + k) * 8 + g] = sum over b < n_blocks of gseg[(b * k_max + k) * 8 + g], float64, for k < len (the
  * workgroups in chunks of 256, each summed in order, then the chunks in order). work:
