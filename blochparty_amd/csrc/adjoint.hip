@@ -297,7 +297,12 @@ __device__ __forceinline__ void replay_interval(const hb_case& cs, const hb_adjo
         r8_after_span(ad.r8, np, j, s0, s1, s0 - 1, e, m);
         s_start = e;
     }
+    int warm = s_start;
     for (int s = s_start; s < s1; ++s) {
+        if (s >= warm && s + 8 <= s1) {
+            warm_records(cs.segs + s);
+            warm = s + 8;
+        }
         if (((s - s0) & 7) == 0) {
             float* r = ad.r8 + (size_t)((s - s0) >> 3) * 3 * np;
             r[j] = m.mx, r[np + j] = m.my, r[2 * np + j] = m.mz + m.lz;
@@ -322,19 +327,20 @@ __device__ __forceinline__ void replay_interval(const hb_case& cs, const hb_adjo
             s = e - 1;
             continue;
         }
-        if (q.flags & HB_TRAIN) {  // an RF train: its own loop, the next record in flight (forward_kernel's)
+        if (q.flags & HB_TRAIN) {  // an RF train: its own loop, the next records in flight (forward_kernel's)
             const int L = min(q.pad[3], s1 - s);
-            RfRec cur = load_rf(&cs.segs[s]);
-            for (int i = 1; i <= L; ++i) {
-                const RfRec nxt = load_rf(&cs.segs[s + (i < L ? i : 0)]);
-                if (i > 1 && ((s + i - 1 - s0) & 7) == 0) {
-                    float* r = ad.r8 + (size_t)((s + i - 1 - s0) >> 3) * 3 * np;
-                    r[j] = m.mx, r[np + j] = m.my, r[2 * np + j] = m.mz + m.lz;
-                }
-                rf_step(cur, live_flags(cur.flags, true, rf_ok, 0, HB_SAME_RF_DT), p, b1sq, m, k);
-                rf_ok = true;
-                cur = nxt;
-            }
+            const hb_segment* first = cs.segs + s;
+            rf_records(
+                L, [&](int i) { return first + i; },
+                [&](int i, const RfRec& c) {
+                    if (i > 0 && ((s + i - s0) & 7) == 0) {
+                        float* r = ad.r8 + (size_t)((s + i - s0) >> 3) * 3 * np;
+                        r[j] = m.mx, r[np + j] = m.my, r[2 * np + j] = m.mz + m.lz;
+                    }
+                    if (!rf_ok || !(c.flags & HB_SAME_RF_DT)) half_relax(first[i].dt, p, k);
+                    rf_step(c, p, b1sq, m, k);
+                    rf_ok = true;
+                });
             s += L - 1;
             continue;
         }
@@ -443,6 +449,7 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
             const float* r = ad.r8 + (size_t)b * 3 * np;
             State m;
             m.mx = r[j], m.my = r[np + j], m.mz = r[2 * np + j], m.lz = 0.0f;
+            if (sb + 8 <= s1) warm_records(cs.segs + sb);
             Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             bool free_ok = false, rf_ok = false;
 #pragma unroll
@@ -642,20 +649,41 @@ __global__ __launch_bounds__(kBlockA) void sweep_kernel(hb_case cs_in, hb_adjoin
         }
     };
     constexpr int kEnds = HB_ADC | HB_SPOIL;
+    int warm = s1 - 1;
     for (int s = s1 - 1; s >= s0; --s) {
+        if (s <= warm && s - 7 >= s0) {
+            warm_records(segs + s - 7);
+            warm = s - 8;
+        }
         keep(s);
         const int f0 = segs[s].flags;
-        if ((f0 & (HB_RF | kEnds)) == HB_RF) {  // RF segments without sample or spoil: the next record in flight
-            RfRec cur = load_rf(&segs[s]);
-            while (true) {
-                const RfRec nxt = load_rf(&segs[max(s - 1, s0)]);
-                lambda_rf(cur, rf_ok && (cur.flags & HB_NEXT_RF_DT), p, b1sq, lx, ly, lz, k);
-                rf_ok = true;
-                if (s == s0 || (nxt.flags & (HB_RF | kEnds)) != HB_RF) break;
-                --s;
-                keep(s);
-                cur = nxt;
+        if ((f0 & (HB_RF | kEnds)) == HB_RF) {  // RF segments without sample or spoil: the next records in flight
+            const hb_segment* last = segs + s;
+            const int n = s - s0 + 1;
+            RfRec cur[kTrain], nxt[kTrain];
+#pragma unroll
+            for (int i = 0; i < kTrain; ++i) cur[i] = load_rf(last - min(i, n - 1));
+            int done = 0;
+            for (bool more = true; more;) {
+#pragma unroll
+                for (int i = 0; i < kTrain; ++i) nxt[i] = load_rf(last - min(done + kTrain + i, n - 1));
+                const int d0 = done;
+#pragma unroll
+                for (int i = 0; i < kTrain; ++i) {
+                    if (more) {
+                        if (done) keep(s - done);
+                        if (!rf_ok || !(cur[i].flags & HB_NEXT_RF_DT)) half_relax(last[-done].dt, p, k);
+                        lambda_rf(cur[i], p, b1sq, lx, ly, lz, k);
+                        rf_ok = true;
+                        ++done;
+                        const int fn = i + 1 < kTrain ? cur[i + 1].flags : nxt[0].flags;
+                        more = d0 + i + 1 < n && (fn & (HB_RF | kEnds)) == HB_RF;
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < kTrain; ++i) cur[i] = nxt[i];
             }
+            s -= done - 1;
             continue;
         }
         const hb_segment q = segs[s];
@@ -671,7 +699,8 @@ __global__ __launch_bounds__(kBlockA) void sweep_kernel(hb_case cs_in, hb_adjoin
             }
         }
         if (f & HB_RF) {
-            lambda_rf(load_rf(&segs[s]), f & HB_NEXT_RF_DT, p, b1sq, lx, ly, lz, k);
+            if (!(f & HB_NEXT_RF_DT)) half_relax(q.dt, p, k);
+            lambda_rf(load_rf(&segs[s]), p, b1sq, lx, ly, lz, k);
             rf_ok = true;
         } else {
             if (!(f & HB_NEXT_FREE)) {

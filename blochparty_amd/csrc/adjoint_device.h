@@ -41,25 +41,21 @@ __device__ __forceinline__ void rot_factors(float p2, float& c, float& s1, float
     }
 }
 
-// lambda alone back through an RF segment (its transpose needs no state): the steps of reverse_step's. same: k.h1, k.h2
-// hold for its dt.
-__device__ __forceinline__ void lambda_rf(const RfRec& q, bool same, const Spin& p, float b1sq, float& lx, float& ly,
-                                          float& lz, Cache& k) {
-    if (!same) {
-        k.h1 = expm1x(-0.5f * q.dt * p.r1);
-        k.h2 = expm1x(-0.5f * q.dt * p.r2);
-    }
+// lambda alone back through an RF segment (its transpose needs no state): the steps of reverse_step's, k.h1 and
+// k.h2 the half relaxations of its dt.
+__device__ __forceinline__ void lambda_rf(const RfRec& q, const Spin& p, float b1sq, float& lx, float& ly, float& lz,
+                                          const Cache& k) {
+#pragma clang fp contract(off)
     const float wx = p.b1 * q.w_rf_x, wy = p.b1 * q.w_rf_y;
-    const float wz = p.px * q.w_g_x + p.py * q.w_g_y + p.pz * q.w_g_z + (p.db0 * q.w + q.w_b0);
-    float s1, s2;
-    rot_ab(b1sq * q.w_rf2 + wz * wz, s1, s2);
-    const float ax = lx + lx * k.h2, ay = ly + ly * k.h2, az = lz + lz * k.h1;
-    const float cx = wy * az - wz * ay, cy = wz * ax - wx * az, cz = wx * ay - wy * ax;
-    const float ex = wy * cz - wz * cy, ey = wz * cx - wx * cz, ez = wx * cy - wy * cx;
-    const float bx = ax + (s2 * ex - s1 * cx), by = ay + (s2 * ey - s1 * cy), bz = az + (s2 * ez - s1 * cz);
-    lx = bx + bx * k.h2;
-    ly = by + by * k.h2;
-    lz = bz + bz * k.h1;
+    float wz, phi2, s1, s2, dx, dy, dz;
+    rf_angles(q, p, b1sq, wz, phi2);
+    rot_ab(phi2, s1, s2);
+    const float ax = fmaf(lx, k.h2, lx), ay = fmaf(ly, k.h2, ly), az = fmaf(lz, k.h1, lz);
+    rotate_less(wx, wy, wz, -s1, s2, ax, ay, az, dx, dy, dz);
+    const float bx = ax + dx, by = ay + dy, bz = az + dz;
+    lx = fmaf(bx, k.h2, bx);
+    ly = fmaf(by, k.h2, by);
+    lz = fmaf(bz, k.h1, bz);
 }
 
 // Reverse through segment q from the state (x0, y0, z0) before it. (lx, ly, lz): dL/d(state after) in, dL/d(state

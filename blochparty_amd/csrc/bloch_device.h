@@ -172,6 +172,16 @@ __device__ __forceinline__ void store_state(float* __restrict__ st, int n_pad, i
     st[3 * n_pad + j] = 0.0f, st[4 * n_pad + j] = 0.0f, st[5 * n_pad + j] = m.lz;
 }
 
+// Mxy turned by (c, s) and decayed by 1 + e2. Here and in the RF steps below the fused operations are written out and the
+// compiler forms no others, so that the copies of an unrolled loop and of the kernels' loops, and with them a table cut
+// into other dispatches or intervals, give the same bits.
+__device__ __forceinline__ void precess(float c, float s, float e2, State& m) {
+#pragma clang fp contract(off)
+    const float nx = fmaf(c, m.mx, -(s * m.my)), ny = fmaf(s, m.mx, c * m.my);
+    m.mx = fmaf(nx, e2, nx);
+    m.my = fmaf(ny, e2, ny);
+}
+
 // The jump over a readout run of L = q.pad[3] samples (q its first segment): one exact free step of L dt, phase
 // L cyc (cyc the segment's float64 phase in cycles), Mxy zeroed instead when the run ends spoiled or its Mxy is never
 // read; Mz relaxes by e1 = expm1(-L dt R1).
@@ -185,9 +195,7 @@ __device__ __forceinline__ void run_jump(const hb_segment& q, const Spin& p, dou
         float s2, c2;
         sincospi(-2.0f * (float)cl, &s2, &c2);
         const float e2 = expm1x(-T * p.r2);
-        const float nx = c2 * m.mx - s2 * m.my, ny = s2 * m.mx + c2 * m.my;
-        m.mx = nx + nx * e2;
-        m.my = ny + ny * e2;
+        precess(c2, s2, e2, m);
     }
     two_sum(m.mz, m.lz, (m.mz - p.pd) * e1);
 }
@@ -215,39 +223,54 @@ __device__ __forceinline__ void apply_map(const float* __restrict__ U, int np, f
 // rounding Mz to float32 after every segment biases the steady state (2e-5 of the signal of a 264-TR spoiled GRE,
 // against 5e-7 with two-sum); the transverse components are rotated and spoiled, so their rounding does not build up
 // (a 5,000-substep CW saturation stays within 1e-6 of float64 without it).
-// The fields of a record an RF step reads (dt, flags and the rotation factors): a train loop loads the next one while
-// it steps the current one.
+// The fields of a record an RF step reads but its dt, which only the first of equal ones needs: one 64-byte line.
 struct RfRec {
-    float dt, w, w_rf_x, w_rf_y, w_g_x, w_g_y, w_g_z, w_b0, w_rf2;
+    float w, w_rf_x, w_rf_y, w_g_x, w_g_y, w_g_z, w_b0, w_rf2;
     int flags;
 };
 
 __device__ __forceinline__ RfRec load_rf(const hb_segment* __restrict__ r) {
     const float4 a = *reinterpret_cast<const float4*>(&r->w), b = *reinterpret_cast<const float4*>(&r->w_g_y);
-    return {r->dt, a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, r->flags};
+    return {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, r->flags};
 }
 
+__device__ __forceinline__ void half_relax(float dt, const Spin& p, Cache& k) {
+    k.h1 = expm1x(-0.5f * dt * p.r1);
+    k.h2 = expm1x(-0.5f * dt * p.r2);
+}
+
+// The rotation of (x, y, z) by the vector (wx, wy, wz), less the vector itself: s1 (w x v) + s2 (w x (w x v)).
+__device__ __forceinline__ void rotate_less(float wx, float wy, float wz, float s1, float s2, float x, float y, float z,
+                                            float& dx, float& dy, float& dz) {
+#pragma clang fp contract(off)
+    const float cx = fmaf(wy, z, -(wz * y)), cy = fmaf(wz, x, -(wx * z)), cz = fmaf(wx, y, -(wy * x));
+    const float ex = fmaf(wy, cz, -(wz * cy)), ey = fmaf(wz, cx, -(wx * cz)), ez = fmaf(wx, cy, -(wy * cx));
+    dx = fmaf(s1, cx, s2 * ex), dy = fmaf(s1, cy, s2 * ey), dz = fmaf(s1, cz, s2 * ez);
+}
+
+// Its z angle and squared angle.
 template <class R>
-__device__ __forceinline__ void rf_step(const R& q, int f, const Spin& p, float b1sq, State& m, Cache& k) {
-    {
-        if (!(f & HB_SAME_RF_DT)) {
-            k.h1 = expm1x(-0.5f * q.dt * p.r1);
-            k.h2 = expm1x(-0.5f * q.dt * p.r2);
-        }
-        const float dx1 = m.mx * k.h2, dy1 = m.my * k.h2, dz1 = (m.mz - p.pd) * k.h1;
-        const float x1 = m.mx + dx1, y1 = m.my + dy1, z1 = m.mz + dz1;
-        const float wx = p.b1 * q.w_rf_x, wy = p.b1 * q.w_rf_y;
-        const float wz = p.px * q.w_g_x + p.py * q.w_g_y + p.pz * q.w_g_z + (p.db0 * q.w + q.w_b0);
-        float a, b;
-        rot_ab(b1sq * q.w_rf2 + wz * wz, a, b);
-        const float cx = wy * z1 - wz * y1, cy = wz * x1 - wx * z1, cz = wx * y1 - wy * x1;
-        const float ex = wy * cz - wz * cy, ey = wz * cx - wx * cz, ez = wx * cy - wy * cx;
-        const float drx = a * cx + b * ex, dry = a * cy + b * ey, drz = a * cz + b * ez;
-        const float x2 = x1 + drx, y2 = y1 + dry, z2 = z1 + drz;
-        m.mx += dx1 + drx + x2 * k.h2;
-        m.my += dy1 + dry + y2 * k.h2;
-        two_sum(m.mz, m.lz, dz1 + drz + (z2 - p.pd) * k.h1);
-    }
+__device__ __forceinline__ void rf_angles(const R& q, const Spin& p, float b1sq, float& wz, float& phi2) {
+#pragma clang fp contract(off)
+    wz = fmaf(p.pz, q.w_g_z, fmaf(p.py, q.w_g_y, fmaf(p.px, q.w_g_x, fmaf(p.db0, q.w, q.w_b0))));
+    phi2 = fmaf(b1sq, q.w_rf2, wz * wz);
+}
+
+// (k.h1, k.h2 the half relaxations of its dt)
+template <class R>
+__device__ __forceinline__ void rf_step(const R& q, const Spin& p, float b1sq, State& m, const Cache& k) {
+#pragma clang fp contract(off)
+    const float dz1 = (m.mz - p.pd) * k.h1;
+    const float x1 = fmaf(m.mx, k.h2, m.mx), y1 = fmaf(m.my, k.h2, m.my), z1 = m.mz + dz1;
+    const float wx = p.b1 * q.w_rf_x, wy = p.b1 * q.w_rf_y;
+    float wz, phi2, a, b, drx, dry, drz;
+    rf_angles(q, p, b1sq, wz, phi2);
+    rot_ab(phi2, a, b);
+    rotate_less(wx, wy, wz, a, b, x1, y1, z1, drx, dry, drz);
+    const float x2 = x1 + drx, y2 = y1 + dry, z2 = z1 + drz;
+    m.mx += fmaf(x2, k.h2, fmaf(m.mx, k.h2, drx));
+    m.my += fmaf(y2, k.h2, fmaf(m.my, k.h2, dry));
+    two_sum(m.mz, m.lz, fmaf(z2 - p.pd, k.h1, dz1 + drz));
 }
 
 __device__ __forceinline__ void free_step(const hb_segment& q, int f, const Spin& p, const Pos64& r, State& m,
@@ -260,27 +283,61 @@ __device__ __forceinline__ void free_step(const hb_segment& q, int f, const Spin
                 k.e2 = expm1x(-q.dt * p.r2);
             }
         }
-        const float nx = k.c * m.mx - k.s * m.my, ny = k.s * m.mx + k.c * m.my;
-        m.mx = nx + nx * k.e2;
-        m.my = ny + ny * k.e2;
+        precess(k.c, k.s, k.e2, m);
         two_sum(m.mz, m.lz, (m.mz - p.pd) * k.e1);
     }
 }
 
 __device__ __forceinline__ void step(const hb_segment& q, int f, const Spin& p, const Pos64& r, float b1sq, State& m,
                                      Cache& k) {
-    if (f & HB_RF)
-        rf_step(q, f, p, b1sq, m, k);
-    else
+    if (f & HB_RF) {
+        if (!(f & HB_SAME_RF_DT)) half_relax(q.dt, p, k);
+        rf_step(q, p, b1sq, m, k);
+    } else {
         free_step(q, f, p, r, m, k);
+    }
+}
+
+// The 8 records from r on (the caller sees to it that they are inside the table) into the scalar cache, one word of each
+// 64-byte line: the loads go out together and are waited for once, where a walk that reads record by record waits for
+// the L2 at nearly every line. For walks that use most of the 8 (the reverse sweep's blocks: 4,336 records of 64^3 spins
+// with maps and runs 682 -> 552 us); the forward's walk over heads lost by it (96^3: 189 -> 199 ms).
+__device__ __forceinline__ void warm_records(const hb_segment* __restrict__ r) {
+    asm volatile("" ::"s"(r[0].dt), "s"(r[1].dt), "s"(r[2].dt), "s"(r[3].dt), "s"(r[4].dt), "s"(r[5].dt), "s"(r[6].dt),
+                 "s"(r[7].dt), "s"(r[0].flags), "s"(r[1].flags), "s"(r[2].flags), "s"(r[3].flags), "s"(r[4].flags),
+                 "s"(r[5].flags), "s"(r[6].flags), "s"(r[7].flags));
 }
 
 // The same for kernels that keep no float64 position (it is formed per free segment).
 __device__ __forceinline__ void step(const hb_segment& q, int f, const Spin& p, float b1sq, State& m, Cache& k) {
-    if (f & HB_RF)
-        rf_step(q, f, p, b1sq, m, k);
-    else
+    if (f & HB_RF) {
+        if (!(f & HB_SAME_RF_DT)) half_relax(q.dt, p, k);
+        rf_step(q, p, b1sq, m, k);
+    } else {
         free_step(q, f, p, pos64(p), m, k);
+    }
+}
+
+// The RF records at(0) .. at(L - 1) in turn, go(i, record): kTrain of them are loaded while the kTrain before are stepped,
+// as a load costs up to an L2 round trip, more than one step takes. Stepped RF of 32^3 x 4 spins (two waves per SIMD):
+// 60.9 ms one ahead, 54.2 two, 49.9 three, 49.9 four; 44^3 x 4: 257, 246, 237, 229; with gradients, 24^3 x 4: 149, 146.7,
+// 145.5, 146.7 (short launches, where longer code costs instruction fetches).
+constexpr int kTrain = 3;
+
+template <class At, class Go>
+__device__ __forceinline__ void rf_records(int L, At at, Go go) {
+    RfRec cur[kTrain], nxt[kTrain];
+#pragma unroll
+    for (int k = 0; k < kTrain; ++k) cur[k] = load_rf(at(min(k, L - 1)));
+    for (int i = 0; i < L; i += kTrain) {
+#pragma unroll
+        for (int k = 0; k < kTrain; ++k) nxt[k] = load_rf(at(min(i + kTrain + k, L - 1)));
+#pragma unroll
+        for (int k = 0; k < kTrain; ++k) {
+            if (i + k < L) go(i + k, cur[k]);
+            cur[k] = nxt[k];
+        }
+    }
 }
 
 }  // namespace hb

@@ -446,12 +446,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
             }
             if (RF && (f & HB_TRAIN)) {  // RF substeps of a shaped pulse, in a loop of their own (only RF state live)
                 const int L = q.pad[3];
-                RfRec cur = load_rf(&cs.segs[s]);
-                for (int i = 1; i <= L; ++i) {
-                    const RfRec nxt = load_rf(&cs.segs[s + (i < L ? i : 0)]);  // in flight while this one is stepped
-                    rf_step(cur, cur.flags, p, b1sq, m, k);
-                    cur = nxt;
-                }
+                const hb_segment* first = cs.segs + s;
+                rf_records(
+                    L, [&](int i) { return first + i; },
+                    [&](int i, const RfRec& r) {
+                        if (!(r.flags & HB_SAME_RF_DT)) half_relax(first[i].dt, p, k);
+                        rf_step(r, p, b1sq, m, k);
+                    });
                 s += L - 1;
                 continue;
             }
@@ -466,9 +467,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
                 }
                 if (!(f & HB_SAME_RUN)) e1_run = expm1x(-(float)L * q.dt * p.r1);
                 for (int i = 0; i < L; ++i) {
-                    const float nx = k.c * m.mx - k.s * m.my, ny = k.s * m.mx + k.c * m.my;
-                    m.mx = nx + nx * k.e2;
-                    m.my = ny + ny * k.e2;
+                    precess(k.c, k.s, k.e2, m);
                     stg[nb * kStgStride + lane] = m.mx * S.x_scale;
                     stg[(8 + nb) * kStgStride + lane] = m.my * S.x_scale;
                     if (++nb == 8) {
