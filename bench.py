@@ -393,6 +393,9 @@ def recon_timing(run, n_coils: int, shape: tuple, steps: int) -> dict:
                    ** 2).sum(axis=0))
     t_cpu = time.perf_counter() - t0
     err = float(np.abs(img.cpu().double().numpy() - ref).max() / np.abs(ref).max())
+    from blochparty_amd.engines import hip
+
+    passes = len(shape) - hip.load().hb_ifftc_plane_takes(*shape[-2:])  # the last two axes in one
     floor = k.numel() * 8 + ref.size * 4
     gbs = floor / (ms * 1e-3) / 1e9
     log(f"recon (grid, ifft3c, rss) of {n_coils} x {shape}: {ms:.3f} ms on the GPU ({gbs:.0f} GB/s of the floor; "
@@ -401,8 +404,8 @@ def recon_timing(run, n_coils: int, shape: tuple, steps: int) -> dict:
             "cpu_numpy_f64_ms": t_cpu * 1e3, "rel_err_vs_numpy_f64": err,
             "roofline": {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": gbs / HBM_PEAK_GBS, "algorithmic_bytes": floor,
-                         # what the HIP passes move: a read and a write of every value per axis, then the RSS
-                         "traffic": len(shape) * 16 * k.numel() + 8 * k.numel() + 4 * ref.size}}
+                         # what the HIP passes move: a read and a write of every value per pass, then the RSS
+                         "traffic": passes * 16 * k.numel() + 8 * k.numel() + 4 * ref.size}}
 
 
 def downstream_leg(W, driver, n: int, n_coils: int, steps: int) -> dict:

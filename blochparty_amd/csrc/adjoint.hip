@@ -17,7 +17,8 @@
 // segment, and over workgroups in a fixed order by seg_reduce. Nothing depends on the interval length (a multiple of
 // 64) or on scheduling: the gradients are the same bit for bit for any checkpoint_every and every run.
 // Reused pulses (maps) and NUFFT readout runs are one record each, their other segments identity bodies: the replay
-// jumps over them, the reverse skips the 8-blocks inside them (pulse_reverse, nufft_reverse below).
+// jumps over them, the reverse skips the 8-blocks inside them (pulse_reverse, nufft_reverse below). Few spins: intervals in
+// chunks side by side (sweep_kernel below); NUFFT runs with narrow windows: their samples beside the sweep (nufft_back.hip).
 #include "adjoint_device.h"
 #include "nufft_back.h"
 

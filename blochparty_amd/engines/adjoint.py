@@ -8,7 +8,7 @@ of 64 (default about sqrt(segments)), else ``ValueError``.
 
 Forward: the dispatches are exactly the checkpoint intervals, the state before each is kept on the device (hi + lo,
 24 bytes per spin per interval). Backward: dL/dsignal turned by exp(+i psi) (the source of the sweep), then one
-``hb_adjoint_interval`` per interval, last first, and ``hb_seg_reduce`` for the per-segment gradients. Parameter
+``hb_adjoint_chunks`` (few spins) or ``hb_adjoint_runs`` (NUFFT runs) per interval, last first, and ``hb_seg_reduce`` for the per-segment gradients. Parameter
 gradients map as the reference's (adjoint.py:222-261): t1 = 1 / r1 (-dL/dr1 / t1^2), t2 likewise, d/dpsi from the
 signal itself (dsignal/dpsi = -i signal), dL/dm0 = lambda at the start.
 

@@ -1,5 +1,5 @@
 """Gradients through the full variant: a rate bound pool, a scanner's concomitant fields and bound-only RF, through
-``hb_forward_mt`` forward and ``hb_adjoint_full`` in reverse (``csrc/full_adjoint.hip``, ``csrc/full_device.h``).
+``hb_forward_mt`` forward and ``hb_adjoint_full_chunks`` in reverse (``csrc/full_adjoint.hip``, ``csrc/full_device.h``).
 
 Reference: ``_GPUSimulate`` / ``_simulate_grad`` with V = 1 (``src/blochparty/engines/gpu/adjoint.py:55-323``). The
 contract is the reference's: inputs (pos, pd, t1, t2, db0, coils as real pairs (N, C, 2), dt, rf, grad, adc_phase,
@@ -11,7 +11,7 @@ pool's (T1b = 1 / R1b), m0's (with the pool's default Mzb = f PD, through autogr
 segment's dt, rf, grad, b0_offset and RF frequency (so, through ``exchange.rf_frequency``, rf's phase and dt again).
 
 Forward: the dispatches are exactly the checkpoint intervals; the state before each is kept (6 rows, plus Mzb and its
-low part with a bound pool). Backward: dL/dsignal turned by exp(+i psi), then one ``hb_adjoint_full`` per interval,
+low part with a bound pool). Backward: dL/dsignal turned by exp(+i psi), then one ``hb_adjoint_full_chunks`` per interval,
 last first (one sweep per tile of 16 coils, the sweep being linear in its sources), and ``hb_seg_reduce`` for the
 per-segment gradients.
 """
@@ -158,7 +158,7 @@ class FullSimulate(torch.autograd.Function):
 
 def run_backward(case: driver.DeviceCase, ckpts: list, every: int, h: torch.Tensor, lam: torch.Tensor,
                  sens: torch.Tensor, nc: int, need_seg: bool, need_coil: bool):
-    """``hb_adjoint_full`` over every interval of ``case`` (aligned dispatches, forward run with ``keep``): ``h``
+    """``hb_adjoint_full_chunks`` over every interval of ``case`` (aligned dispatches, forward run with ``keep``): ``h``
     (n_adc, nc, 2) dL/dsignal turned by exp(+i psi), ``lam`` (4, n_pad) dL/d(Mx, My, Mz, Mzb) at the end (it ends as
     dL/dm0), ``sens`` (2 nc, n_pad). Returns gs (N_GRADS, n_pad), gc (2 nc, n_pad), seg (S, 8) float64 and lam. More
     than PASS_COILS coils: one sweep per tile of PASS_COILS coils, dL/dm at the end entering the first only."""

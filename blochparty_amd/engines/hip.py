@@ -106,6 +106,7 @@ SIGNATURES = {
     "hb_sur_first_quats": [_P, _P, _I, _P, _V],
     "hb_mlp_train_steps": [_P, _P, _P, _I, _I, _P, _I, _I, ctypes.c_float, ctypes.c_float, _V],
     "hb_surrogate_maps": [ctypes.POINTER(HbCase), _P, _P, _P, _P, _V],
+    "hb_ifftc_plane": [_P, _P, ctypes.c_int64, _I, _I, _V],
     "hb_ifftc_axis": [_P, _P, ctypes.c_int64, _I, ctypes.c_int64, _V],
     "hb_rss": [_P, _I, ctypes.c_int64, _P, _V],
 }
@@ -125,6 +126,8 @@ def load() -> ctypes.CDLL:
         lib.hb_abi_version.restype = ctypes.c_int
         lib.hb_mlp_workspace.restype = ctypes.c_int64
         lib.hb_mlp_workspace.argtypes = [ctypes.c_int32]
+        lib.hb_ifftc_plane_takes.restype = ctypes.c_int32
+        lib.hb_ifftc_plane_takes.argtypes = [ctypes.c_int64] * 2
         lib.hb_adjoint_runs_takes.restype = ctypes.c_int32
         lib.hb_adjoint_runs_takes.argtypes = [ctypes.c_int32] * 2
         lib.hb_adjoint_chunks_workspace.restype = ctypes.c_int64

@@ -4,7 +4,7 @@ and bound-only RF, through ``hb_forward_mt`` (``csrc/mt.hip``, ``include/blochpa
 Reference: the V = 1 / ``_full`` variant of the reference's GPU engine (``engines/gpu/driver.py:435-520`` with
 ``shaders/common.metal:113-208, 563-601``), the physics of ``exchange.py`` and ``fields.py`` (restated in
 ``blochparty_amd/exchange.py`` and ``blochparty_amd/fields.py``); gradients through ``hb_adjoint_full``
-(``engines/full_adjoint.py``). The case keeps the plain records (no runs, merged
+(``engines/full_adjoint.py``). The case keeps records marked with readout runs and trains (no merged
 runs, reused pulses or NUFFT runs), the sensitivities in rows (2 C, n_pad) and, as present, the bound pool's per-spin
 parameters (f, k, R1b, T2b, dw), its Mzb with a low part, every segment's RF frequency and the super-Lorentzian's
 ln F table, and the spins' concomitant coefficients (7, n_pad); the signal goes through ``hb_signal_reduce`` as the

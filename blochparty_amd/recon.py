@@ -46,8 +46,8 @@ def _pow2(n: int) -> bool:
 
 def ifftnc(k: Tensor, ndim: int) -> Tensor:
     """Centred inverse DFT over the last ``ndim`` axes, backward normalisation: a spin of magnetization m at a
-    voxel centre gives that voxel the value m. complex64 on the GPU with power-of-two axes (2..4096): one HIP pass
-    per axis (``hb_ifftc_axis``), the first out of place; otherwise torch's FFT on the tensor's device."""
+    voxel centre gives that voxel the value m. complex64 on the GPU with power-of-two axes (2..4096): the last two
+    in one HIP pass where a plane fits in LDS (``hb_ifftc_plane``), else one pass per axis (``hb_ifftc_axis``); otherwise torch's FFT on the tensor's device."""
     axes = tuple(range(-ndim, 0))
     if _on_hip(k, torch.complex64) and 1 <= ndim <= k.ndim and all(_pow2(k.shape[a]) for a in axes):
         from .engines import hip
@@ -56,9 +56,12 @@ def ifftnc(k: Tensor, ndim: int) -> Tensor:
         src = k.contiguous()
         out = torch.empty_like(src)
         shape = list(src.shape)
-        for i, a in enumerate(range(src.ndim - ndim, src.ndim)):
+        plane = ndim >= 2 and hip.load().hb_ifftc_plane_takes(shape[-2], shape[-1])
+        for i, a in enumerate(range(src.ndim - ndim, src.ndim - (2 if plane else 0))):
             lib.ifftc_axis((src if i == 0 else out).data_ptr(), out.data_ptr(), math.prod(shape[:a]), shape[a],
                            math.prod(shape[a + 1 :]))
+        if plane:
+            lib.ifftc_plane((src if ndim == 2 else out).data_ptr(), out.data_ptr(), math.prod(shape[:-2]), *shape[-2:])
         return out
     return torch.fft.fftshift(torch.fft.ifftn(torch.fft.ifftshift(k, dim=axes), dim=axes), dim=axes)
 

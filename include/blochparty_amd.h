@@ -357,6 +357,11 @@ int hb_seg_reduce(const float* gseg, int32_t n_blocks, int32_t k_max, int32_t s0
  * hb_rss: out[v] = sqrt(sum_c |x[c][v]|^2) for x (n_coils, per_coil) complex64, the coils summed in order in float32
  * (recon.py:36-37 rss over dim 0). */
 int hb_ifftc_axis(const float* src, float* dst, int64_t outer, int32_t L, int64_t inner, void* stream);
+/* The same along both of the last two axes of (planes, A, B) values in one pass (dst may be src); taken where
+ * hb_ifftc_plane_takes(A, B) says so (powers of two of 16 or more, 1,024 to 16,384 values a plane), else
+ * hipErrorInvalidValue. */
+int32_t hb_ifftc_plane_takes(int64_t A, int64_t B);
+int hb_ifftc_plane(const float* src, float* dst, int64_t planes, int32_t A, int32_t B, void* stream);
 int hb_rss(const float* x, int32_t n_coils, int64_t per_coil, float* out, void* stream);
 
 /* Name of a return code. */
