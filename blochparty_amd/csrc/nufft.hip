@@ -84,47 +84,67 @@ __global__ __launch_bounds__(kGridBlock) void nufft_grid_kernel(const float* __r
     }
 }
 
+constexpr int kSigFill = 256;   // workgroups below which a workgroup takes one sample (one per CU)
 constexpr int kSigParts = 32;  // lanes per coil, each summing the cells u = p, p + 32, ...
 
-// One workgroup per (sample i, slot r): lanes (coil c of a group of 8, part p) sum the DFT over their cells and
-// every decay term, weighted; the 32 parts are added in order; then the receiver phase is taken off.
+// One workgroup per (K samples, slot r): lanes (coil c of a group of 8, part p) sum the DFT over their cells and every
+// decay term, weighted; the 32 parts are added in order; then the receiver phase is taken off. Every workgroup reads its
+// slot's whole grid (147 KB at 96^3 and 16 coils) from the L2, which bounds one sample a workgroup: K = 4 read it a
+// quarter as often, each sample summed as before. Where the samples make too few workgroups, K = 1. 9,216 runs of 96
+// samples, 16 coils: 9.9 -> 7.4 ms.
+template <int K>
 __global__ __launch_bounds__(256) void nufft_signal_kernel(const double* __restrict__ grid,
-                                                           const int* __restrict__ run_of,
-                                                           const int* __restrict__ row_of, int n, int ng, int terms,
-                                                           int vals, int n_coils, const double* __restrict__ tw,
-                                                           const double* __restrict__ lw,
-                                                           const double* __restrict__ psi, double* __restrict__ sig) {
-    __shared__ double red[2][256];
-    const int i = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
+                                                            const int* __restrict__ run_of,
+                                                            const int* __restrict__ row_of, int n, int ng, int terms,
+                                                            int vals, int n_coils, const double* __restrict__ tw,
+                                                            const double* __restrict__ lw,
+                                                            const double* __restrict__ psi, double* __restrict__ sig) {
+    __shared__ double red[K][2][256];
+    const int i0 = blockIdx.x * K, r = blockIdx.y, tid = threadIdx.x;
     const int cl = tid % 8, p = tid / 8;
-    const double* twi = tw + (size_t)i * ng * 2;
-    const int row = row_of[run_of[r]] + i;
+    const double* twi[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) twi[k] = tw + (size_t)min(i0 + k, n - 1) * ng * 2;
+    // the lane that finishes sample i0 + tid / 8 of coil tid % 8
+    const int fin = tid / 8;
+    const bool last = fin < K && i0 + fin < n;
+    const int row = row_of[run_of[r]] + i0 + (last ? fin : 0);
     double sp, cp;
     sincos(psi[row], &sp, &cp);
     for (int c0 = 0; c0 < n_coils; c0 += 8) {
         const int c = c0 + cl;
-        double re = 0.0, im = 0.0;
+        double re[K], im[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) re[k] = im[k] = 0.0;
         if (c < n_coils) {
             for (int m = 0; m < terms; ++m) {
                 const double* g = grid + ((size_t)(r * terms + m) * ng) * vals + 2 * c;
-                double fr = 0.0, fi = 0.0;
+                double fr[K], fi[K];
+#pragma unroll
+                for (int k = 0; k < K; ++k) fr[k] = fi[k] = 0.0;
                 for (int u = p; u < ng; u += kSigParts) {
                     const double gr = g[(size_t)u * vals], gi = g[(size_t)u * vals + 1];
-                    const double tr = twi[2 * u], ti = twi[2 * u + 1];
-                    fr += gr * tr - gi * ti;
-                    fi += gr * ti + gi * tr;
+#pragma unroll
+                    for (int k = 0; k < K; ++k) {
+                        const double tr = twi[k][2 * u], ti = twi[k][2 * u + 1];
+                        fr[k] += gr * tr - gi * ti;
+                        fi[k] += gr * ti + gi * tr;
+                    }
                 }
-                const double wgt = lw[(size_t)m * n + i];
-                re += wgt * fr;
-                im += wgt * fi;
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const double wgt = lw[(size_t)m * n + min(i0 + k, n - 1)];
+                    re[k] += wgt * fr[k];
+                    im[k] += wgt * fi[k];
+                }
             }
         }
-        red[0][tid] = re;
-        red[1][tid] = im;
+#pragma unroll
+        for (int k = 0; k < K; ++k) red[k][0][tid] = re[k], red[k][1][tid] = im[k];
         __syncthreads();
-        if (tid < 8 && c < n_coils) {
+        if (last && c < n_coils) {
             double sr = 0.0, si = 0.0;
-            for (int q = 0; q < kSigParts; ++q) sr += red[0][q * 8 + tid], si += red[1][q * 8 + tid];
+            for (int q = 0; q < kSigParts; ++q) sr += red[fin][0][q * 8 + cl], si += red[fin][1][q * 8 + cl];
             double* out = sig + ((size_t)row * n_coils + c) * 2;
             out[0] = sr * cp + si * sp;
             out[1] = si * cp - sr * sp;
@@ -191,7 +211,9 @@ extern "C" int hb_nufft_signal(const double* grid, int32_t n_slots, const int32_
         terms > HB_NUFFT_MAX_TERMS || n_tiles < 1 || n_coils < 1 || n_coils > 8 * n_tiles)
         return hipErrorInvalidValue;
     if (n_slots == 0) return hipSuccess;
-    hipLaunchKernelGGL(hb::nufft_signal_kernel, dim3(n, n_slots), dim3(256), 0, (hipStream_t)stream, grid, run_of,
+    const bool four = (int64_t)((n + 3) / 4) * n_slots >= hb::kSigFill;
+    auto kernel = four ? hb::nufft_signal_kernel<4> : hb::nufft_signal_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3(four ? (n + 3) / 4 : n, n_slots), dim3(256), 0, (hipStream_t)stream, grid, run_of,
                        row_of, n, ng, terms, 16 * n_tiles, n_coils, tw, lw, psi, sig);
     return hipGetLastError();
 }
