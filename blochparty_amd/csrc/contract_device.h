@@ -39,7 +39,8 @@ constexpr int kMaxTiles = 16;   // 128 coils: LDS = 4 x 16 x 68 + 4 x 8 x 256 fl
 __host__ __device__ constexpr int lds_floats(int nt) { return kWaves * kStgFloats + 2 * kWaves * 8 * 16 * nt; }
 
 // Float16's smallest step is 2^-24, so the low part of a value scaled to 2^-6 of the bound would keep it to 2^-19 only:
-// the operands are lifted by this power of two (undone exactly by out_scale), which leaves 2^8 above the bound.
+// the operands are lifted by this power of two (undone exactly by out_scale), which leaves 2^8 above the bound (for an
+// operand that is one such value, not a product of two).
 constexpr float kLift = 256.0f;
 
 // x of lane (jj + 8) mod 16 of this lane's row of 16 (DPP row_ror:8).

@@ -116,6 +116,11 @@ __device__ __forceinline__ void nufft_run(const hb_case& cs, const hb_nufft& nu,
 // round of workgroups. Only for dispatches without stepped RF: the RF loop is faster with five waves than this is with
 // four. Reading the next record ahead costs 32 scalar moves a record and measured 8 % slower.
 constexpr int kCols = 32;
+// S_c c is an operand itself: with S lifted by kLift and c by this, a product of values at their bounds (|Re S|, |Im S|,
+// |M| scaled to 1) is at most sqrt(2) 2^14 = 23,170 of float16's 65,504, and its pair holds it to 2^-39 of the bound
+// (both lifted by kLift it would reach 92,681). The signal's error against 64 bits is 1.6e-6 with either lift, at 64^3 x 4
+// spins and 8 coils and at 96^3 and 16.
+constexpr float kProductLift = 64.0f;
 constexpr float kWeightLift = 1024.0f;  // the weights (<= 1) in float16's range, as kLift
 constexpr int kColTiles = kCols / 16;
 
@@ -135,7 +140,7 @@ template <int NT>
 struct Spread {
     float a[NT][16];                         // value jj of spins 16 g + u: Re S_0, Im S_0, Re S_1, ... scaled
     h8 wh[kColTiles][2], wl[kColTiles][2];   // the weights of column 16 tile + jj, spins 16 g + u (u < 8, u >= 8)
-    float cp, sp;                            // cos, sin of the start's phase factor times the values' scale
+    float cp, sp;                            // cos, sin of the start's phase factor times the case's x_scale, lifted
     int kind, cols;                          // the kind they belong to (-1: none yet), its window's columns
 
     // sens_scale: Sens::scales' (lifted)
@@ -322,7 +327,7 @@ __device__ __forceinline__ void spread_run(const Spread<NT>& W, const hb_nufft& 
 #pragma unroll
         for (int w = 1; w < kWaves; ++w) s += reinterpret_cast<const f4*>(buf + w * (kCols * vals))[tid];
         float* out = nu.part + ((size_t)q.pad[1] * gridDim.x + blockIdx.x) * nu.cols * vals;
-        reinterpret_cast<f4*>(out)[tid] = s * (out_scale * (1.0f / kWeightLift));
+        reinterpret_cast<f4*>(out)[tid] = s * (out_scale * (kLift / kProductLift / kWeightLift));
     }
     if (!(q.flags & HB_SAME_RUN)) e1_run = expm1x(-((float)q.pad[3] * q.dt) * p.r1);
     double cyc = 0.0;
@@ -426,7 +431,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
         if constexpr (MAT) {
             const hb_segment q = cs.segs[s];
             if ((q.flags & HB_NUFFT) && q.pad[2] != W.kind)
-                make_weights<NS>(W, nu, q, p, r64, wred, S.x_scale, lane, wave);
+                make_weights<NS>(W, nu, q, p, r64, wred, S.x_scale * (kProductLift / kLift), lane, wave);
         }
         for (; s < s1; ++s) {
             const hb_segment q = cs.segs[s];

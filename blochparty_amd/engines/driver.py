@@ -384,7 +384,7 @@ class DeviceCase:
     nu: dict | None = None  # NUFFT readouts: plan, device tables, work buffers, per-dispatch runs
     perm: np.ndarray | None = None  # the spins' order on the device (sorted for NUFFT readouts), or None
     rf_free: list[bool] = field(default_factory=list)  # per dispatch: no segment stepped as RF (hb_case.rf_free)
-    sens_scale: float = 1.0  # powers of two: |sensitivity| sens_scale <= 1, |M| x_scale <= 1 (hb_case)
+    sens_scale: float = 1.0  # powers of two: |Re S|, |Im S| sens_scale <= 1, |M| x_scale <= 1 (hb_case)
     x_scale: float = 1.0
 
     def struct(self) -> hip.HbCase:

@@ -1,0 +1,72 @@
+"""NUFFT runs spread as one matrix product with the largest operands the scales allow, GPU: full transverse
+magnetization (90 degree pulses; m_init along x without RF, a run as the first record) under coils whose parts sit at a
+power of two or just below one (modulus up to sqrt(2) after scaling).
+
+Tolerance: against the oracle the NUFFT's own bound, 1e-4 of the largest sample at (6, 3); against the staged spreading
+2e-6 (a few 2^-24 of each term, as the spreading's other tests)."""
+
+import numpy as np
+import pytest
+import torch
+
+import blochparty_amd as bp
+from blochparty_amd.engines import driver
+from cases import rel
+from oracle import core
+from test_gpu_spread import scan
+
+f64 = torch.float64
+
+
+def spins(n, t1=(0.5, 2.0), t2=(0.3, 0.5)):
+    g = torch.Generator().manual_seed(n)
+    u = lambda lo, hi: lo + (hi - lo) * torch.rand(n, generator=g, dtype=f64)
+    return bp.Phantom(torch.stack([0.006 + u(0, 0.012) * -(-n // 256), u(-2e-4, 2e-4), u(-2e-4, 2e-4)], 1),
+                      torch.ones(n, dtype=f64), u(*t1), u(*t2), u(-5.0, 5.0))
+
+
+def both_routes(ph, seq, coils, m_init=None):
+    case = driver.prepare_case(ph, seq, coils, m_init, reuse=True, nufft=(6, 3))
+    assert case.nu is not None and all(case.rf_free) and case.nu["cols"] <= 32
+    driver.run_forward(case)
+    spread = driver.read_result(case)
+    case.rf_free = [False] * len(case.rf_free)  # always correct: the general variant
+    driver.run_forward(case)
+    return spread, driver.read_result(case)
+
+
+def check(ph, seq, coils, m_init=None):
+    spread, staged = both_routes(ph, seq, coils, m_init)
+    c = torch.ones(len(ph), 1, dtype=torch.complex128) if coils is None else coils
+    ref, _ = core.simulate(ph, seq, c, m_init=m_init)
+    e = rel(spread.signal.to(torch.complex128), ref), rel(spread.signal, staged.signal)
+    print(f"oracle {e[0]:.1e}, staged {e[1]:.1e}", flush=True)
+    assert bool(torch.isfinite(torch.view_as_real(spread.signal)).all())
+    assert e[0] < 1e-4 and e[1] < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("coil", [None, 1.0, 1 + 1j, 0.9 + 0.9j, -0.999 - 0.999j, 1.01 + 0.5j])
+@pytest.mark.parametrize("coils", [1, 9])
+def test_quarter_turn(gpu, coil, coils):
+    """90 degree pulses (two substeps of 10 us)."""
+    if coil is None and coils > 1:
+        pytest.skip("no coils is one coil")
+    n = 500
+    seq = scan(24, 2, 1, 5, spoil=True)
+    amp = 1 / (4 * 10e-6 * 3)  # 2 pi (a + 2 a) 10 us = pi / 2
+    seq = bp.Sequence(seq.dt, seq.rf * (amp / 2000.0), seq.grad, seq.adc_phase, seq.is_rf, seq.adc, seq.spoil)
+    check(spins(n), seq, None if coil is None else torch.full((n, coils), complex(coil), dtype=torch.complex128))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scale", [1.0, 0.5, 1e4])
+def test_run_first(gpu, scale):
+    """No RF: the run is the first record and the spins start transverse, |M| = |m_init| the case's bound."""
+    n, N = 300, 32
+    t = lambda v: torch.tensor(np.array(v), dtype=f64)
+    seq = bp.Sequence(t([10e-6] * N + [1e-3]), t([(0.0, 0.0)] * (N + 1)), t([(40.0 / N / 10e-6, 0, 0)] * N + [(0, 0, 0)]),
+                      t([0.0] * (N + 1)), [False] * (N + 1), [True] * N + [False], [False] * (N + 1))
+    m0 = torch.zeros(n, 3, dtype=f64)
+    m0[:, 0] = scale
+    check(spins(n), seq, torch.full((n, 1), 1 + 1j, dtype=torch.complex128), m0)
