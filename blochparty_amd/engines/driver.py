@@ -337,6 +337,21 @@ def pow2_scale(bound: float) -> float:
     return math.ldexp(1.0, -min(100, max(-100, math.ceil(math.log2(bound)))))
 
 
+def magnetization_bound(pd: torch.Tensor, t1: torch.Tensor, t2: torch.Tensor, m0: torch.Tensor, total: float) -> float:
+    """The largest |M| that any sequence of ``total`` seconds reaches from |M| = ``m0`` (all (N,) float64). Rotations
+    keep |M|; relaxation changes its square at 2 (R1 Mz (PD - Mz) - R2 |Mxy|^2) per second. For T2 <= 2 T1 that is
+    negative beyond PD, so the bound is max(PD, m0). Beyond 2 T1 it is at most R1 PD^2 / 2, and negative beyond
+    PD R1 / (2 sqrt(R2 (R1 - R2))), the steady state of pulses that hold Mz at its best."""
+    if not len(pd):
+        return 0.0
+    pd, r1, r2 = pd.abs(), 1 / t1, 1 / t2
+    start = torch.maximum(pd, m0)
+    grown = (start * start + pd * pd * (r1 * (0.5 * total))).sqrt()
+    steady = torch.where(r2 > 0, 0.5 * pd * r1 / (r2 * (r1 - r2)).clamp_min(1e-300).sqrt(), math.inf)
+    long_t2 = torch.maximum(start, torch.minimum(grown, steady))
+    return float(torch.where(r2 < 0.5 * r1, long_t2, start).max())
+
+
 def sens_operand(coils: torch.Tensor, n: int, n_pad: int, n_tiles: int) -> torch.Tensor:
     """(N, C) complex sensitivities in the matrix-core A order: (n_pad / 64, tiles, 16 steps, 64 lanes), where lane
     l = 16 g + i of step u holds row i (Re S_0, Im S_0, Re S_1, Im S_1, ... of the tile) at spin 16 g + u of the
@@ -530,16 +545,16 @@ def prepare_case(phantom: Phantom, seq: Sequence, coils=None, m_init=None, *, ch
         for a, _ in occ:
             covered[a : a + k] = True
     rf_cum = np.concatenate([[0], np.cumsum(flag_array(seq.is_rf) & ~covered)])
-    # the coil contraction's scales: |M| <= max(PD, |m_init|) along any sequence (rotations keep |M|, relaxation
-    # moves it toward (0, 0, PD))
+    # the coil contraction's scales
     if full:  # its kernels read the sensitivities in rows (mt.attach)
         sens_a, largest = torch.zeros(0, dtype=torch.float32), torch.view_as_real(coils.detach().to(torch.complex128))
     else:
         sens_a = largest = sens_operand(coils, n, n_pad, n_tiles)
     sens_scale = pow2_scale(float(largest.abs().max()) if largest.numel() else 0.0)
-    x_scale = pow2_scale(max(float(phantom.pd.detach().abs().max()) if n else 0.0,
-                             float((m64[0] * m64[0] + m64[1] * m64[1] + m64[2] * m64[2]).max().sqrt()) if n
-                             else 0.0))
+    host = lambda t: t.detach().double().cpu()
+    x_scale = pow2_scale(magnetization_bound(host(phantom.pd), host(phantom.t1), host(phantom.t2),
+                                             (m64[0] * m64[0] + m64[1] * m64[1] + m64[2] * m64[2]).sqrt(),
+                                             float(host(seq.dt).sum())))
     psi_rows = np.remainder(seq.adc_phase.detach().double().cpu().numpy()[flag_array(seq.adc)],
                             2 * math.pi)
     max_rows = max(rows + [0])

@@ -83,8 +83,9 @@ typedef struct hb_case {
      * applied as a map), so the kernel may leave the RF step out; 0 is always correct. Ignored elsewhere. */
     int32_t rf_free;
     /* hb_forward: powers of two (0 reads as 1) with |Re S| * sens_scale <= 1, |Im S| * sens_scale <= 1 for every
-     * sensitivity S and |M| * x_scale <= 1 for every magnetization the case can reach (|M| <= max(PD, |m_init|)): the coil contraction works on these scaled values (as float16 hi +
-     * lo pairs for up to 16 coils; |M| may pass the bound 2.8 times before the largest product of a sensitivity and a
+     * sensitivity S and |M| * x_scale <= 1 for every magnetization the case can reach (|M| <= max(PD, |m_init|) where
+     * T2 <= 2 T1; beyond that it can grow above PD): the coil contraction works on these scaled values (as float16 hi +
+     * lo pairs for up to 16 coils; |M| may pass its bound 2.8 times before the largest product of a sensitivity and a
      * magnetization leaves float16's range) and undoes the scales exactly. */
     float sens_scale;
     float x_scale;

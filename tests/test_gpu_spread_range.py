@@ -1,9 +1,11 @@
 """NUFFT runs spread as one matrix product with the largest operands the scales allow, GPU: full transverse
 magnetization (90 degree pulses; m_init along x without RF, a run as the first record) under coils whose parts sit at a
-power of two or just below one (modulus up to sqrt(2) after scaling).
+power of two or just below one (modulus up to sqrt(2) after scaling), and magnetization above PD (T2 far above 2 T1).
 
 Tolerance: against the oracle the NUFFT's own bound, 1e-4 of the largest sample at (6, 3); against the staged spreading
 2e-6 (a few 2^-24 of each term, as the spreading's other tests)."""
+
+import math
 
 import numpy as np
 import pytest
@@ -70,3 +72,56 @@ def test_run_first(gpu, scale):
     m0 = torch.zeros(n, 3, dtype=f64)
     m0[:, 0] = scale
     check(spins(n), seq, torch.full((n, 1), 1 + 1j, dtype=torch.complex128), m0)
+
+
+def balanced(reps, n=16, t=1.9e-3):
+    """Turns by pi - 0.25 about +x and -x, a run between, every gradient refocused: magnetization near +-y is turned onto
+    its mirror image and gains along z in between, so with T2 >> T1 it grows far above PD."""
+    dt, rf, g, is_rf, adc = [], [], [], [], []
+    amp, gx = (math.pi - 0.25) / (2 * math.pi * 3 * 10e-6), 40.0 / n / 10e-6
+    for i in range(reps):
+        parts = [(10e-6, (1 + k) * (-amp if i % 2 else amp), 0.0, False) for k in range(2)]
+        back = [(t, 0.0, -gx * n * 10e-6 / 2 / t, False)]
+        parts += back + [(10e-6, 0.0, gx, True)] * n + back
+        for d, w, x, a in parts:
+            dt.append(d), rf.append((w, 0.0)), g.append((x, 0.0, 0.0)), is_rf.append(w != 0.0), adc.append(a)
+    v = lambda x: torch.tensor(np.array(x, dtype=np.float64))
+    return bp.Sequence(v(dt), v(rf), v(g), v([0.0] * len(dt)), is_rf, adc, [False] * len(dt))
+
+
+@pytest.mark.gpu
+def test_magnetization_above_pd(gpu):
+    """T2 = 10^6 T1: balanced pulses take the magnetization above four times PD."""
+    n = 256
+    ph = spins(n, t1=(0.05, 0.06), t2=(5e4, 6e4))
+    ph = bp.Phantom(ph.pos, ph.pd, ph.t1, ph.t2, torch.zeros(n, dtype=f64))
+    m0 = torch.tensor([[0.0, -math.cos(0.125), math.sin(0.125)]], dtype=f64).expand(n, 3)
+    seq, coils = balanced(500), torch.full((n, 1), 1 + 1j, dtype=torch.complex128)
+    _, m = core.simulate(ph, seq, coils, m_init=m0)
+    assert float(m.norm(dim=1).max()) > 4.0
+    check(ph, seq, coils, m0)
+
+
+def test_bound_of_the_magnetization():
+    """driver.magnetization_bound: PD for T2 <= 2 T1; above it, no sequence of rotations and relaxation passes it
+    (random ones, and the climb along Mz = PD R1 / (2 (R1 - R2)), in float64)."""
+    rng = np.random.default_rng(0)
+    one = lambda v: torch.tensor([v], dtype=f64)
+    for r in (0.05, 1.0, 2.0):
+        assert driver.magnetization_bound(one(0.8), one(1.0), one(r), one(0.5), 100.0) == 0.8
+        assert driver.magnetization_bound(one(0.8), one(1.0), one(r), one(3.0), 100.0) == 3.0
+    assert driver.magnetization_bound(one(0.8), one(1.0), one(math.inf), one(0.8), 0.0) == pytest.approx(0.8)
+    assert driver.magnetization_bound(one(-0.8), one(math.inf), one(math.inf), one(0.0), 5.0) == 0.8
+    assert driver.magnetization_bound(*(torch.zeros(0, dtype=f64),) * 4, 5.0) == 0.0
+    for t2, total in ((3.0, 50.0), (40.0, 200.0), (1e4, 60.0), (math.inf, 30.0)):
+        bound = driver.magnetization_bound(one(1.0), one(1.0), one(t2), one(1.0), total)
+        steps = 20000
+        h, rho, best = total / steps, 1.0, 1.0
+        r2 = 1 / t2
+        for k in range(steps):  # turned to the best Mz before each step (or a random one)
+            z = min(rho, 1 / (2 * (1 - r2))) if rng.random() < 0.98 else rho * rng.uniform(-1, 1)
+            xy = math.sqrt(max(rho * rho - z * z, 0.0)) * math.exp(-h * r2)
+            z = 1 + (z - 1) * math.exp(-h)
+            rho = math.hypot(xy, z)
+            best = max(best, rho)
+        assert best <= bound * (1 + 1e-9) and best > 0.7 * bound, (t2, best, bound)
