@@ -12,12 +12,15 @@
 // A run is three matrix products per wave of 64 spins: with the weights w = psi e^{-R2 tau} on the workgroup's window of at
 // most kColsB columns (cell x term) and their derivative along z, both the same for every run of a kind and so formed
 // once and held as matrix-core operands (rows: spins), against the window's G (columns: Re, Im of the coils) and tau G:
-// Y = w G, R = w (tau G), X = (dw/dz) G on v_mfma_f32_16x16x32_f16, three products of float16 hi and lo parts each (G
-// scaled into the window's range by a power of two), 36 instructions; each lane gets its spin's values back through LDS
-// (one wave's block, no barrier) and contracts them with its sensitivities. That is about 350 VALU instructions a run;
-// taken column by column in the sweep it was 2,300, at two waves per SIMD. Measured at 64^3 spins, 8 coils, 16 runs of 64
-// samples an interval: the sweep 1,086 -> 682 us, with 120 us here and 109 us for the replay on its own; the whole
-// backward of 4,096 runs 341 -> 295 ms.
+// Y = w G, R = w (tau G), X = (dw/dz) G on v_mfma_f32_16x16x32_f16, three products of float16 hi and lo parts each, 36
+// instructions; each lane gets its spin's values back through LDS (one wave's block, no barrier) and contracts them with
+// its sensitivities. G is scaled by a power of two per column (a coil's Re or Im, by its largest value in the window), so
+// that the pairs hold each coil's values to 2^-24, or to 2^-33 of that coil's largest, whatever the others' residuals: with
+// one scale for all coils, a coil with a residual 2^-17 of the largest had gradients 2.6e-5 off and one with 2^-34 of it
+// 80 %. (In float32 on v_mfma_f32_16x16x4_f32 the products take four times as long: the backward at 64^3 264.8 -> 273.5 ms.)
+// That is about 350 VALU instructions a run; taken column by column in the sweep it was 2,300, at two waves per SIMD.
+// Measured at 64^3 spins, 8 coils, 16 runs of 64 samples an interval: the sweep 1,086 -> 682 us, with 120 us here and 109 us
+// for the replay on its own; the whole backward of 4,096 runs 341 -> 295 ms.
 #include "nufft_back.h"
 
 #include "bloch_device.h"
@@ -135,24 +138,27 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NC <= 8 
             const float* Gr = G + (size_t)r * terms * ng * (2 * NC);
             // this lane's part of the window: columns 8 g .. 8 g + 7, values jj (and 16 + jj)
             float x[CT][8];
-            float big = 0.0f;
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
                 for (int i = 0; i < 8; ++i) {
                     const int v = 16 * ct + jj;
                     x[ct][i] = at[i] >= 0 && v < 2 * NC ? Gr[at[i] + v] : 0.0f;
-                    big = fmaxf(big, fabsf(x[ct][i]));
                 }
-#pragma unroll
-            for (int off = 1; off < 64; off <<= 1) big = fmaxf(big, __shfl_xor(big, off, 64));
-            // the power of two that brings the window's largest value to [1/2, 1) times the lift
-            const int ex = (__float_as_int(big) >> 23) & 255;  // 0: zero or subnormal, 255: not finite
-            const int up = min(max(253 - ex, 1), 245);
-            const float scale = __int_as_float(up << 23) * kLiftG, unscale = __int_as_float((254 - up) << 23) / kLiftG;
             h8 bh[CT], bl[CT], th[CT], tl[CT];
+            float unscale[CT];
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
+                // the power of two that brings the column's largest value to [1/2, 1) times the lift
+                float big = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) big = fmaxf(big, fabsf(x[ct][i]));
+                big = fmaxf(big, __shfl_xor(big, 16, 64));
+                big = fmaxf(big, __shfl_xor(big, 32, 64));
+                const int ex = (__float_as_int(big) >> 23) & 255;  // 0: zero or subnormal, 255: not finite
+                const int up = min(max(253 - ex, 1), 245);
+                const float scale = __int_as_float(up << 23) * kLiftG;
+                unscale[ct] = __int_as_float((254 - up) << 23) / kLiftG;
                 float y[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) x[ct][i] *= scale, y[i] = x[ct][i] * tau_w[i];
@@ -165,6 +171,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NC <= 8 
 #pragma unroll
             for (int set = 0; set < 3; ++set) {
                 // D[spin 16 t + 4 g + r][value] of the set into the wave's block, then this lane's spin's values
+                float s[CT];  // undoes the column's scale and the lifts
+#pragma unroll
+                for (int ct = 0; ct < CT; ++ct)
+                    s[ct] = unscale[ct] * (set == 0 ? 1.0f / kLiftW : set == 1 ? -tau_max / kLiftW : 1.0f / kLiftD);
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
@@ -176,10 +186,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NC <= 8 
                         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, vl, acc, 0, 0, 0);
                         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, vh, acc, 0, 0, 0);
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) mine[(16 * t + 4 * g + i) * kStrideB + 16 * ct + jj] = acc[i];
+                        for (int i = 0; i < 4; ++i) mine[(16 * t + 4 * g + i) * kStrideB + 16 * ct + jj] = acc[i] * s[ct];
                     }
                 fence_wave();
-                const float s = unscale * (set == 0 ? 1.0f / kLiftW : set == 1 ? -tau_max / kLiftW : 1.0f / kLiftD);
                 float yr_s = 0.0f, yi_s = 0.0f;
                 constexpr int kQuads = (2 * NC + 3) / 4;
 #pragma unroll
@@ -189,7 +198,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NC <= 8 
                     for (int e = 0; e < 2; ++e) {
                         const int c = 2 * v + e;
                         if (c < NC) {
-                            const float yr = y[2 * e] * s, yi = y[2 * e + 1] * s;
+                            const float yr = y[2 * e], yi = y[2 * e + 1];
                             yr_s += sr[c] * yr + si[c] * yi;  // conj(S_c) Y_c
                             yi_s += sr[c] * yi - si[c] * yr;
                             if (set == 0) {  // coil gradients conj(m0) A_c
