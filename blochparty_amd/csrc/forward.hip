@@ -335,9 +335,9 @@ __device__ __forceinline__ void spread_run(const Spread<NT>& W, const hb_nufft& 
     run_jump(q, p, cyc, e1_run, m);
 }
 
-// NT: coil tiles (0: any, the sensitivities read from memory per flush); NUT: NUFFT runs: 0 none, 1 by spread_run (NT 1 or
-// 2, windows of at most kCols columns), 4 and 8 by nufft_run with up to NUT decay terms (their weights in registers); RF: RF segments are stepped (false when every pulse of the
-// dispatch is applied as a map: the RF step is then left out, and its registers).
+// NT: coil tiles (0: any, the sensitivities read from memory per flush); NUT: NUFFT runs: 0 none, 1 by spread_run
+// (hb_forward_product), 4 and 8 by nufft_run with up to NUT decay terms (their weights in registers); RF: RF segments are
+// stepped (false when every pulse of the dispatch is applied as a map: the RF step is then left out, and its registers).
 // The read-only inputs and the NUFFT partials come in again as noalias parameters (the same pointers as in cs_in and
 // nu_in): no store of the kernel can change the records, so they load through the scalar cache instead of one vector
 // load per wave and a readfirstlane per value.
@@ -585,6 +585,16 @@ static void launch_forward(const hb_case& cs, int s0, int s1, float* partial, in
 }
 }  // namespace hb
 
+// spread_run against nufft_run. A run gains with its columns, and two tiles' products lose where the windows are narrow; a
+// change of kind costs the weights formed anew. 1,024 runs of 64 samples, 262,144 spins, product against columns staged, one
+// kind: 8 coils 3.81 against 3.91 ms with 5 columns, 3.81 / 4.21 with 7, 4.17 / 5.72 with 21, 4.19 / 6.50 with 28; 16 coils
+// 5.74 / 4.02 with 5, 5.91 / 5.56 with 14, 6.74 / 6.86 with 21, 7.04 / 8.15 with 28. Two kinds in turn (bipolar readouts), 21
+// columns: 10.29 / 5.75 and 14.38 / 6.89. So a column is worth a change in 64 runs, from 4 columns (one tile) or 20 (two).
+extern "C" int32_t hb_forward_product(int32_t cols, int32_t n_tiles, int32_t kind_changes) {
+    using namespace hb;
+    return cols <= kCols && n_tiles <= 2 && kind_changes <= 16 * (cols - (n_tiles == 1 ? 4 : 20));
+}
+
 extern "C" int hb_forward(const hb_case* cs, int32_t s0, int32_t s1, float* partial, int32_t rows,
                           const hb_nufft* nu, void* stream) {
     using namespace hb;
@@ -603,7 +613,7 @@ extern "C" int hb_forward(const hb_case* cs, int32_t s0, int32_t s1, float* part
     const hb_nufft arg = nu ? *nu : none;
     if (!nu)
         launch_forward<0>(*cs, s0, s1, partial, rows, arg, grid, block, lds, st);
-    else if (nu->cols <= kCols && cs->n_tiles <= 2 && cs->rf_free)  // see spread_run
+    else if (cs->rf_free && hb_forward_product(nu->cols, cs->n_tiles, nu->kind_changes))
         launch_forward<1>(*cs, s0, s1, partial, rows, arg, grid, block, sizeof(float) * lds_floats_cols(cs->n_tiles),
                           st);
     else if (nu->terms <= 4)

@@ -606,6 +606,7 @@ def attach_nufft(case: DeviceCase, plan, order, seq: Sequence, adc_np, starts, e
     n_blocks = case.n_pad // BLOCK
     case.perm = order
     case.nu = dict(nu_mod.to_device(plan, dev), plan=plan, cols=cols, runs_max=runs_max,
+                   kind_changes=plan.kind_changes,
                    row_map=torch.from_numpy(mapped.astype(np.int32)).to(dev),
                    row_of=torch.from_numpy(sig_row[heads].astype(np.int32)).to(dev),
                    kind_of=torch.from_numpy(plan.kind).to(dev),
@@ -650,7 +651,7 @@ def run_forward(case: DeviceCase, lib=None, keep: bool = False, timer=None) -> l
     nu_arg = None
     if nu is not None:
         nu_arg = hip.HbNufft(nu["nu"].data_ptr(), nu["nu_win"].data_ptr(), nu["part"].data_ptr(), nu["runs_max"],
-                             nu["cols"], nu["plan"].terms, 0)
+                             nu["cols"], nu["plan"].terms, nu["kind_changes"])
     for d, (s0, s1, r0, nr) in enumerate(zip(case.starts, case.ends, case.row_starts, case.rows)):
         if keep:  # with a bound pool, its Mzb and low part as rows 6, 7
             mb = None if mt_bufs is None else mt_bufs["mb"]

@@ -76,7 +76,7 @@ class HbNufft(ctypes.Structure):
         ("runs_max", ctypes.c_int32),
         ("cols", ctypes.c_int32),
         ("terms", ctypes.c_int32),
-        ("reserved", ctypes.c_int32),
+        ("kind_changes", ctypes.c_int32),
     ]
 
 
@@ -126,6 +126,8 @@ def load() -> ctypes.CDLL:
         lib.hb_abi_version.restype = ctypes.c_int
         lib.hb_mlp_workspace.restype = ctypes.c_int64
         lib.hb_mlp_workspace.argtypes = [ctypes.c_int32]
+        lib.hb_forward_product.restype = ctypes.c_int32
+        lib.hb_forward_product.argtypes = [ctypes.c_int32] * 3
         lib.hb_ifftc_plane_takes.restype = ctypes.c_int32
         lib.hb_ifftc_plane_takes.argtypes = [ctypes.c_int64] * 2
         lib.hb_adjoint_runs_takes.restype = ctypes.c_int32

@@ -126,6 +126,11 @@ class Plan:
     def cols(self) -> int:
         return WMAX * self.terms
 
+    @property
+    def kind_changes(self) -> int:
+        """Of 1,024 runs, how many follow one of another kind (rounded up)."""
+        return -(-1024 * int(np.count_nonzero(np.diff(self.kind))) // len(self.runs))
+
 
 def make_plan(seq: Sequence, width: int = 6, terms: int = 3) -> Plan | None:
     """The run selection and the grid parameters (no spin-dependent parts), or None without readout runs."""

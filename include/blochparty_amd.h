@@ -103,7 +103,7 @@ typedef struct hb_nufft {
     float* part;
     int32_t runs_max, cols;
     int32_t terms;    /* = params[2], 1..HB_NUFFT_MAX_TERMS (selects the kernel variant) */
-    int32_t reserved; /* 0 */
+    int32_t kind_changes; /* of 1,024 of the case's runs, how many follow one of another kind (0: one kind, or not known) */
 } hb_nufft;
 
 /* Forward event loop over segments [s0, s1) (replaces bloch_chunk_mma, cuda/kernels.cu.in:2-185, one launch per
@@ -114,6 +114,10 @@ typedef struct hb_nufft {
  * after that occurrence (its map was applied at the occurrence's first segment, in an earlier dispatch). */
 int hb_forward(const hb_case* cs, int32_t s0, int32_t s1, float* partial, int32_t rows, const hb_nufft* nu,
                void* stream);
+
+/* Whether hb_forward spreads NUFFT runs as one matrix product each (a kind's weights kept from run to run) in a dispatch
+ * with rf_free: windows of cols columns, n_tiles coil tiles, hb_nufft's kind_changes. Otherwise column by column. */
+int32_t hb_forward_product(int32_t cols, int32_t n_tiles, int32_t kind_changes);
 
 /* Deterministic cross-block sum (replaces the float atomicAdd of cuda/common.cuh:77-89): for r < rows,
  * sig[((row0 + r) * n_coils + c) * 2 + {re, im}] = exp(-i psi[row0 + r]) * sum over blocks, in float64 in a fixed

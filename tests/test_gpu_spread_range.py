@@ -29,7 +29,8 @@ def spins(n, t1=(0.5, 2.0), t2=(0.3, 0.5)):
 
 def both_routes(ph, seq, coils, m_init=None):
     case = driver.prepare_case(ph, seq, coils, m_init, reuse=True, nufft=(6, 3))
-    assert case.nu is not None and all(case.rf_free) and case.nu["cols"] <= 32
+    assert case.nu is not None and all(case.rf_free) and 20 < case.nu["cols"] <= 32
+    case.nu["kind_changes"] = 0  # the matrix product, also for kinds in turn
     driver.run_forward(case)
     spread = driver.read_result(case)
     case.rf_free = [False] * len(case.rf_free)  # always correct: the general variant
