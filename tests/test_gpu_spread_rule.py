@@ -1,14 +1,17 @@
 """Which spreading NUFFT runs take (hb_forward_product): by the windows' columns, the coil tiles and how often the runs' kind
 changes; and the matrix product on kinds in turn with one and two tiles, which the rule no longer sends there, against the
-staged spreading (as test_gpu_spread.py, with its tolerance)."""
+staged spreading (as test_gpu_spread.py, with its tolerance). The same for the runs' part of the reverse sweep
+(adjoint.runs_beside; as test_gpu_nufft_back.py, with its tolerance)."""
+
+from dataclasses import replace
 
 import pytest
 import torch
 
 import blochparty_amd as bp
-from blochparty_amd.engines import driver, hip
+from blochparty_amd.engines import adjoint, driver, hip
 from blochparty_amd.engines import nufft as nu_mod
-from cases import rel
+from cases import rel, weighted_loss
 from test_gpu_spread import scan
 
 f64 = torch.float64
@@ -55,3 +58,36 @@ def test_product_on_kinds_in_turn(gpu, n_spins, coils, kinds, nufft, chunk, spoi
         out.append(driver.read_result(case))
     assert rel(out[0].m, out[1].m) < 1e-5
     assert rel(out[0].signal, out[1].signal) < 2e-6
+
+
+def test_rule_of_the_reverse():
+    """Beside the sweep with one kind from 7 columns on (6 with 8 coils, 5 with 16), inside it for kinds in turn unless the
+    coils pay for the weights, and wherever the kernel refuses."""
+    beside = adjoint.runs_beside
+    for nc, first in ((1, 7), (2, 7), (4, 7), (8, 6), (16, 5)):
+        assert all(beside(nc, cols, 0) == (cols >= first) for cols in range(1, 33))
+        assert not beside(nc, 33, 0) and beside(nc, 21, 100) and beside(nc, 21, 1024) == (nc == 16)
+    assert not beside(3, 21, 0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_spins,coils,kinds,every", [(255, 1, 2, 128), (700, 2, 3, 64), (300, 4, 2, 192)])
+def test_beside_on_kinds_in_turn(gpu, monkeypatch, n_spins, coils, kinds, every):
+    g = torch.Generator().manual_seed(n_spins)
+    u = lambda lo, hi: lo + (hi - lo) * torch.rand(n_spins, generator=g, dtype=f64)
+    x = 0.006 + u(0, 0.012) * -(-n_spins // 256)
+    ph = bp.Phantom(torch.stack([x, u(-2e-4, 2e-4), u(-2e-4, 2e-4)], 1), u(0.5, 2.0), u(0.3, 2.0), u(0.02, 0.3),
+                    u(-60.0, 60.0))
+    c = torch.complex(*torch.randn(2, n_spins, coils, generator=g, dtype=f64))
+    seq, taken, out = scan(24, kinds, 1, 7), [], []
+    for beside in (True, False):
+        monkeypatch.setattr(adjoint, "runs_beside", lambda nc, cols, changes, b=beside: taken.append((cols, changes)) or b)
+        leaves = {k: getattr(ph, k).clone().requires_grad_() for k in ("pos", "pd", "t1", "t2", "db0")}
+        ck = c.clone().requires_grad_()
+        r = bp.simulate(replace(ph, **leaves), seq, ck, engine="gpu", pulses="reuse", readouts="nufft",
+                        checkpoint_every=every)
+        out.append(torch.autograd.grad(weighted_loss(r.signal, r.m), [*leaves.values(), ck]))
+    assert taken and all(cols <= 32 and changes > 800 for cols, changes in taken)
+    for name, a, b in zip((*leaves, "coils"), *out):
+        assert bool(torch.isfinite(a.abs()).all()) and float(b.abs().max()) > 0
+        assert rel(a, b) <= 1e-4, name
