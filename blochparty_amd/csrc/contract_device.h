@@ -16,7 +16,8 @@
 // products are exact in the float32 accumulator, and the pairs hold each operand to 2^-24 relative (2^-33 of the bound
 // at least), so D is as close to the exact sum as a float32 product would be, at six 16-cycle instructions per tile
 // and flush in place of sixteen 32-cycle v_mfma_f32_16x16x4f32. More tiles use the float32 instruction, with the
-// sensitivities read from memory.
+// sensitivities read from memory. So does F32 (the full variant), with the sensitivities in registers as they are: it takes
+// no scales, and a coil, a spin or a late echo far below the case's largest keeps its 24 bits.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -72,9 +73,11 @@ __device__ __forceinline__ void split8(const float* x, h8& hi, h8& lo) {
 // of two v_mfma_f32_16x16x32_f16 (u = 0..7 and 8..15); NT = 0: read from memory in float32 at every flush, value u of
 // tile t at sa[t st + u su] (rows of the tile from n_rows on are zeros and not read).
 // out_scale undoes the sensitivities' and the staged values' scales (powers of two: exact).
-template <int NT>
+template <int NT, bool F32 = false>
 struct Sens {
-    h8 hi[NT > 0 ? NT : 1][2], lo[NT > 0 ? NT : 1][2];
+    static constexpr bool kPairs = NT > 0 && !F32;
+    h8 hi[kPairs ? NT : 1][2], lo[kPairs ? NT : 1][2];
+    float a[NT > 0 && F32 ? NT : 1][16];
     const float* sa;
     size_t st;
     int su, n_rows;
@@ -88,21 +91,33 @@ struct Sens {
     __device__ __forceinline__ void scales(float x_scale_, float& sens_scale) {
         x_scale = x_scale_ > 0.0f ? x_scale_ : 1.0f;
         if (!(sens_scale > 0.0f)) sens_scale = 1.0f;
-        if (NT > 0) x_scale *= kLift, sens_scale *= kLift;
-        out_scale = 1.0f / (NT > 0 ? x_scale * sens_scale : x_scale);
+        if (kPairs) x_scale *= kLift, sens_scale *= kLift;
+        out_scale = 1.0f / (kPairs ? x_scale * sens_scale : x_scale);
     }
 
-    __device__ __forceinline__ void load(float x_scale_, float sens_scale, int lane) {
-        scales(x_scale_, sens_scale);
+    // F32: no scales
+    __device__ __forceinline__ void load_f32(int lane) {
+        static_assert(F32, "float32 operands");
+        x_scale = out_scale = 1.0f;
         if constexpr (NT > 0) {
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    float a[8];
+                for (int u = 0; u < 16; ++u) a[t][u] = at(t, u, lane & 15);
+        }
+    }
+
+    __device__ __forceinline__ void load(float x_scale_, float sens_scale, int lane) {
+        scales(x_scale_, sens_scale);
+        if constexpr (kPairs) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) a[e] = at(t, 8 * i + e, lane & 15) * sens_scale;
-                    split8(a, hi[t][i], lo[t][i]);
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    float x[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[e] = at(t, 8 * i + e, lane & 15) * sens_scale;
+                    split8(x, hi[t][i], lo[t][i]);
                 }
         }
     }
@@ -125,8 +140,8 @@ __device__ __forceinline__ void store_pq(float* mine, int vals, int t, int lane,
 // staging block (a wave-scope fence orders its lanes' writes before the reads), and the waves' sums alternate
 // between two buffers, so a flush's writes never meet the previous flush's reads (every wave has passed this
 // flush's barrier, after those reads, before it can write the buffer again two flushes later).
-template <int NT>
-__device__ __forceinline__ void flush_to(float* stg, float* wred2, int& par, const Sens<NT>& S, int nt,
+template <int NT, bool F32>
+__device__ __forceinline__ void flush_to(float* stg, float* wred2, int& par, const Sens<NT, F32>& S, int nt,
                                          int n_out_cols, float* __restrict__ out, int k_first = 8,
                                          float* __restrict__ out_rest = nullptr, int k_skip = 0) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -147,14 +162,15 @@ __device__ __forceinline__ void flush_to(float* stg, float* wred2, int& par, con
         }
     }
     float* mine = wred + wave * 8 * vals;
+    constexpr bool kPairs = Sens<NT, F32>::kPairs;
     h8 bh[2], bl[2];
-    if constexpr (NT > 0) {
+    if constexpr (kPairs) {
         split8(b, bh[0], bl[0]);
         split8(b + 8, bh[1], bl[1]);
     }
     for (int t = 0; t < nt; ++t) {
         f4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        if constexpr (NT > 0) {
+        if constexpr (kPairs) {
             // A B = Ah Bh + Ah Bl + Al Bh (+ Al Bl, under 2^-22 of the product: dropped), small terms first; each
             // product of float16 values is exact in the float32 accumulator
 #pragma unroll
@@ -166,7 +182,8 @@ __device__ __forceinline__ void flush_to(float* stg, float* wred2, int& par, con
         } else {
 #pragma unroll
             for (int u = 0; u < 16; ++u)
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(S.at(t, u, jj), b[u], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(NT > 0 ? S.a[NT > 0 ? t : 0][u] : S.at(t, u, jj), b[u], acc, 0,
+                                                           0, 0);
         }
         store_pq(mine, vals, t, lane, acc);
     }
@@ -187,11 +204,11 @@ __device__ __forceinline__ void flush_to(float* stg, float* wred2, int& par, con
 }
 
 // The staged samples into the partial rows [row, row + nb) of this workgroup (never past the buffer's rows).
-template <int NT>
-__device__ __forceinline__ void flush(float* stg, float* wred2, int& par, const Sens<NT>& S, int nt, int nb, int row,
+template <int NT, bool F32>
+__device__ __forceinline__ void flush(float* stg, float* wred2, int& par, const Sens<NT, F32>& S, int nt, int nb, int row,
                                       int rows, float* __restrict__ partial) {
     const int n_out = row + nb <= rows ? nb : (rows > row ? rows - row : 0);
-    flush_to<NT>(stg, wred2, par, S, nt, n_out, partial + ((size_t)blockIdx.x * rows + row) * (16 * nt));
+    flush_to(stg, wred2, par, S, nt, n_out, partial + ((size_t)blockIdx.x * rows + row) * (16 * nt));
 }
 
 }  // namespace hb

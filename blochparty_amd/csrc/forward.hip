@@ -21,11 +21,11 @@ __device__ __forceinline__ void flush_cols(float* stg, float* wred, int& par, co
                                            float* __restrict__ grid_out) {
     const int vals = 16 * nt;
     if (pending == 0) {
-        flush_to<NT>(stg, wred, par, S, nt, nb, grid_out);
+        flush_to(stg, wred, par, S, nt, nb, grid_out);
         return;
     }
     const int keep = row + pending <= rows ? pending : (rows > row ? rows - row : 0);  // never past the rows
-    flush_to<NT>(stg, wred, par, S, nt, nb, partial + ((size_t)blockIdx.x * rows + row) * vals, keep, grid_out,
+    flush_to(stg, wred, par, S, nt, nb, partial + ((size_t)blockIdx.x * rows + row) * vals, keep, grid_out,
                  pending - keep);
     row += pending;
 }
@@ -394,7 +394,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
         if constexpr (MAT) {
             flush_spread<NS>(stg, wred, par, W, S.out_scale, count, at, rows, partial);
         } else {
-            flush<NT>(stg, wred, par, S, nt, count, at, rows, partial);
+            flush(stg, wred, par, S, nt, count, at, rows, partial);
         }
     };
     Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};

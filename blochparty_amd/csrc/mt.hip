@@ -20,9 +20,10 @@
 //   vanish at equilibrium, so that its rounding vanishes there too, and no steady state (two divisions) is needed.
 //   Short steps (an RF substep: eigenvalues times t under 0.03) take alpha and beta from their series: no square root,
 //   exponential or division; longer ones from the eigenvalues' expm1.
-// - ADC: eight samples at a time are staged in LDS and contracted with the coils on the matrix cores
+// - ADC: eight samples at a time are staged in LDS and contracted with the coils on the matrix cores in float32
 //   (contract_device.h), one barrier per eight; the workgroup's sums go to the partial rows that hb_signal_reduce sums
-//   in a fixed order: no atomics.
+//   in a fixed order: no atomics. (float16 pairs took 9.67 ms in place of 10.00, but lost a coil 2^-17 of another, or spins
+//   beside one 2^24 as bright that no coil sees, most of their bits.)
 //
 // What bounds it: with 65,536 spins every SIMD has one wave, so nothing hides a wave's latency, and a segment costs its
 // chain of dependent instructions. What only depends on a segment's offset (its concomitant field, the saturation's
@@ -31,7 +32,7 @@
 // an RF train is stepped in a loop of its own that reads four values per substep, a readout run in one that reads none
 // and relaxes the longitudinal components once. The next record is loaded while the current one is stepped, and the
 // lanes touch the records 64 ahead, so that they are in the L2 when their turn comes. 65,536 spins with a bound pool and
-// leading-order fields, 8 coils, 32,256 segments (12,800 RF, 16,384 samples): 9.7 ms, against 34.8 ms with a barrier and
+// leading-order fields, 8 coils, 32,256 segments (12,800 RF, 16,384 samples): 10.0 ms, against 34.8 ms with a barrier and
 // a shuffle tree per sample, steady states by division and every factor formed per segment. Of its 5.75 million issue
 // slots a wave uses 2.3 for VALU and 1.0 for scalar instructions and waits in 1.8 (SQ counters).
 #include "bloch_device.h"
@@ -183,10 +184,10 @@ __global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt
 #pragma unroll
         for (int i = 0; i < 7; ++i) cc[i] = mt.conc[(size_t)i * np + j];
     }
-    Sens<NT> S;
+    Sens<NT, true> S;
     S.sa = sens_r + (size_t)(lane & 15) * np + blockIdx.x * kBlock + wave * 64 + 16 * (lane >> 4);
     S.st = 16 * (size_t)np, S.su = 1, S.n_rows = 2 * cs.n_coils;
-    S.load(cs.x_scale, cs.sens_scale, lane);
+    S.load_f32(lane);
     int nb = 0, row = 0, par = 0;   // staged samples, the first one's partial row, the flush's buffer
     XStep xf = {0.0f, 0.0f, 0.0f};  // free segments: the unsaturated exchange over dt (with a bound pool)
     XStep xl = {0.0f, 0.0f, 0.0f};  // and over the last readout run
@@ -270,10 +271,10 @@ __global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt
     auto stage = [&](int r) {  // uniform: every lane takes it
         if (r < 0 || r >= rows) return;
         if (nb == 0) row = r;
-        stg[nb * kStgStride + lane] = m.mx * S.x_scale;
-        stg[(8 + nb) * kStgStride + lane] = m.my * S.x_scale;
+        stg[nb * kStgStride + lane] = m.mx;
+        stg[(8 + nb) * kStgStride + lane] = m.my;
         if (++nb == 8) {
-            flush<NT>(stg, wred, par, S, nt, 8, row, rows, partial);
+            flush(stg, wred, par, S, nt, 8, row, rows, partial);
             nb = 0;
         }
     };
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt
         if (fl & HB_SPOIL) m.mx = m.my = 0.0f;
         s += len;
     }
-    if (nb > 0) flush<NT>(stg, wred, par, S, nt, nb, row, rows, partial);
+    if (nb > 0) flush(stg, wred, par, S, nt, nb, row, rows, partial);
     store_state(cs.state, np, j, m);
     if (pool) mt.mb[j] = mb, mt.mb[np + j] = lb;
 }

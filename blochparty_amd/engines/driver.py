@@ -545,16 +545,14 @@ def prepare_case(phantom: Phantom, seq: Sequence, coils=None, m_init=None, *, ch
         for a, _ in occ:
             covered[a : a + k] = True
     rf_cum = np.concatenate([[0], np.cumsum(flag_array(seq.is_rf) & ~covered)])
-    # the coil contraction's scales
-    if full:  # its kernels read the sensitivities in rows (mt.attach)
-        sens_a, largest = torch.zeros(0, dtype=torch.float32), torch.view_as_real(coils.detach().to(torch.complex128))
-    else:
-        sens_a = largest = sens_operand(coils, n, n_pad, n_tiles)
-    sens_scale = pow2_scale(float(largest.abs().max()) if largest.numel() else 0.0)
-    host = lambda t: t.detach().double().cpu()
-    x_scale = pow2_scale(magnetization_bound(host(phantom.pd), host(phantom.t1), host(phantom.t2),
-                                             (m64[0] * m64[0] + m64[1] * m64[1] + m64[2] * m64[2]).sqrt(),
-                                             float(host(seq.dt).sum())))
+    sens_a, sens_scale, x_scale = torch.zeros(0, dtype=torch.float32), 1.0, 1.0
+    if not full:  # (the full variant reads the sensitivities in rows, mt.attach, and takes no scales)
+        sens_a = sens_operand(coils, n, n_pad, n_tiles)
+        sens_scale = pow2_scale(float(sens_a.abs().max()) if sens_a.numel() else 0.0)
+        host = lambda t: t.detach().double().cpu()
+        x_scale = pow2_scale(magnetization_bound(host(phantom.pd), host(phantom.t1), host(phantom.t2),
+                                                 (m64[0] * m64[0] + m64[1] * m64[1] + m64[2] * m64[2]).sqrt(),
+                                                 float(host(seq.dt).sum())))
     psi_rows = np.remainder(seq.adc_phase.detach().double().cpu().numpy()[flag_array(seq.adc)],
                             2 * math.pi)
     max_rows = max(rows + [0])

@@ -14,7 +14,6 @@ plain path's.
 from __future__ import annotations
 
 import ctypes
-import math
 
 import numpy as np
 import torch
@@ -77,11 +76,6 @@ def attach(case, phantom, coils, m_init, n: int, n_pad: int, dev, conc=None, fre
         out.update(conc=coef.to(dev).contiguous(), conc_mode=int(conc[1]))
     if phantom.bound is not None:
         out.update(_pool_buffers(phantom, freq, m_init, n, n_pad, dev))
-        # the exchange may bring the bound pool's magnetization into the free pool: its bound for the contraction
-        # (powers of two: the smaller scale serves both)
-        mb = float(out["mb"].abs().sum(0).max())
-        if mb > 0 and math.isfinite(mb):
-            case.x_scale = min(case.x_scale, math.ldexp(1.0, -min(100, max(-100, math.ceil(math.log2(mb)) + 1))))
     case.extra["mt"] = out
 
 
