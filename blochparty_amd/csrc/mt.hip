@@ -22,7 +22,7 @@
 //   exponential or division; longer ones from the eigenvalues' expm1.
 // - ADC: eight samples at a time are staged in LDS and contracted with the coils on the matrix cores in float32
 //   (contract_device.h), one barrier per eight; the workgroup's sums go to the partial rows that hb_signal_reduce sums
-//   in a fixed order: no atomics. (float16 pairs took 9.67 ms in place of 10.00, but lost a coil 2^-17 of another, or spins
+//   in a fixed order: no atomics. (float16 pairs took 0.33 ms less, but lost a coil 2^-17 of another, or spins
 //   beside one 2^24 as bright that no coil sees, most of their bits.)
 //
 // What bounds it: with 65,536 spins every SIMD has one wave, so nothing hides a wave's latency, and a segment costs its
@@ -32,7 +32,7 @@
 // an RF train is stepped in a loop of its own that reads four values per substep, a readout run in one that reads none
 // and relaxes the longitudinal components once. The next record is loaded while the current one is stepped, and the
 // lanes touch the records 64 ahead, so that they are in the L2 when their turn comes. 65,536 spins with a bound pool and
-// leading-order fields, 8 coils, 32,256 segments (12,800 RF, 16,384 samples): 10.0 ms, against 34.8 ms with a barrier and
+// leading-order fields, 8 coils, 32,256 segments (12,800 RF, 16,384 samples): 10.1 ms, against 34.8 ms with a barrier and
 // a shuffle tree per sample, steady states by division and every factor formed per segment. Of its 5.75 million issue
 // slots a wave uses 2.3 for VALU and 1.0 for scalar instructions and waits in 1.8 (SQ counters).
 #include "bloch_device.h"
@@ -42,14 +42,6 @@
 
 namespace hb {
 namespace {
-
-// hi + lo += d, the low part as Kahan's sum keeps it: exact where |hi| >= |d + lo|, within d's own rounding otherwise
-// (4 operations against two_sum's 7).
-__device__ __forceinline__ void add_low(float& hi, float& lo, float d) {
-    const float y = d + lo, t = hi + y;
-    lo = y - (t - hi);
-    hi = t;
-}
 
 // A spin's bound pool: f, the exchange rates k and k f, R1b, T2b, dw, and f PD.
 struct Pool {
@@ -114,8 +106,8 @@ __device__ __forceinline__ void exchange_free(const XStep& x, const Pool& p, flo
     const float ex = p.k * (fmaf(-p.f, m.mz, mb) + fmaf(-p.f, m.lz, lb));
     float dz, db;
     increments(x, p, fmaf(r1, (pd - m.mz) - m.lz, ex), fmaf(p.r1b, (p.fpd - mb) - lb, -ex), dz, db);
-    add_low(m.mz, m.lz, dz);
-    add_low(mb, lb, db);
+    two_sum(m.mz, m.lz, dz);
+    two_sum(mb, lb, db);
 }
 
 // G(2 pi delta) [s]: the Lorentzian, or T2b F(x) from the table of ln F (held at the cut, 0 past the table's end).
@@ -239,10 +231,10 @@ __global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt
         if (pool) {
             float dz2, db2;
             exchange_rf(x, b, p.pd, p.r1, w, z2, b1, dz2, db2);
-            add_low(m.mz, m.lz, dz1 + drz + dz2);
-            add_low(mb, lb, db1 + db2);
+            two_sum(m.mz, m.lz, dz1 + drz + dz2);
+            two_sum(mb, lb, db1 + db2);
         } else {
-            add_low(m.mz, m.lz, dz1 + drz + (z2 - p.pd) * e1r);
+            two_sum(m.mz, m.lz, dz1 + drz + (z2 - p.pd) * e1r);
         }
     };
     // the free segment's factors (hints in f, honoured once factors are held)
@@ -334,7 +326,7 @@ __global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt
                 if (pool)
                     exchange_free(xl, b, p.pd, p.r1, m, mb, lb);
                 else
-                    add_low(m.mz, m.lz, (m.mz - p.pd) * e1l);
+                    two_sum(m.mz, m.lz, (m.mz - p.pd) * e1l);
                 s += len;
                 continue;
             }
@@ -342,7 +334,7 @@ __global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt
             if (pool)
                 exchange_free(xf, b, p.pd, p.r1, m, mb, lb);
             else
-                add_low(m.mz, m.lz, (m.mz - p.pd) * e1f);
+                two_sum(m.mz, m.lz, (m.mz - p.pd) * e1f);
         }
         if (fl & HB_ADC) stage(q.pad[0] - row0);
         if (fl & HB_SPOIL) m.mx = m.my = 0.0f;
