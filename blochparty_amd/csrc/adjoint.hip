@@ -19,6 +19,8 @@
 // Reused pulses (maps) and NUFFT readout runs are one record each, their other segments identity bodies: the replay
 // jumps over them, the reverse skips the 8-blocks inside them (pulse_reverse, nufft_reverse below). Few spins: intervals in
 // chunks side by side (sweep_kernel below); NUFFT runs with narrow windows: their samples beside the sweep (nufft_back.hip).
+#include <algorithm>
+
 #include "adjoint_device.h"
 #include "nufft_back.h"
 
@@ -605,17 +607,19 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
 //
 // Walked by one lane per spin, 55,296 spins keep one wave on each SIMD and wait for a record or a row at every segment.
 // The bare adjoint needs no state and the replay no adjoint: sweep_kernel takes both over the interval side by side
-// (workgroups [0, n_pad / 256) the replay, the rest lambda from lam after s1 to lam before s0, its value at every chunk's
-// end in lam_c); then adjoint_kernel<.., CHUNK> reverses the chunks, with their gradients, in parallel, and
-// chunk_sums_kernel adds them, last chunk first, in float64. Chunks start at multiples of their length, which depends
+// (the first workgroups the replay, the rest lambda from lam after the last segment to lam before the first, its value at
+// every chunk's end in lam_c); then adjoint_kernel<.., CHUNK> reverses the chunks, with their gradients, in parallel, and
+// chunk_sums_kernel adds them, last chunk first, in float64. A long interval is replayed whole and then reversed kBatch
+// segments at a time, last first, in the same workspace. Chunks start at multiples of their length, which depends
 // only on the number of spins, so the gradients are the same bit for bit for any interval length (a multiple of 64).
 // What bounds it then: the sweep's chain (0.31 us a segment, its records from the scalar cache one ahead) and the chunks'
 // VALU work. 24^3 x 4 spins (216 workgroups), every RF substep, 8 coils, 347 intervals of 384 segments, forward and
 // reverse: 271 -> 149 ms (533 us an interval in one walk, 318 in chunks); 28^3 x 4, 16 coils: 671 -> 284 ms; a 128^2
 // turbo spin echo's map fit (32 workgroups, 64 segments an interval): 81 -> 50 ms a call.
+// replays: workgroups that replay [r0, r1) (n_pad / 256 of them, or none); the others take lambda back over [s0, s1).
 template <int NC>
-__global__ __launch_bounds__(kBlockA) void sweep_kernel(hb_case cs_in, hb_adjoint ad_in, int s0, int s1, int chunk,
-                                                        float* __restrict__ lam_c, const hb_segment* __restrict__ segs,
+__global__ __launch_bounds__(kBlockA) void sweep_kernel(hb_case cs_in, hb_adjoint ad_in, int replays, int r0, int r1,
+                                                        int s0, int s1, int chunk, float* __restrict__ lam_c, const hb_segment* __restrict__ segs,
                                                         const float* __restrict__ spins,
                                                         const float* __restrict__ pos_lo, const float* __restrict__ ckpt,
                                                         const float* __restrict__ h, const float* __restrict__ sens) {
@@ -623,14 +627,14 @@ __global__ __launch_bounds__(kBlockA) void sweep_kernel(hb_case cs_in, hb_adjoin
     cs.segs = segs, cs.spins = spins, cs.pos_lo = pos_lo;
     hb_adjoint ad = ad_in;
     ad.ckpt = ckpt;
-    const int np = cs.n_pad, n_blocks = np / kBlockA;
-    const bool back = (int)blockIdx.x >= n_blocks;  // uniform
-    const int j = ((int)blockIdx.x - (back ? n_blocks : 0)) * kBlockA + threadIdx.x;
-    touch_interval<NC>(segs, h, s0, s1);
+    const int np = cs.n_pad;
+    const bool back = (int)blockIdx.x >= replays;  // uniform
+    const int j = ((int)blockIdx.x - (back ? replays : 0)) * kBlockA + threadIdx.x;
+    touch_interval<NC>(segs, h, replays ? r0 : s0, replays ? r1 : s1);
     const Spin p = load_spin(cs.spins, cs.pos_lo, np, j);
     const float b1sq = p.b1 * p.b1;
     if (!back) {
-        replay_interval<false>(cs, ad, p, b1sq, j, s0, s1);
+        replay_interval<false>(cs, ad, p, b1sq, j, r0, r1);
         return;
     }
     float sr[NC > 0 ? NC : 1], si[NC > 0 ? NC : 1];
@@ -786,19 +790,30 @@ static int chunk_of(int n_blocks) {
     return chunk;
 }
 
+// Segments reversed at a time: the workspace (3 + 8 + 2 nc floats per chunk and spin) stays under 360 MB at 32 workgroups
+// and 1.5 GB at 1,024, whatever the interval's length, and 256 chunks are enough for any case.
+constexpr int kBatch = 2048;
+
 template <int NC>
 static hipError_t launch_chunks(const hb_case* cs, const hb_adjoint* ad, int s0, int s1, float* work, hipStream_t st) {
-    const int n_blocks = cs->n_pad / kBlockA, chunk = chunk_of(n_blocks), n_chunks = (s1 - s0 + chunk - 1) / chunk;
-    float* part = work + (size_t)n_chunks * 3 * cs->n_pad;
-    hipLaunchKernelGGL((sweep_kernel<NC>), dim3(2 * n_blocks), dim3(kBlockA), 0, st, *cs, *ad, s0, s1, chunk, work,
-                       cs->segs, cs->spins, cs->pos_lo, ad->ckpt, ad->h, ad->sens);
-    auto kernel = ad->seg_grads ? adjoint_kernel<NC, true, false, true> : adjoint_kernel<NC, false, false, true>;
-    hipLaunchKernelGGL(kernel, dim3(n_blocks, n_chunks), dim3(kBlockA), 0, st, *cs, *ad, s0, s1, cs->segs, cs->spins,
-                       cs->pos_lo, cs->maps, ad->ckpt, ad->h, ad->sens, ad->maps_d, ad->nu_params, ad->nu_win,
-                       ad->nu_grid, chunk, work, part);
+    const int n_blocks = cs->n_pad / kBlockA, chunk = chunk_of(n_blocks);
     const int coil_rows = NC > 0 && ad->coil_grads ? 2 * NC : 0;
-    hipLaunchKernelGGL(adjoint_chunk_sums_kernel, dim3(n_blocks, 8 + coil_rows), dim3(kBlockA), 0, st, part, n_chunks,
-                       8 + 2 * NC, cs->n_pad, ad->gs, ad->gc);
+    auto kernel = ad->seg_grads ? adjoint_kernel<NC, true, false, true> : adjoint_kernel<NC, false, false, true>;
+    int b1 = s1;
+    for (int b0 = s0 + (s1 - s0 - 1) / kBatch * kBatch; b0 >= s0; b1 = b0, b0 -= kBatch) {
+        const int replays = b1 == s1 ? n_blocks : 0, n_chunks = (b1 - b0 + chunk - 1) / chunk;
+        float* part = work + (size_t)n_chunks * 3 * cs->n_pad;
+        hipLaunchKernelGGL((sweep_kernel<NC>), dim3(replays + n_blocks), dim3(kBlockA), 0, st, *cs, *ad, replays, s0, s1,
+                           b0, b1, chunk, work, cs->segs, cs->spins, cs->pos_lo, ad->ckpt, ad->h, ad->sens);
+        hb_adjoint at = *ad;  // the batch's rows of r8 and gseg
+        at.r8 += (size_t)((b0 - s0) >> 3) * 3 * cs->n_pad;
+        if (at.gseg) at.gseg += (size_t)(b0 - s0) * 8;
+        hipLaunchKernelGGL(kernel, dim3(n_blocks, n_chunks), dim3(kBlockA), 0, st, *cs, at, b0, b1, cs->segs, cs->spins,
+                           cs->pos_lo, cs->maps, ad->ckpt, ad->h, ad->sens, ad->maps_d, ad->nu_params, ad->nu_win,
+                           ad->nu_grid, chunk, work, part);
+        hipLaunchKernelGGL(adjoint_chunk_sums_kernel, dim3(n_blocks, 8 + coil_rows), dim3(kBlockA), 0, st, part, n_chunks,
+                           8 + 2 * NC, cs->n_pad, ad->gs, ad->gc);
+    }
     return hipGetLastError();
 }
 
@@ -880,7 +895,7 @@ extern "C" int64_t hb_adjoint_chunks_workspace(int32_t n_pad, int32_t k_max, int
     using namespace hb;
     if (n_pad < kBlockA || n_pad % kBlockA || k_max < 1 || nc < 0 || nc > 16) return 0;
     const int chunk = chunk_of(n_pad / kBlockA);
-    return chunk ? (int64_t)((k_max + chunk - 1) / chunk) * (3 + 8 + 2 * nc) * n_pad : 0;
+    return chunk ? (int64_t)((std::min(k_max, kBatch) + chunk - 1) / chunk) * (3 + 8 + 2 * nc) * n_pad : 0;
 }
 
 extern "C" int hb_adjoint_chunks(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, float* work,

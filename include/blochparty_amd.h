@@ -329,7 +329,8 @@ int hb_adjoint_interval(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int
  * reused pulses and NUFFT runs (n_pulses 0, nu_params NULL) that starts at a multiple of 64, of a case with too few
  * spins to fill the chip, is reversed in chunks of segments side by side, from the adjoint at each chunk's end (found by
  * a sweep of its own beside the replay); the chunks' gradients are added in a fixed order, the same bit for bit for any
- * interval length. Any other interval, and work NULL (also where the workspace is 0): as hb_adjoint_interval. */
+ * interval length (the workspace grows with k_max up to 2,048 segments; longer intervals are reversed 2,048 at a time).
+ * Any other interval, and work NULL (also where the workspace is 0): as hb_adjoint_interval. */
 int64_t hb_adjoint_chunks_workspace(int32_t n_pad, int32_t k_max, int32_t nc);
 int hb_adjoint_chunks(const hb_case* cs, const hb_adjoint* ad, int32_t s0, int32_t s1, float* work, void* stream);
 
