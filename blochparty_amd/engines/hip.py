@@ -15,7 +15,7 @@ from pathlib import Path
 import torch
 
 LIB_PATH = Path(__file__).resolve().parent.parent / "libblochparty_amd.so"
-ABI_VERSION = 25
+ABI_VERSION = 26
 MAX_COILS = 128  # 16 tiles of 8 coils (the forward kernel's LDS budget)
 
 
@@ -121,9 +121,11 @@ def load() -> ctypes.CDLL:
                 f"blochparty_amd HIP library not built ({LIB_PATH} missing): run `python -m blochparty_amd.build`"
             )
         lib = ctypes.CDLL(str(LIB_PATH))
+        lib.hb_abi_version.restype = ctypes.c_int
+        if lib.hb_abi_version() != ABI_VERSION:
+            raise RuntimeError(f"{LIB_PATH} has ABI {lib.hb_abi_version()}, expected {ABI_VERSION}: rebuild it")
         lib.hb_error_string.restype = ctypes.c_char_p
         lib.hb_error_string.argtypes = [ctypes.c_int]
-        lib.hb_abi_version.restype = ctypes.c_int
         lib.hb_mlp_workspace.restype = ctypes.c_int64
         lib.hb_mlp_workspace.argtypes = [ctypes.c_int32]
         lib.hb_forward_product.restype = ctypes.c_int32
@@ -136,8 +138,6 @@ def load() -> ctypes.CDLL:
         lib.hb_adjoint_chunks_workspace.argtypes = [ctypes.c_int32] * 3
         lib.hb_signal_reduce_workspace.restype = ctypes.c_int64
         lib.hb_signal_reduce_workspace.argtypes = [ctypes.c_int32] * 3
-        if lib.hb_abi_version() != ABI_VERSION:
-            raise RuntimeError(f"{LIB_PATH} has ABI {lib.hb_abi_version()}, expected {ABI_VERSION}: rebuild it")
         for name, args in SIGNATURES.items():
             fn = getattr(lib, name)
             fn.restype = ctypes.c_int
