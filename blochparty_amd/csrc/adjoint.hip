@@ -611,7 +611,7 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
 // every chunk's end in lam_c); then adjoint_kernel<.., CHUNK> reverses the chunks, with their gradients, in parallel, and
 // chunk_sums_kernel adds them, last chunk first, in float64. A long interval is replayed whole and then reversed kBatch
 // segments at a time, last first, in the same workspace. Chunks start at multiples of their length, which depends
-// only on the number of spins, so the gradients are the same bit for bit for any interval length (a multiple of 64).
+// only on the numbers of spins and coils, so the gradients are the same bit for bit for any interval length (a multiple of 64).
 // What bounds it then: the sweep's chain (0.31 us a segment, its records from the scalar cache one ahead) and the chunks'
 // VALU work. 24^3 x 4 spins (216 workgroups), every RF substep, 8 coils, 347 intervals of 384 segments, forward and
 // reverse: 271 -> 149 ms (533 us an interval in one walk, 318 in chunks); 28^3 x 4, 16 coils: 671 -> 284 ms; a 128^2
@@ -780,11 +780,13 @@ static hipError_t launch_adjoint(const hb_case* cs, const hb_adjoint* ad, int s0
 // Segments per chunk of a case of n_blocks workgroups, or 0: not in chunks. Chunks are as long as 256 workgroups per 64
 // segments allow (32 workgroups: 8 segments, measured 50 ms against 54 with 16). In chunks the reverse also needs no
 // float64 sums in LDS, so it gains beyond a full chip: 512 workgroups 457 -> 449 ms, 1,000 workgroups 1,395 -> 1,239 ms;
-// the line is the largest size measured (the workspace grows with the spins).
+// the line is the largest size measured (the workspace grows with the spins). Up to two coils leave room in LDS for three
+// workgroups of the walk per CU, so from 513 to 768 it is one round of them and faster: 600 workgroups, 24 repetitions of
+// 72 segments, 1 coil 2,321 us against 2,389 in chunks, 700 2,348 against 2,673 (4 coils 4,497 against 2,837).
 constexpr int kChunkBlocks = 1024;
 
-static int chunk_of(int n_blocks) {
-    if (n_blocks > kChunkBlocks) return 0;
+static int chunk_of(int n_blocks, int nc) {
+    if (n_blocks > kChunkBlocks || (nc <= 2 && n_blocks > 512 && n_blocks <= 768)) return 0;
     int chunk = 8;
     while (chunk < 64 && 64 / (2 * chunk) * n_blocks >= 256) chunk *= 2;
     return chunk;
@@ -796,7 +798,7 @@ constexpr int kBatch = 2048;
 
 template <int NC>
 static hipError_t launch_chunks(const hb_case* cs, const hb_adjoint* ad, int s0, int s1, float* work, hipStream_t st) {
-    const int n_blocks = cs->n_pad / kBlockA, chunk = chunk_of(n_blocks);
+    const int n_blocks = cs->n_pad / kBlockA, chunk = chunk_of(n_blocks, NC);
     const int coil_rows = NC > 0 && ad->coil_grads ? 2 * NC : 0;
     auto kernel = ad->seg_grads ? adjoint_kernel<NC, true, false, true> : adjoint_kernel<NC, false, false, true>;
     int b1 = s1;
@@ -894,7 +896,7 @@ extern "C" int hb_adjoint_interval(const hb_case* cs, const hb_adjoint* ad, int3
 extern "C" int64_t hb_adjoint_chunks_workspace(int32_t n_pad, int32_t k_max, int32_t nc) {
     using namespace hb;
     if (n_pad < kBlockA || n_pad % kBlockA || k_max < 1 || nc < 0 || nc > 16) return 0;
-    const int chunk = chunk_of(n_pad / kBlockA);
+    const int chunk = chunk_of(n_pad / kBlockA, nc);
     return chunk ? (int64_t)((std::min(k_max, kBatch) + chunk - 1) / chunk) * (3 + 8 + 2 * nc) * n_pad : 0;
 }
 
@@ -903,7 +905,7 @@ extern "C" int hb_adjoint_chunks(const hb_case* cs, const hb_adjoint* ad, int32_
     using namespace hb;
     if (!cs || !ad || cs->n_pad <= 0 || cs->n_pad % kBlockA) return hipErrorInvalidValue;
     if (s0 < 0 || s1 < s0 || s1 > cs->n_segments || s1 - s0 > ad->k_max) return hipErrorInvalidValue;
-    if (!work || cs->n_pulses || ad->nu_params || s0 % 64 || !chunk_of(cs->n_pad / kBlockA))
+    if (!work || cs->n_pulses || ad->nu_params || s0 % 64 || !chunk_of(cs->n_pad / kBlockA, ad->nc))
         return hb_adjoint_interval(cs, ad, s0, s1, stream);
     if (s1 == s0) return hipSuccess;
     hipStream_t st = (hipStream_t)stream;

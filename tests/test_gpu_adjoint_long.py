@@ -18,6 +18,15 @@ def test_workspace_has_a_limit():
         assert ws(256 * blocks, 2048, nc) * 4 < 1.6e9
 
 
+def test_where_one_walk_is_faster():
+    """Up to two coils from 513 to 768 workgroups: not in chunks; on both sides and with more coils in chunks."""
+    ws = hip.load().hb_adjoint_chunks_workspace
+    for nc in (0, 1, 2):
+        assert all(ws(256 * b, 384, nc) == 0 for b in (513, 600, 768))
+        assert all(ws(256 * b, 384, nc) > 0 for b in (512, 769, 1024))
+    assert all(ws(256 * b, 384, nc) > 0 for b in (513, 768) for nc in (4, 8, 16))
+
+
 def gradients(ph, seq, c, every, need_seg):
     case = driver.prepare_case(ph, seq, c, chunk=every, aligned=True)
     ckpts = driver.run_forward(case, keep=True)
