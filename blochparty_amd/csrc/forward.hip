@@ -452,10 +452,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
             if (RF && (f & HB_TRAIN)) {  // RF substeps of a shaped pulse, in a loop of their own (only RF state live)
                 const int L = q.pad[3];
                 const hb_segment* first = cs.segs + s;
+                if (!(f & HB_SAME_RF_DT)) half_relax(q.dt, p, k);
                 rf_records(
                     L, [&](int i) { return first + i; },
                     [&](int i, const RfRec& r) {
-                        if (!(r.flags & HB_SAME_RF_DT)) half_relax(first[i].dt, p, k);
+                        if (i > 0 && !(r.flags & HB_SAME_RF_DT)) half_relax(first[i].dt, p, k);
                         rf_step(r, p, b1sq, m, k);
                     });
                 s += L - 1;
