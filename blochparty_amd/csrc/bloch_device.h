@@ -326,23 +326,23 @@ __device__ __forceinline__ void step(const hb_segment& q, int f, const Spin& p, 
 // spins (850 workgroups, three to four waves per SIMD) 4,437 -> 4,201, where one record ahead took 4,198.
 constexpr int kTrain = 3;
 
-template <class At, class Go>
+template <int K = kTrain, class At, class Go>
 __device__ __forceinline__ void rf_records(int L, At at, Go go) {
-    RfRec cur[kTrain], nxt[kTrain];
+    RfRec cur[K], nxt[K];
 #pragma unroll
-    for (int k = 0; k < kTrain; ++k) cur[k] = load_rf(at(min(k, L - 1)));
-    for (int i = 0; i < L; i += 2 * kTrain) {
+    for (int k = 0; k < K; ++k) cur[k] = load_rf(at(min(k, L - 1)));
+    for (int i = 0; i < L; i += 2 * K) {
 #pragma unroll
-        for (int k = 0; k < kTrain; ++k) nxt[k] = load_rf(at(min(i + kTrain + k, L - 1)));
+        for (int k = 0; k < K; ++k) nxt[k] = load_rf(at(min(i + K + k, L - 1)));
 #pragma unroll
-        for (int k = 0; k < kTrain; ++k)
+        for (int k = 0; k < K; ++k)
             if (i + k < L) go(i + k, cur[k]);
-        if (i + kTrain >= L) break;
+        if (i + K >= L) break;
 #pragma unroll
-        for (int k = 0; k < kTrain; ++k) cur[k] = load_rf(at(min(i + 2 * kTrain + k, L - 1)));
+        for (int k = 0; k < K; ++k) cur[k] = load_rf(at(min(i + 2 * K + k, L - 1)));
 #pragma unroll
-        for (int k = 0; k < kTrain; ++k)
-            if (i + kTrain + k < L) go(i + kTrain + k, nxt[k]);
+        for (int k = 0; k < K; ++k)
+            if (i + K + k < L) go(i + K + k, nxt[k]);
     }
 }
 

@@ -71,20 +71,26 @@ __device__ __forceinline__ void split8(const float* x, h8& hi, h8& lo) {
 // The wave's sensitivities as matrix-core operands. NT > 0: each tile's 16 values per lane (spins 16 g + u,
 // u = 0..15, of row l % 16) scaled by the case's sens_scale and split into float16 hi and lo parts, as the A operands
 // of two v_mfma_f32_16x16x32_f16 (u = 0..7 and 8..15); NT = 0: read from memory in float32 at every flush, value u of
-// tile t at sa[t st + u su] (rows of the tile from n_rows on are zeros and not read).
+// tile t at sa[t st + u su].
 // out_scale undoes the sensitivities' and the staged values' scales (powers of two: exact).
 template <int NT, bool F32 = false>
 struct Sens {
     static constexpr bool kPairs = NT > 0 && !F32;
     h8 hi[kPairs ? NT : 1][2], lo[kPairs ? NT : 1][2];
     float a[NT > 0 && F32 ? NT : 1][16];
-    const float* sa;
+    const float *sa, *sa0;
     size_t st;
     int su, n_rows;
     float x_scale, out_scale;
 
+    // F32: rows from n_rows on are zeros, row 0 (sa0) read in their place: every load is unconditional
     __device__ __forceinline__ float at(int t, int u, int row) const {
-        return 16 * t + row < n_rows ? sa[t * st + (size_t)u * su] : 0.0f;
+        if constexpr (F32) {
+            const bool in = 16 * t + row < n_rows;
+            const float v = (in ? sa + t * st : sa0)[(size_t)u * su];
+            return in ? v : 0.0f;
+        }
+        return sa[t * st + (size_t)u * su];
     }
 
     // sa, st, su and n_rows are set; x_scale_ and sens_scale as hb_case's (0 reads as 1)

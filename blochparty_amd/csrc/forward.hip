@@ -376,7 +376,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
     }
     Sens<NT> S;
     S.sa = cs.sens_a + (size_t)(blockIdx.x * kWaves + wave) * nt * 1024 + lane;
-    S.st = 1024, S.su = 64, S.n_rows = 16 * nt;
+    S.st = 1024, S.su = 64;
     int nb = 0, row = 0, par = 0;
     constexpr bool MAT = NUT == 1;
     constexpr int NS = NT > 0 ? NT : 1;

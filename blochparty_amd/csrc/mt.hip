@@ -177,7 +177,8 @@ __global__ __launch_bounds__(kBlock) void forward_mt_kernel(hb_case cs, hb_mt mt
         for (int i = 0; i < 7; ++i) cc[i] = mt.conc[(size_t)i * np + j];
     }
     Sens<NT, true> S;
-    S.sa = sens_r + (size_t)(lane & 15) * np + blockIdx.x * kBlock + wave * 64 + 16 * (lane >> 4);
+    S.sa0 = sens_r + blockIdx.x * kBlock + wave * 64 + 16 * (lane >> 4);
+    S.sa = S.sa0 + (size_t)(lane & 15) * np;
     S.st = 16 * (size_t)np, S.su = 1, S.n_rows = 2 * cs.n_coils;
     S.load_f32(lane);
     int nb = 0, row = 0, par = 0;   // staged samples, the first one's partial row, the flush's buffer
