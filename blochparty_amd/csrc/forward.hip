@@ -397,6 +397,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
             flush(stg, wred, par, S, nt, count, at, rows, partial);
         }
     };
+    // records of an RF train in flight: where the NUFFT runs' or many coils' scalars are live, three spill scalar registers
+    // in the walk itself (200 repetitions of two RF substeps and a NUFFT run, 340,736 spins, 8 coils: 2.59 ms with three,
+    // 2.25 with two)
+    constexpr int kAhead = NUT == 0 && NT > 0 ? kTrain : 2;
     Cache k = {1.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
     float e1_run = 0.0f;  // expm1(-L dt R1) of the last readout run (per sample or NUFFT)
     // the NUFFT decay terms e^{-R2 tau_m}: the spin's, the same for every run
@@ -453,7 +457,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(NT == 2 
                 const int L = q.pad[3];
                 const hb_segment* first = cs.segs + s;
                 if (!(f & HB_SAME_RF_DT)) half_relax(q.dt, p, k);
-                rf_records(
+                rf_records<kAhead>(
                     L, [&](int i) { return first + i; },
                     [&](int i, const RfRec& r) {
                         if (i > 0 && !(r.flags & HB_SAME_RF_DT)) half_relax(first[i].dt, p, k);
