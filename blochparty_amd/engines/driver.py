@@ -344,12 +344,14 @@ def magnetization_bound(pd: torch.Tensor, t1: torch.Tensor, t2: torch.Tensor, m0
     PD R1 / (2 sqrt(R2 (R1 - R2))), the steady state of pulses that hold Mz at its best."""
     if not len(pd):
         return 0.0
+    if not bool((t2 > 2 * t1).any()):
+        return max(float(pd.abs().max()), float(m0.max()))
     pd, r1, r2 = pd.abs(), 1 / t1, 1 / t2
     start = torch.maximum(pd, m0)
     grown = (start * start + pd * pd * (r1 * (0.5 * total))).sqrt()
     steady = torch.where(r2 > 0, 0.5 * pd * r1 / (r2 * (r1 - r2)).clamp_min(1e-300).sqrt(), math.inf)
     long_t2 = torch.maximum(start, torch.minimum(grown, steady))
-    return float(torch.where(r2 < 0.5 * r1, long_t2, start).max())
+    return float(torch.where(t2 > 2 * t1, long_t2, start).max())
 
 
 def sens_operand(coils: torch.Tensor, n: int, n_pad: int, n_tiles: int) -> torch.Tensor:
