@@ -321,9 +321,9 @@ __device__ __forceinline__ void step(const hb_segment& q, int f, const Spin& p, 
 // The RF records at(0) .. at(L - 1) in turn, go(i, record): kTrain of them are loaded while the kTrain before are stepped,
 // as a load costs up to an L2 round trip, more than one step takes; two sets of registers in turn, so that none are moved.
 // Stepped RF of 32^3 x 4 spins (two waves per SIMD): 60.9 ms one ahead, 54.2 two, 49.9 three, 49.9 four; 44^3 x 4: 257, 246,
-// 237, 229; with gradients, 24^3 x 4: 149, 146.7, 145.5, 146.7 (short launches, where longer code costs instruction
-// fetches). Against records moved from one set to the other: 60 trains of 200, 131,072 spins 2,906 -> 2,627 us, 217,600
-// spins (850 workgroups, three to four waves per SIMD) 4,437 -> 4,201, where one record ahead took 4,198.
+// 237, 229 (the reverse sweep's walk, 24^3 x 4: 149, 146.7, 145.5, 146.7). Against records moved from one set to the
+// other: 60 trains of 200, 131,072 spins 2,906 -> 2,627 us, 217,600 spins (850 workgroups, three to four waves per SIMD)
+// 4,437 -> 4,201, where one record ahead took 4,198.
 constexpr int kTrain = 3;
 
 template <int K = kTrain, class At, class Go>
