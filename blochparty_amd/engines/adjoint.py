@@ -223,12 +223,20 @@ def run_backward(case: driver.DeviceCase, ckpts: list, every: int, h: torch.Tens
 
 def runs_beside(nc: int, cols: int, kind_changes: int) -> bool:
     """Whether NUFFT runs' samples are taken beside the sweep (``hb_adjoint_runs``) rather than inside it: as far as the
-    windows' columns and the coils pay for the weights formed at every change of kind (``nufft.Plan.kind_changes``). The
-    backward of 1,024 runs of 64 samples, 262,144 spins, beside against inside, one kind and 21 columns: 1 coil 20.2 /
-    23.2 ms, 4 coils 22.3 / 30.6, 8 coils 25.1 / 40.7, 16 coils 51.2 / 106.7; 7 columns: 1 coil 20.0 / 19.9, 16 coils
-    50.8 / 61.0; 5 columns: 8 coils 24.9 / 24.7, 16 coils 50.4 / 53.2. A kind that changes at every run adds 16.7 ms (16 coils
-    29.6)."""
+    windows' columns and the coils pay for the weights formed at every change of kind and in every interval
+    (``kind_changes``: of 1,024 runs, how many the weights are formed for). The backward of 1,024 runs of 64 samples,
+    262,144 spins, beside against inside, one kind and 21 columns: 1 coil 20.2 / 23.2 ms, 4 coils 22.3 / 30.6, 8 coils
+    25.1 / 40.7, 16 coils 51.2 / 106.7; 7 columns: 1 coil 20.0 / 19.9, 16 coils 50.8 / 61.0; 5 columns: 8 coils 24.9 /
+    24.7, 16 coils 50.4 / 53.2. A kind that changes at every run adds 16.7 ms (16 coils 29.6)."""
     return bool(hip.load().hb_adjoint_runs_takes(nc, cols)) and kind_changes <= nc * (8 * (cols - 7) + nc)
+
+
+def _weights_formed(case) -> int:
+    """Of 1,024 NUFFT runs, how many follow one of another kind or an interval's start, with the default intervals (and so
+    the same for any)."""
+    S, plan = case.n_segments, case.nu["plan"]
+    intervals = -(-S // default_checkpoint_every(S, True))
+    return plan.kind_changes + -(-1024 * intervals // len(plan.runs))
 
 
 def _sweep(case, cs, ckpts, every, h, lam, sens, nc, need_seg, need_coil, lib, seeds, maps_d, gs, gc, seg) -> None:
@@ -250,7 +258,7 @@ def _sweep(case, cs, ckpts, every, h, lam, sens, nc, need_seg, need_coil, lib, s
     need = hip.load().hb_adjoint_chunks_workspace(n_pad, every, nc) if not case.n_pulses and nu is None else 0
     work = torch.empty(need, dtype=torch.float32, device=dev) if need else None
     runs = None
-    if grid is not None and runs_beside(nc, nu["cols"], nu["kind_changes"]):
+    if grid is not None and runs_beside(nc, nu["cols"], _weights_formed(case)):
         heads = np.fromiter((a for a, _ in nu["plan"].runs), dtype=np.int32, count=len(nu["plan"].runs))
         at = np.searchsorted(heads, [*case.starts, case.ends[-1]])  # each interval's first run
         runs = (torch.from_numpy(heads).to(dev),

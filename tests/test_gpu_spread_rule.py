@@ -70,6 +70,19 @@ def test_rule_of_the_reverse():
     assert not beside(3, 21, 0)
 
 
+@pytest.mark.parametrize("kinds,reps,interval", [(1, 7, 256), (1, 40, 512), (2, 40, 512)])
+def test_weights_formed_in_the_reverse(kinds, reps, interval):
+    """Every change of kind and every default interval forms them, whatever interval is asked for."""
+    from types import SimpleNamespace
+
+    seq = scan(200, kinds, 1, reps)
+    plan = nu_mod.make_plan(seq, 6, 3)
+    assert adjoint.default_checkpoint_every(len(seq), True) == interval
+    case = SimpleNamespace(n_segments=len(seq), nu=dict(plan=plan))
+    changes = reps - 1 if kinds > 1 else 0
+    assert adjoint._weights_formed(case) == -(-1024 * changes // reps) + -(-1024 * -(-len(seq) // interval) // reps)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n_spins,coils,kinds,every", [(255, 1, 2, 128), (700, 2, 3, 64), (300, 4, 2, 192)])
 def test_beside_on_kinds_in_turn(gpu, monkeypatch, n_spins, coils, kinds, every):
