@@ -53,7 +53,7 @@ def ifftnc(k: Tensor, ndim: int) -> Tensor:
         from .engines import hip
 
         lib = hip.HIP.lib()
-        src = k.contiguous()
+        src = k.resolve_conj().contiguous()
         out = torch.empty_like(src)
         shape = list(src.shape)
         plane = ndim >= 2 and hip.load().hb_ifftc_plane_takes(shape[-2], shape[-1])
@@ -97,7 +97,7 @@ def rss(images: Tensor, dim: int = 0) -> Tensor:
     if _on_hip(images, torch.complex64) and images.ndim >= 1 and dim in (0, -images.ndim) and images.numel():
         from .engines import hip
 
-        src = images.contiguous()
+        src = images.resolve_conj().contiguous()
         out = torch.empty(src.shape[1:], dtype=torch.float32, device=src.device)
         hip.HIP.lib().rss(src.data_ptr(), src.shape[0], out.numel(), out.data_ptr())
         return out
