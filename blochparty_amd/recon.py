@@ -37,7 +37,8 @@ def kspace_grid(signal: Tensor, seq: Sequence) -> Tensor:
 
 
 def _on_hip(t: Tensor, dtype: torch.dtype) -> bool:
-    return t.is_cuda and t.dtype == dtype
+    """The HIP kernels take ``t``: not where its gradient is wanted (torch's operations carry it)."""
+    return t.is_cuda and t.dtype == dtype and not (t.requires_grad and torch.is_grad_enabled())
 
 
 def _pow2(n: int) -> bool:
