@@ -154,6 +154,16 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return t.data_ptr()
 
 
+_RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # not a public name of torch
+
+
+def raw_stream() -> int:
+    """The handle of torch's current stream, without the Stream object where torch offers it (12 -> 1 us of every call)."""
+    if _RAW_STREAM is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _RAW_STREAM(torch.cuda.current_device())
+
+
 class Kernels:
     """``lib.<entry point>(*args)``: calls the C ABI on the current stream, raising RuntimeError on failure."""
 
@@ -164,8 +174,7 @@ class Kernels:
         fn = getattr(lib, "hb_" + name)
 
         def call(*args):
-            # current_stream().cuda_stream without the Stream object (12 -> 1 us of every call)
-            rc = fn(*args, torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+            rc = fn(*args, raw_stream())
             if rc != 0:
                 raise RuntimeError(f"HIP error {rc} in hb_{name}: {lib.hb_error_string(rc).decode()}")
 
