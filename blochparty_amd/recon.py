@@ -54,7 +54,7 @@ def ifftnc(k: Tensor, ndim: int) -> Tensor:
         from .engines import hip
 
         lib = hip.HIP.lib()
-        src = k.resolve_conj().contiguous()
+        src = (k.resolve_conj() if k.is_conj() else k).contiguous()
         out = torch.empty_like(src)
         shape = list(src.shape)
         plane = ndim >= 2 and hip.load().hb_ifftc_plane_takes(shape[-2], shape[-1])
@@ -98,7 +98,7 @@ def rss(images: Tensor, dim: int = 0) -> Tensor:
     if _on_hip(images, torch.complex64) and images.ndim >= 1 and dim in (0, -images.ndim) and images.numel():
         from .engines import hip
 
-        src = images.resolve_conj().contiguous()
+        src = (images.resolve_conj() if images.is_conj() else images).contiguous()
         out = torch.empty(src.shape[1:], dtype=torch.float32, device=src.device)
         hip.HIP.lib().rss(src.data_ptr(), src.shape[0], out.numel(), out.data_ptr())
         return out
