@@ -330,12 +330,13 @@ __device__ __forceinline__ void replay_interval(const hb_case& cs, const hb_adjo
             s = e - 1;
             continue;
         }
-        // an RF train: its own loop, the next record in flight (more spill scalar registers, also where no train is stepped:
-        // the replay of 4,336 records with maps and runs at 64^3 110 -> 128 us)
+        // an RF train: its own loop, two records in flight, beside NUFFT runs one (more spill scalar registers, also where
+        // no train is stepped: the replay of 4,336 records with maps and runs at 64^3 110 -> 128 us with three; a million
+        // spins, trains of 200, intervals of 1,024: one 58.0 ms, two 56.2, three 55.7, but 24^3 x 4 stepped slower)
         if (q.flags & HB_TRAIN) {
             const int L = min(q.pad[3], s1 - s);
             const hb_segment* first = cs.segs + s;
-            rf_records<1>(
+            rf_records<NU ? 1 : 2>(
                 L, [&](int i) { return first + i; },
                 [&](int i, const RfRec& c) {
                     if (i > 0 && ((s + i - s0) & 7) == 0) {
