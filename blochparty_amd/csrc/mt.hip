@@ -22,7 +22,7 @@
 //   exponential or division; longer ones from the eigenvalues' expm1.
 // - ADC: eight samples at a time are staged in LDS and contracted with the coils on the matrix cores in float32
 //   (contract_device.h), one barrier per eight; the workgroup's sums go to the partial rows that hb_signal_reduce sums
-//   in a fixed order: no atomics. (float16 pairs took 0.33 ms less, but lost a coil 2^-17 of another, or spins
+//   in a fixed order: no atomics. (float16 pairs took 0.2 ms less, but lost a coil 2^-17 of another, or spins
 //   beside one 2^24 as bright that no coil sees, most of their bits.)
 //
 // What bounds it: with 65,536 spins every SIMD has one wave, so nothing hides a wave's latency, and a segment costs its
@@ -32,7 +32,7 @@
 // an RF train is stepped in a loop of its own that reads four values per substep, a readout run in one that reads none
 // and relaxes the longitudinal components once. The next record is loaded while the current one is stepped, and the
 // lanes touch the records 64 ahead, so that they are in the L2 when their turn comes. 65,536 spins with a bound pool and
-// leading-order fields, 8 coils, 32,256 segments (12,800 RF, 16,384 samples): 10.1 ms, against 34.8 ms with a barrier and
+// leading-order fields, 8 coils, 32,256 segments (12,800 RF, 16,384 samples): 9.9 ms, against 34.8 ms with a barrier and
 // a shuffle tree per sample, steady states by division and every factor formed per segment. Of its 5.75 million issue
 // slots a wave uses 2.3 for VALU and 1.0 for scalar instructions and waits in 1.8 (SQ counters).
 #include "bloch_device.h"

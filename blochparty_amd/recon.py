@@ -4,8 +4,9 @@ combination, the k-space trajectory of a sequence, and the raw data as ISMRMRD a
 Reference interface: ``src/blochparty/recon.py:13-60`` (``kspace_grid``, ``ifftnc``, ``reconstruct``, ``rss``,
 ``coil_combine``, ``fft2c``), ``sequence.py:173-217`` (``flip_angle``, ``kspace_trajectory``) and
 ``io/ismrmrd.py`` (one acquisition per readout, its trajectory and encode indices). On the GPU, complex64 k-space with
-power-of-two axes takes the HIP kernels (``csrc/recon.hip``: one centred inverse DFT pass per axis, and the RSS);
-other shapes and dtypes, and CPU tensors, take torch's FFT as the reference does. Writing an ISMRMRD HDF5 file needs
+power-of-two axes takes the HIP kernels (``csrc/recon.hip``: one centred inverse DFT pass per axis, or for the last two
+at once, and the RSS); other shapes and dtypes, CPU tensors, and k-space whose gradient is wanted take torch's FFT as the
+reference does. Writing an ISMRMRD HDF5 file needs
 ``h5py`` (absent here, as in the reference without its ``io`` extra: ``ImportError``); the acquisitions are built
 without it.
 """
@@ -47,8 +48,9 @@ def _pow2(n: int) -> bool:
 
 def ifftnc(k: Tensor, ndim: int) -> Tensor:
     """Centred inverse DFT over the last ``ndim`` axes, backward normalisation: a spin of magnetization m at a
-    voxel centre gives that voxel the value m. complex64 on the GPU with power-of-two axes (2..4096): the last two
-    in one HIP pass where a plane fits in LDS (``hb_ifftc_plane``), else one pass per axis (``hb_ifftc_axis``); otherwise torch's FFT on the tensor's device."""
+    voxel centre gives that voxel the value m. complex64 on the GPU with power-of-two axes (2..4096) and no gradient
+    wanted: the last two in one HIP pass where a plane fits in LDS (``hb_ifftc_plane``), else one pass per axis
+    (``hb_ifftc_axis``); otherwise torch's FFT on the tensor's device."""
     axes = tuple(range(-ndim, 0))
     if _on_hip(k, torch.complex64) and 1 <= ndim <= k.ndim and all(_pow2(k.shape[a]) for a in axes):
         from .engines import hip

@@ -55,10 +55,10 @@ typedef struct hb_mt {
 
 /* The full-variant event loop (a bound pool, concomitant fields, bound-only RF: any of them) over segments
  * [s0, s1) of plain records (no merged runs, reused pulses or NUFFT runs in the table; readout runs, HB_RUN, and
- * trains, HB_TRAIN, may be marked, each within one dispatch), one lane per spin: every ADC sample's coil sums per workgroup of 256 spins go to partial[(block * rows + r) * 16 * n_tiles +
- * 2 c + {re, im}], r = the segment's pad[0] - row0 (< rows), as hb_forward's, for hb_signal_reduce; in float32 (hb_case's
- * sens_scale and x_scale are not read). Replaces the
- * reference's bloch_chunk_mma with V = 1 (a rate bound pool and / or concomitant fields). */
+ * trains, HB_TRAIN, may be marked, each within one dispatch), one lane per spin: every ADC sample's coil sums per
+ * workgroup of 256 spins go to partial[(block * rows + r) * 16 * n_tiles + 2 c + {re, im}], r = the segment's pad[0] -
+ * row0 (< rows), as hb_forward's, for hb_signal_reduce; in float32 (hb_case's sens_scale and x_scale are not read).
+ * Replaces the reference's bloch_chunk_mma with V = 1 (a rate bound pool and / or concomitant fields). */
 int hb_forward_mt(const hb_case* cs, const hb_mt* mt, int32_t s0, int32_t s1, float* partial, int32_t rows,
                   int32_t row0, void* stream);
 
