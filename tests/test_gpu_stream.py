@@ -1,5 +1,5 @@
-"""The C calls' stream handle, GPU: torch's current stream, inside a stream context and outside, also where torch does not
-offer the raw handle."""
+"""The C calls' stream handle, GPU: torch's current stream, inside a stream context and outside, the raw handle where torch
+offers it and the public one."""
 
 import pytest
 import torch
@@ -8,11 +8,9 @@ from blochparty_amd.engines import hip
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("offered", [True, False])
-def test_handle_of_the_current_stream(gpu, monkeypatch, offered):
-    if not offered:
-        monkeypatch.setattr(hip, "_RAW_STREAM", None)
-    side = torch.cuda.Stream()
-    assert hip.raw_stream() == torch.cuda.current_stream().cuda_stream
+@pytest.mark.parametrize("handle", [hip.raw_stream, hip._public_stream])
+def test_handle_of_the_current_stream(gpu, handle):
+    side, dev = torch.cuda.Stream(), torch.cuda.current_device()
+    assert handle(dev) == torch.cuda.current_stream().cuda_stream
     with torch.cuda.stream(side):
-        assert hip.raw_stream() == side.cuda_stream != torch.cuda.default_stream().cuda_stream
+        assert handle(dev) == side.cuda_stream != torch.cuda.default_stream().cuda_stream
