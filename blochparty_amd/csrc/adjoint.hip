@@ -617,7 +617,7 @@ __global__ __launch_bounds__(kBlockA) __attribute__((amdgpu_waves_per_eu(NC <= 8
 // only on the numbers of spins and coils, so the gradients are the same bit for bit for any interval length (a multiple of 64).
 // What bounds it then: the sweep's chain (0.31 us a segment, its records from the scalar cache one ahead) and the chunks'
 // VALU work. 24^3 x 4 spins (216 workgroups), every RF substep, 8 coils, 347 intervals of 384 segments, forward and
-// reverse: 271 -> 149 ms (533 us an interval in one walk, 318 in chunks); 28^3 x 4, 16 coils: 671 -> 284 ms; a 128^2
+// reverse: 271 -> 143 ms (533 us an interval in one walk, 318 in chunks); 28^3 x 4, 16 coils: 671 -> 284 ms; a 128^2
 // turbo spin echo's map fit (32 workgroups, 64 segments an interval): 81 -> 50 ms a call.
 // replays: workgroups that replay [r0, r1) (n_pad / 256 of them, or none); the others take lambda back over [s0, s1).
 template <int NC>

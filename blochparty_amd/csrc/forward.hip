@@ -111,7 +111,7 @@ __device__ __forceinline__ void nufft_run(const hb_case& cs, const hb_nufft& nu,
 // 430 (SQ counters of the whole
 // kernel: 330 VALU instructions per wave and repetition of the 64^3 GRE, 512 staged). A single reused pulse's map is
 // held too (12 registers, some of them spilled: still faster than reading it from the L2 at every occurrence, 83.2 ->
-// 72.9 ms). 64^3 x 4 spins, 8 coils: 83.5 -> 70.6 ms a pass; 96^3, 16 coils: 219.3 -> 189.3 ms. Four waves per SIMD
+// 72.9 ms). 64^3 x 4 spins, 8 coils: 83.5 -> 70.9 ms a pass; 96^3, 16 coils: 219.3 -> 188 ms. Four waves per SIMD
 // (128 registers) and three (168, no spills) measured the same at a million spins; four keep 262,144 spins in one
 // round of workgroups. Only for dispatches without stepped RF: the RF loop is faster with five waves than this is with
 // four. Reading the next record ahead costs 32 scalar moves a record and measured 8 % slower.

@@ -20,7 +20,8 @@
 // 80 %. (In float32 on v_mfma_f32_16x16x4_f32 the products take four times as long: the backward at 64^3 264.8 -> 273.5 ms.)
 // That is about 350 VALU instructions a run; taken column by column in the sweep it was 2,300, at two waves per SIMD.
 // Measured at 64^3 spins, 8 coils, 16 runs of 64 samples an interval: the sweep 1,086 -> 682 us, with 120 us here and 109 us
-// for the replay on its own; the whole backward of 4,096 runs 341 -> 295 ms.
+// for the replay on its own; the whole backward of 4,096 runs 341 -> 295 ms (now 549, 113 and 103 us; forward and backward
+// 254 ms). Where it is not taken: engines/adjoint.py, runs_beside.
 #include "nufft_back.h"
 
 #include "bloch_device.h"
